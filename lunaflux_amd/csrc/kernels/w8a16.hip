@@ -1128,12 +1128,12 @@ extern "C" {
     w8a16_kernel<LF_W16_WAVES, MT, 2, D, XC>(counts, x, wg, wu, wu, h, ws);           \
   }
 
+// (17..64 rows: the LDS-tiled GEMM of w8a16_gemm.hip under the _m32 and _m64
+// symbols)
 LF_W8A16_ENTRIES(1, 16, 4, 4)
-LF_W8A16_ENTRIES(2, 32, 4, 4)
-LF_W8A16_ENTRIES(4, 64, 4, 4)
 LF_W8A16_ENTRIES(8, 128, 2, 2)
 
-// The same column-group forms over weights with 128 x 128 block scales.
+// The same column-group form over weights with 128 x 128 block scales.
 #define LF_W8A16_B128_ENTRIES(MT, M, D, XC)                                                     \
   __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_dense_b128_m##M(         \
       const int32_t *counts, const uint16_t *x, const uint8_t *w, uint16_t *y, uint8_t *ws) { \
@@ -1150,9 +1150,6 @@ LF_W8A16_ENTRIES(8, 128, 2, 2)
     w8a16_kernel<LF_W16_WAVES, MT, 2, D, XC, true>(counts, x, wg, wu, wu, h, ws);            \
   }
 
-LF_W8A16_B128_ENTRIES(1, 16, 4, 4)
-LF_W8A16_B128_ENTRIES(2, 32, 4, 4)
-LF_W8A16_B128_ENTRIES(4, 64, 4, 4)
 LF_W8A16_B128_ENTRIES(8, 128, 2, 2)
 
 #ifndef LF_W16T_WAVES

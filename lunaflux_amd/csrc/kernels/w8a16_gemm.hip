@@ -1,5 +1,6 @@
-// w8a16_gemm.hip - W8A16 (bf16 activations x e4m3 weights) for profiles of
-// 65..128 rows, as an LDS-tiled GEMM.
+// w8a16_gemm.hip - W8A16 (bf16 activations x e4m3 weights) as an LDS-tiled
+// GEMM, for profiles of 65..128 rows and for smaller ones without a
+// shape-specialized entry (the tiles are at the entries, below).
 //
 // At 128 rows every weight byte feeds 128 rows of MFMA work. A block of 8
 // waves (two per SIMD, so one wave's LDS reads overlap the other's MFMAs)
@@ -57,9 +58,9 @@
 
 namespace w16g {
 
-template <int BN, int WGM, int WGN, int NSA, int NSB>
+template <int BM, int BN, int WGM, int WGN, int NSA, int NSB>
 struct Tile {
-  static constexpr int kBM = 128, kWgm = WGM, kWgn = WGN, kWaves = WGM * WGN;
+  static constexpr int kBM = BM, kWgm = WGM, kWgn = WGN, kWaves = WGM * WGN;
   static constexpr int kWaveM = kBM / kWgm, kWaveN = BN / kWgn;
   static constexpr int kFM = kWaveM / 16, kFN = kWaveN / 16;
   static constexpr int kAStage = kBM * 256;  // bytes
@@ -70,7 +71,10 @@ struct Tile {
   static constexpr int kBIns = kBStage / 1024 / kLoaders;
   static_assert(kSmem + 16 <= 160 * 1024, "LDS budget");
   static_assert(kBStage % (1024 * kLoaders) == 0, "weight half-tiles split evenly");
-  static_assert(kFN % 2 == 0, "gate/up pairs a wave's fragments");
+  // Widths not a multiple of a block's columns (any N that is a multiple of
+  // 16): the last block's spare fragments read the last tile again and
+  // store nothing. The 128-row geometry only takes widths that divide.
+  static constexpr bool kPartial = BM < 128;
   static_assert(NSA >= 2 && NSB >= 2, "rings of at least two stages");
   static_assert((NSA - 2) * kAIns < 64 && (NSB - 2) * kBIns < 64, "vmcnt range");
 };
@@ -91,6 +95,14 @@ LF_DEVICE void wait_ring(int later) {
   }
 }
 
+// K-slices of the forms below 128 rows: as many as keep 8 k-tiles per slice
+// and one block per CU (256), as the 128-row geometry. Measured (us, M = 24
+// dense 4096 x 2048: 1 / 2 / 3 / 4 / 8 slices 8.8 / 8.1 / 7.9 / 8.0 / 10.0;
+// 4096 x 1024: 1 / 2 / 4 5.7 / 6.2 / 6.8; M = 61 4096 x 7168: 3 / 4 15.7 /
+// 14.8; gate/up 7168 x 4096: 1 / 2 21.2 / 18.7). csrc/pack.cpp holds the
+// same rule.
+LF_DEVICE int w16_slices(int blocks_n, int kt) { return max(1, min(256 / blocks_n, kt / 8)); }
+
 // MODE 0: dense, 1: QKV (three weights, packed Q|K|V output), 2: gate/up
 // (each wave column's fragments: kFN / 2 gate tiles, then the up tiles of the
 // same h-columns, so SwiGLU pairs fragment j with j + kFN / 2 in a lane).
@@ -109,13 +121,14 @@ LF_DEVICE void wait_ring(int later) {
 // (one per wave and fragment, a scalar load) and added to the running sums
 // (y = sum_kt s[nb][kt] sum_{k in kt} x_k q_k, fp32); the epilogue's
 // multiplier is 1.
-template <int BN, int WGM, int WGN, int NSA, int NSB, int MODE, bool THROUGH = false, class Gate = NoWait,
+template <int BM, int BN, int WGM, int WGN, int NSA, int NSB, int MODE, bool THROUGH = false, class Gate = NoWait,
           bool BLOCK = false>
 __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *counts, const uint16_t *x,
                                                   const uint8_t *w0, const uint8_t *w1, const uint8_t *w2,
                                                   uint16_t *y, uint8_t *ws, int bid = -1, int nblocks = -1,
                                                   const Gate &gate = Gate{}) {
-  using T = Tile<BN, WGM, WGN, NSA, NSB>;
+  using T = Tile<BM, BN, WGM, WGN, NSA, NSB>;
+  static_assert(MODE != 2 || T::kFN % 2 == 0, "gate/up pairs a wave's fragments");
   __shared__ int last_block;
   if (!dense_regions_ok<MODE, BLOCK ? kScaleBlock128 : kScalePerChannel>(w0, w1, w2)) return;
   const WeightHeader &h0 = header_of(w0);
@@ -126,11 +139,15 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
   // output columns: ld; a block covers BN weight columns (gate/up: BN / 2
   // h-columns)
   const int ld = MODE == 1 ? nq + nk + static_cast<int>(header_of(w2).rows) : nq;
-  const int blocks_n = MODE == 2 ? ld / (BN / 2) : ld / BN;
+  constexpr int kCols = MODE == 2 ? BN / 2 : BN;
+  const int blocks_n = T::kPartial ? (ld + kCols - 1) / kCols : ld / kCols;
   if (blocks_n < 1) return;
   const int nb = nblocks < 0 ? static_cast<int>(gridDim.x) : nblocks;
   const int block = bid < 0 ? static_cast<int>(blockIdx.x) : bid;
-  const int S = nb / blocks_n;
+  // K-slices. Forms below 128 rows: at most w16_slices of them (the rule
+  // and its measurements: there); the geometry's grid may hold more, whose
+  // blocks end here.
+  const int S = T::kPartial ? min(nb / blocks_n, w16_slices(blocks_n, KT)) : nb / blocks_n;
   // A grid whose split is not 1..KT (the geometry rules it out) stores
   // nothing in any block: an empty K-slice would never arrive, and its
   // column block's counter would stay raised for later launches.
@@ -150,25 +167,27 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
   const int lw = a_loader ? wave : wave - T::kLoaders;  // index among its ring's loaders
 
   // Block slot sl (16 weight columns) -> (region, tile index in it, output
-  // column of the slot's first column).
+  // column of the slot's first column; past ld in a partial block's spare
+  // slots, which take the last tile).
   auto slot = [&](int sl, const uint8_t *&region, int &tile, int &ocol) {
     if constexpr (MODE == 2) {
       const int sw = sl / T::kFN, f = sl % T::kFN;
       const bool up = f >= T::kFN / 2;
       ocol = cb * (BN / 2) + sw * (T::kWaveN / 2) + 16 * (up ? f - T::kFN / 2 : f);
       region = up ? w1 : w0;
-      tile = ocol >> 4;
+      tile = (T::kPartial ? min(ocol, ld - 16) : ocol) >> 4;
     } else {
       ocol = cb * BN + 16 * sl;
+      const int col = T::kPartial ? min(ocol, ld - 16) : ocol;
       region = w0;
-      tile = ocol >> 4;
+      tile = col >> 4;
       if constexpr (MODE == 1) {
-        if (ocol >= nq + nk) {
+        if (col >= nq + nk) {
           region = w2;
-          tile = (ocol - nq - nk) >> 4;
-        } else if (ocol >= nq) {
+          tile = (col - nq - nk) >> 4;
+        } else if (col >= nq) {
           region = w1;
-          tile = (ocol - nq) >> 4;
+          tile = (col - nq) >> 4;
         }
       }
     }
@@ -405,6 +424,7 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
             const uint8_t *region;
             int tile, ocol;
             slot(wn * T::kFN + j, region, tile, ocol);
+            if (T::kPartial && ocol >= ld) continue;
             const float out = silu_mul(v[i][j][e] * sc[j],
                                        v[i][j + T::kFN / 2][e] * sc[j + T::kFN / 2]);
             put(y + static_cast<uint64_t>(m) * ld + ocol + r, out);
@@ -415,6 +435,7 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
             const uint8_t *region;
             int tile, ocol;
             slot(wn * T::kFN + j, region, tile, ocol);
+            if (T::kPartial && ocol >= ld) continue;
             put(y + static_cast<uint64_t>(m) * ld + ocol + r, v[i][j][e] * sc[j]);
           }
         }
@@ -506,8 +527,8 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
 template <int GU_BN, int DN_BN, int WGM, int WGN, int GU_NSA, int GU_NSB, int DN_NSA, int DN_NSB,
           bool BLOCK = false>
 struct GatedMlpGemm {
-  using GU = Tile<GU_BN, WGM, WGN, GU_NSA, GU_NSB>;
-  using DN = Tile<DN_BN, WGM, WGN, DN_NSA, DN_NSB>;
+  using GU = Tile<128, GU_BN, WGM, WGN, GU_NSA, GU_NSB>;
+  using DN = Tile<128, DN_BN, WGM, WGN, DN_NSA, DN_NSB>;
   static constexpr int kSmem = GU::kSmem > DN::kSmem ? GU::kSmem : DN::kSmem;
   LF_DEVICE static void run(const int32_t *counts, const uint16_t *x, const uint8_t *wg,
                             const uint8_t *wu, const uint8_t *wd, uint16_t *y, uint8_t *ws) {
@@ -540,7 +561,7 @@ struct GatedMlpGemm {
     };
     const int b = static_cast<int>(blockIdx.x);
     if (b < g1) {
-      w8a16_gemm_kernel<GU_BN, WGM, WGN, GU_NSA, GU_NSB, 2, true, NoWait, BLOCK>(smem, counts, x, wg, wu, wu,
+      w8a16_gemm_kernel<128, GU_BN, WGM, WGN, GU_NSA, GU_NSB, 2, true, NoWait, BLOCK>(smem, counts, x, wg, wu, wu,
                                                                                  h, ws_down, b, g1);
       phase::signal(sync + phase::kLineInts * slice_of(b * (GU_BN / 2) / 128));
       return;
@@ -549,7 +570,7 @@ struct GatedMlpGemm {
       const int target = (KT * (sl + 1) / S - KT * sl / S) * (128 / (GU_BN / 2));
       return phase::wait_for(sync + phase::kLineInts * sl, target, error, flag);
     };
-    w8a16_gemm_kernel<DN_BN, WGM, WGN, DN_NSA, DN_NSB, 0, false, decltype(gate), BLOCK>(
+    w8a16_gemm_kernel<128, DN_BN, WGM, WGN, DN_NSA, DN_NSB, 0, false, decltype(gate), BLOCK>(
         smem, counts, h, wd, wd, wd, y, ws_down, b - g1, g2, gate);
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -568,53 +589,59 @@ extern "C" {
 
 // Symbols: lf_fp8_w8a16_{op}_m128_n{BN}; the launch geometry picks BN and the
 // K split S (grid = column blocks x S; blocks of 64 WGM WGN threads).
-#define LF_W16_GEMM_ENTRIES(BN, WGM, WGN, NSA, NSB)                                              \
-  __global__ __launch_bounds__(64 * WGM * WGN) void lf_fp8_w8a16_dense_m128_n##BN(               \
-      const int32_t *counts, const uint16_t *x, const uint8_t *w, uint16_t *y, uint8_t *ws) {     \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[w16g::Tile<BN, WGM, WGN, NSA, NSB>::kSmem]; \
-    w16g::w8a16_gemm_kernel<BN, WGM, WGN, NSA, NSB, 0>(smem, counts, x, w, w, w, y, ws);          \
+// _b128: over weights with 128 x 128 block scales. DN_ / GU_: the tile of the
+// dense and QKV, and of the gate/up entry.
+#define LF_W16_GEMM_BODY(MODE, BLOCK, ARGS, ...)                                                 \
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[w16g::Tile<__VA_ARGS__>::kSmem];        \
+  w16g::w8a16_gemm_kernel<__VA_ARGS__, MODE, false, NoWait, BLOCK> ARGS;
+#define LF_W16_GEMM_DENSE_QKV(SUFFIX, BLOCK, THREADS, ...)                                       \
+  __global__ __launch_bounds__(THREADS) void lf_fp8_w8a16_dense##SUFFIX(                         \
+      const int32_t *counts, const uint16_t *x, const uint8_t *w, uint16_t *y, uint8_t *ws) {    \
+    LF_W16_GEMM_BODY(0, BLOCK, (smem, counts, x, w, w, w, y, ws), __VA_ARGS__)                   \
   }                                                                                              \
-  __global__ __launch_bounds__(64 * WGM * WGN) void lf_fp8_w8a16_qkv_m128_n##BN(                 \
+  __global__ __launch_bounds__(THREADS) void lf_fp8_w8a16_qkv##SUFFIX(                           \
       const int32_t *counts, const uint16_t *x, const uint8_t *wq, const uint8_t *wk,            \
       const uint8_t *wv, uint16_t *y, uint8_t *ws) {                                             \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[w16g::Tile<BN, WGM, WGN, NSA, NSB>::kSmem]; \
-    w16g::w8a16_gemm_kernel<BN, WGM, WGN, NSA, NSB, 1>(smem, counts, x, wq, wk, wv, y, ws);       \
-  }                                                                                              \
-  __global__ __launch_bounds__(64 * WGM * WGN) void lf_fp8_w8a16_gate_up_m128_n##BN(             \
+    LF_W16_GEMM_BODY(1, BLOCK, (smem, counts, x, wq, wk, wv, y, ws), __VA_ARGS__)                \
+  }
+#define LF_W16_GEMM_GATE_UP(SUFFIX, BLOCK, THREADS, ...)                                         \
+  __global__ __launch_bounds__(THREADS) void lf_fp8_w8a16_gate_up##SUFFIX(                       \
       const int32_t *counts, const uint16_t *x, const uint8_t *wg, const uint8_t *wu,            \
       uint16_t *h, uint8_t *ws) {                                                                \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[w16g::Tile<BN, WGM, WGN, NSA, NSB>::kSmem]; \
-    w16g::w8a16_gemm_kernel<BN, WGM, WGN, NSA, NSB, 2>(smem, counts, x, wg, wu, wu, h, ws);       \
+    LF_W16_GEMM_BODY(2, BLOCK, (smem, counts, x, wg, wu, wu, h, ws), __VA_ARGS__)                \
   }
 
-LF_W16_GEMM_ENTRIES(64, 4, 2, 3, 4)
-LF_W16_GEMM_ENTRIES(128, 2, 4, 2, 4)
+LF_W16_GEMM_DENSE_QKV(_m128_n64, false, 512, 128, 64, 4, 2, 3, 4)
+LF_W16_GEMM_GATE_UP(_m128_n64, false, 512, 128, 64, 4, 2, 3, 4)
+LF_W16_GEMM_DENSE_QKV(_m128_n128, false, 512, 128, 128, 2, 4, 2, 4)
+LF_W16_GEMM_GATE_UP(_m128_n128, false, 512, 128, 128, 2, 4, 2, 4)
+LF_W16_GEMM_DENSE_QKV(_b128_m128_n64, true, 512, 128, 64, 4, 2, 3, 4)
+LF_W16_GEMM_GATE_UP(_b128_m128_n64, true, 512, 128, 64, 4, 2, 3, 4)
+LF_W16_GEMM_DENSE_QKV(_b128_m128_n128, true, 512, 128, 128, 2, 4, 2, 4)
+LF_W16_GEMM_GATE_UP(_b128_m128_n128, true, 512, 128, 128, 2, 4, 2, 4)
 
-// The same over weights with 128 x 128 block scales:
-// lf_fp8_w8a16_{op}_b128_m128_n{BN}.
-#define LF_W16_GEMM_B128_ENTRIES(BN, WGM, WGN, NSA, NSB)                                         \
-  __global__ __launch_bounds__(64 * WGM * WGN) void lf_fp8_w8a16_dense_b128_m128_n##BN(          \
-      const int32_t *counts, const uint16_t *x, const uint8_t *w, uint16_t *y, uint8_t *ws) {     \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[w16g::Tile<BN, WGM, WGN, NSA, NSB>::kSmem]; \
-    w16g::w8a16_gemm_kernel<BN, WGM, WGN, NSA, NSB, 0, false, NoWait, true>(smem, counts, x, w, w, w, y, ws); \
-  }                                                                                              \
-  __global__ __launch_bounds__(64 * WGM * WGN) void lf_fp8_w8a16_qkv_b128_m128_n##BN(            \
-      const int32_t *counts, const uint16_t *x, const uint8_t *wq, const uint8_t *wk,            \
-      const uint8_t *wv, uint16_t *y, uint8_t *ws) {                                             \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[w16g::Tile<BN, WGM, WGN, NSA, NSB>::kSmem]; \
-    w16g::w8a16_gemm_kernel<BN, WGM, WGN, NSA, NSB, 1, false, NoWait, true>(smem, counts, x, wq, wk, wv, y, \
-                                                                            ws);                 \
-  }                                                                                              \
-  __global__ __launch_bounds__(64 * WGM * WGN) void lf_fp8_w8a16_gate_up_b128_m128_n##BN(        \
-      const int32_t *counts, const uint16_t *x, const uint8_t *wg, const uint8_t *wu,            \
-      uint16_t *h, uint8_t *ws) {                                                                \
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[w16g::Tile<BN, WGM, WGN, NSA, NSB>::kSmem]; \
-    w16g::w8a16_gemm_kernel<BN, WGM, WGN, NSA, NSB, 2, false, NoWait, true>(smem, counts, x, wg, wu, wu, h, \
-                                                                            ws);                 \
-  }
-
-LF_W16_GEMM_B128_ENTRIES(64, 4, 2, 3, 4)
-LF_W16_GEMM_B128_ENTRIES(128, 2, 4, 2, 4)
+// Profiles of 17..64 rows (block-scaled: 1..64), any width that is a
+// multiple of 16, where no shape-specialized entry is built (w8a16.hip): 64
+// dense / QKV columns per block, 64 gate and 64 up columns for gate/up. At
+// these row counts the kernel is bound by bytes in flight: 32 / 64 rows of
+// activations are a quarter / half of the 128-row stage, which leaves LDS
+// for weight rings of 3-8 stages (40-64 KiB of weights in flight per block).
+// They replace column-group kernels whose rolled register ring drained at
+// every k-tile. Llama-3-8B as one of two tensor-parallel ranks, M = 61, us
+// before -> now: qkv (3072 x 4096) 23.2 -> 11.1, o (4096 x 2048) 19.0 ->
+// 9.3, gate/up (7168 x 4096) 32.8 -> 18.7, down (4096 x 7168) 26.1 -> 14.8
+// (2.0 TB/s of weights); M = 24: qkv 13.2 -> 9.1, o 9.0 -> 8.1, gate/up 16.9
+// -> 15.9, down 12.8 -> 12.5.
+LF_W16_GEMM_DENSE_QKV(_m32, false, 256, 32, 64, 2, 2, 3, 6)
+LF_W16_GEMM_GATE_UP(_m32, false, 256, 32, 128, 1, 4, 3, 3)
+LF_W16_GEMM_DENSE_QKV(_m64, false, 512, 64, 64, 4, 2, 3, 6)
+LF_W16_GEMM_GATE_UP(_m64, false, 512, 64, 128, 2, 4, 3, 5)
+LF_W16_GEMM_DENSE_QKV(_b128_m16, true, 256, 16, 64, 1, 4, 3, 6)
+LF_W16_GEMM_GATE_UP(_b128_m16, true, 256, 16, 128, 1, 4, 3, 4)
+LF_W16_GEMM_DENSE_QKV(_b128_m32, true, 256, 32, 64, 2, 2, 3, 6)
+LF_W16_GEMM_GATE_UP(_b128_m32, true, 256, 32, 128, 1, 4, 3, 3)
+LF_W16_GEMM_DENSE_QKV(_b128_m64, true, 256, 64, 64, 2, 2, 3, 8)
+LF_W16_GEMM_GATE_UP(_b128_m64, true, 256, 64, 128, 1, 4, 3, 5)
 
 // One-launch GatedMlp for profiles of 65..128 rows, any H and I the forms
 // divide: gate/up on the n128 tiles (one K-slice), down on n128 or n64 (the

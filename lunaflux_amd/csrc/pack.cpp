@@ -55,17 +55,30 @@ inline int64_t swizzled_offset(int64_t n, int64_t k, int64_t columns) {
 }
 
 
-// W8A16 work split (the kernels are in lunaflux_amd/csrc/kernels/w8a16.hip).
-// Profiles with at most 16 rows use the one-tile form: a block of
-// kW16TileWaves waves per 16-column tile, K split across its waves, one
-// block per tile. Larger profiles use the column-group form: one tile per
-// wave, kW16Waves tiles per block, K cut into `split` slices across blocks
-// (about 512 blocks: two per CU of an MI355X, which is what its 64 KiB LDS
-// ring allows), partial tiles reduced through the workspace. Measured at
-// M = 32 on the Llama-3-8B shapes: 256 or 768+ blocks are slower (fewer
-// bytes in flight, or more partial traffic).
+// W8A16 work split of the entries that fit any shape (the kernels are in
+// lunaflux_amd/csrc/kernels/w8a16.hip and w8a16_gemm.hip). Profiles with at
+// most 16 rows use the one-tile form: a block of kW16TileWaves waves per
+// 16-column tile, K split across its waves, one block per tile. Larger
+// profiles: kW16Waves 16-column tiles per block (gate/up: of both weights),
+// K cut into `split` slices across blocks, partial tiles reduced through the
+// workspace. 17..64 rows (mt 2, 4; block-scaled also mt 1) run the LDS-tiled
+// GEMM of w8a16_gemm.hip, which cuts K into w16_slices slices. Up to
+// kW16DirectK the grid and workspace are sized for about 512 blocks all the
+// same, as they were for the column-group kernels (two blocks per CU): those
+// past the GEMM's slices end at once, on CUs its at most 256 blocks leave
+// free. Wider K runs exactly the GEMM's blocks (a block's LDS rings fill a
+// CU there, so spare blocks would queue behind the others: 4096 x 14336 at
+// M = 61 21.9 us). 65..128 rows of a width that is no multiple of 64 run the
+// column-group form of w8a16.hip on about 512 blocks.
 constexpr int kW16Waves = 4;
 constexpr int kW16TileWaves = 8;
+constexpr int64_t kW16DirectK = 2048;
+// kernels/w8a16_gemm.hip, w16_slices
+int64_t w16_slices(int64_t blocks_n, int64_t kt) {
+  return std::max<int64_t>(1, std::min<int64_t>(256 / blocks_n, kt / 8));
+}
+// Threads of the entries that fit any shape above 16 rows.
+int w16_threads(int mt, bool block) { return mt == 4 && !block ? 512 : 64 * kW16Waves; }
 struct W8a16Split {
   int mt;
   bool one_tile;
@@ -86,6 +99,7 @@ bool w8a16_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
   int64_t split = (512 + groups / 2) / groups;
   if (split < 1) split = 1;
   if (split > kt) split = kt;
+  if (mt != 8 && k > kW16DirectK) split = w16_slices(groups, kt);
   if (groups * split > INT32_MAX) return false;
   out->groups = groups;
   out->split = split;
@@ -96,10 +110,9 @@ bool w8a16_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
 // LDS-tiled GEMM form with the per-channel entries' tile and split
 // (w8a16_gemm below, the _b128_m128_n{BN} symbols; every block-scaled width
 // is a multiple of 128, so a 16-column fragment lies in one 128-row scale
-// block); every other profile (also <= 16 rows) the column-group form,
-// split as above, with at least enough slices that each holds <= 128
-// k-tiles (the block scales of a slice are staged in LDS, kW16BlockSliceKT
-// in kernels/w8a16.hip).
+// block); every other profile (also <= 16 rows) the GEMM form's _b128_m16 /
+// _m32 / _m64 entries, the grid sized as above and for slices of at most 128
+// k-tiles.
 bool w8a16_b128_entry(int32_t e) {
   return e == LF_FP8_ENTRY_W8A16_DENSE_B128 || e == LF_FP8_ENTRY_W8A16_QKV_B128 ||
          e == LF_FP8_ENTRY_W8A16_GATE_UP_B128;
@@ -113,10 +126,12 @@ int32_t w8a16_channel_entry(int32_t e) {
 bool w8a16_b128_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
   if (n % 128 != 0 || k % 128 != 0 || !w8a16_split(n, k, max_tokens, out)) return false;
   const int64_t kt = k / 128, tiles = n / 16;
-  if (out->one_tile) {
+  if (out->one_tile) {  // <= 16 rows: the GEMM form too
     out->one_tile = false;
     out->groups = (tiles + kW16Waves - 1) / kW16Waves;
-    out->split = std::min<int64_t>(kt, std::max<int64_t>(1, (512 + out->groups / 2) / out->groups));
+    out->split = k > kW16DirectK
+                     ? w16_slices(out->groups, kt)
+                     : std::min<int64_t>(kt, std::max<int64_t>(1, (512 + out->groups / 2) / out->groups));
   }
   out->split = std::max<int64_t>(out->split, (kt + 127) / 128);
   return out->groups * out->split <= INT32_MAX;
@@ -139,6 +154,10 @@ struct W8a16Fixed {
   int64_t min_n = 0;  // chosen only for N >= min_n (earlier rows win)
 };
 constexpr int64_t kWideN = 16384;
+// Unsplit gate/up at 32 rows: 64 columns per block, so below 12288 columns
+// (192 blocks) too few blocks for 256 CUs, where the GEMM form's K split is
+// faster (M = 24, us: 7168 columns 16.9 -> 15.9, 3584 15.6 -> 12.1).
+constexpr int64_t kFullN32 = 12288;
 constexpr W8a16Fixed kW8a16Fixed[] = {
     {LF_FP8_ENTRY_W8A16_DENSE, 4096, 0, 0, 1, true, 2, 1, "lf_fp8_w8a16_dense_wide_k4096_m16", kWideN},
     {LF_FP8_ENTRY_W8A16_DENSE, 4096, 0, 0, 2, true, 4, 1, "lf_fp8_w8a16_dense_wide_k4096_m32", kWideN},
@@ -152,7 +171,7 @@ constexpr W8a16Fixed kW8a16Fixed[] = {
     {LF_FP8_ENTRY_W8A16_QKV, 4096, 4096, 1024, 2, true, 8, 4,
      "lf_fp8_w8a16_qkv_k4096_q4096_kv1024_m32"},
     {LF_FP8_ENTRY_W8A16_GATE_UP, 4096, 0, 0, 1, true, 2, 1, "lf_fp8_w8a16_gate_up_k4096_m16"},
-    {LF_FP8_ENTRY_W8A16_GATE_UP, 4096, 0, 0, 2, true, 4, 1, "lf_fp8_w8a16_gate_up_k4096_m32"},
+    {LF_FP8_ENTRY_W8A16_GATE_UP, 4096, 0, 0, 2, true, 4, 1, "lf_fp8_w8a16_gate_up_k4096_m32", kFullN32},
     // the same forms over 128 x 128 block-scaled weights (no wide entries)
     {LF_FP8_ENTRY_W8A16_DENSE_B128, 4096, 0, 0, 1, false, 8, 1, "lf_fp8_w8a16_dense_b128_k4096_m16"},
     {LF_FP8_ENTRY_W8A16_DENSE_B128, 4096, 0, 0, 2, false, 8, 1, "lf_fp8_w8a16_dense_b128_k4096_m32"},
@@ -163,7 +182,7 @@ constexpr W8a16Fixed kW8a16Fixed[] = {
     {LF_FP8_ENTRY_W8A16_QKV_B128, 4096, 4096, 1024, 2, true, 8, 4,
      "lf_fp8_w8a16_qkv_b128_k4096_q4096_kv1024_m32"},
     {LF_FP8_ENTRY_W8A16_GATE_UP_B128, 4096, 0, 0, 1, true, 2, 1, "lf_fp8_w8a16_gate_up_b128_k4096_m16"},
-    {LF_FP8_ENTRY_W8A16_GATE_UP_B128, 4096, 0, 0, 2, true, 4, 1, "lf_fp8_w8a16_gate_up_b128_k4096_m32"},
+    {LF_FP8_ENTRY_W8A16_GATE_UP_B128, 4096, 0, 0, 2, true, 4, 1, "lf_fp8_w8a16_gate_up_b128_k4096_m32", kFullN32},
 };
 
 // The specialized entry for (entry, N, K, Q / K-V split, profile), or null.
@@ -672,9 +691,11 @@ static int64_t w8a16_workspace(int32_t entry, int64_t n, int64_t k, int64_t nq, 
   }
   if (sp.split == 1) return 256;
   // One 1 KiB fp32 accumulator fragment per (slice, 16-column tile, weight,
-  // 16-row tile), then one arrival counter per column group.
+  // 16-row tile), then one arrival counter per column group. The GEMM form
+  // (mt 2, 4) stores whole blocks of tiles.
   const int64_t nw = entry == LF_FP8_ENTRY_W8A16_GATE_UP ? 2 : 1;
-  return align_up(sp.split * (n / 16) * nw * sp.mt * 1024, 256) + align_up(sp.groups * 4, 256);
+  const int64_t tiles = sp.mt == 8 ? n / 16 : sp.groups * kW16Waves;
+  return align_up(sp.split * tiles * nw * sp.mt * 1024, 256) + align_up(sp.groups * 4, 256);
 }
 
 int64_t lunaflux_fp8_w8a16_workspace_bytes(int32_t entry, int64_t n, int64_t k,
@@ -857,7 +878,7 @@ static int32_t launch_geometry(int32_t entry, int64_t n, int64_t k, int64_t nq, 
                     sp.one_tile ? "_t1" : "");
       name = buffer;
       gx = static_cast<int32_t>(sp.groups * sp.split);
-      bx = 64 * (sp.one_tile ? kW16TileWaves : kW16Waves);
+      bx = sp.one_tile ? 64 * kW16TileWaves : w16_threads(sp.mt, false);
       break;
     }
     case LF_FP8_ENTRY_W8A16_DENSE_B128:
@@ -884,7 +905,7 @@ static int32_t launch_geometry(int32_t entry, int64_t n, int64_t k, int64_t nq, 
       std::snprintf(buffer, sizeof(buffer), "lf_fp8_w8a16_%s_b128_m%d", op, 16 * sp.mt);
       name = buffer;
       gx = static_cast<int32_t>(sp.groups * sp.split);
-      bx = 64 * kW16Waves;
+      bx = w16_threads(sp.mt, true);
       break;
     }
     case LF_FP8_ENTRY_W8A8_DENSE_B128:

@@ -236,6 +236,28 @@ def test_launch_geometry():
     assert fp8.act_quant_bytes(3, 512) == 1536 + 256
 
 
+@pytest.mark.parametrize("entry,cols", [(_abi.ENTRY_W8A16_DENSE, 1), (_abi.ENTRY_W8A16_QKV, 1),
+                                        (_abi.ENTRY_W8A16_GATE_UP, 2)])
+@pytest.mark.parametrize("k", [128, 1024, 2048, 2176, 7168, 28672])
+def test_w8a16_any_shape_grid_holds_the_kernels_slices(entry, cols, k):
+    """Profiles of 17..64 rows: the kernel cuts K into max(1, min(256 /
+    blocks, k-tiles / 8)) slices of 64-column blocks; the grid is whole
+    slices, at least that many, and the workspace holds their partial tiles
+    and a counter per block."""
+    for n in (16, 48, 64, 1040, 4096, 7184, 16384, 40000):
+        for m in (17, 32, 33, 64):
+            dims, sym = fp8.launch_geometry(entry, n, k, m)
+            if not sym.endswith(f"_m{m if m in (32, 64) else 32 if m == 17 else 64}") or "_k" in sym:
+                continue
+            rows, blocks = (32 if m <= 32 else 64), -(-n // 64)
+            slices = max(1, min(256 // blocks, k // 128 // 8))
+            assert dims.grid[0] % blocks == 0 and dims.grid[0] // blocks >= slices
+            assert dims.block[0] == (256 if rows == 32 else 512)
+            if slices > 1:
+                need = slices * blocks * 64 * cols * rows * 4
+                assert fp8.w8a16_workspace_bytes(entry, n, k, m) >= need + blocks * 4
+
+
 def test_one_launch_w8a8_geometry_and_workspace():
     """The _aq entries: the GEMM-only entry's tile form, 256 quantizer blocks
     ahead of its tiles, workspace = sync area (128 B + one counter per row

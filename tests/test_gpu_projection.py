@@ -13,7 +13,7 @@ import pytest
 
 import oracle_lib as o
 from lunaflux_amd import synth
-from parity import MAX_ABS, abs_sum, parity
+from parity import MAX_ABS, abs_sum, parity, swiglu_midpoint_tol
 
 pytestmark = pytest.mark.gpu
 
@@ -528,6 +528,62 @@ def lm_head_weight(rt, rng, vocab, k):
     q = np.tile(q0, (reps, 1))[:vocab]
     s = (np.tile(s0, reps) * np.repeat(np.linspace(0.5, 1.5, reps, dtype=np.float32), 2048))[:vocab]
     return q, s.astype(np.float32), rt.upload_weight(q, s.astype(np.float32))
+
+
+@pytest.mark.parametrize("op,n,k,m,max_tokens", [
+    ("dense", 16, 128, 17, 32),        # one fragment of a block's four, one k-tile
+    ("dense", 80, 384, 32, 32),        # a partial second block, three k-tiles
+    ("dense", 4096, 2048, 1, 32),      # two slices of a grid sized for eight
+    ("dense", 1072, 4224, 33, 64),     # four slices of 33 k-tiles, partial block
+    ("qkv", 112, 1024, 29, 32),        # 80 + 16 + 16: three weights in two blocks
+    ("qkv", 1584, 4096, 64, 64),       # 1040 + 272 + 272, boundaries inside blocks
+    ("gate_up", 48, 256, 18, 32),      # part of one 64-column block
+    ("gate_up", 3600, 4096, 50, 64),   # 57 blocks, the last with 16 columns, four slices
+])
+def test_w8a16_gemm_form_any_width(rt, op, n, k, m, max_tokens):
+    """The LDS-tiled GEMM of profiles of 17..64 rows at widths its blocks do
+    not divide and at its shortest and split K: against the oracle over every
+    column; rows past M untouched; three launches on one workspace agree bit
+    for bit."""
+    from lunaflux_amd import _abi, fp8
+    from lunaflux_amd.fp8 import _region
+    rng = np.random.default_rng(9200 + n + k + m)
+    x = synth.activations(rng, m, k)
+    xa = rt.context.upload(np.concatenate([x, np.zeros((max_tokens - m, k), np.uint16)]))
+    ya = rt.context.allocate(max_tokens * n * 2)
+    xr_, yr_, counts = _region(xa, alignment=256), _region(ya, alignment=256), rt.step_counts(m)
+    xr = x_ref(x, "w8a16")
+    extra = {}
+    if op == "gate_up":
+        (qg, sg, wg), (qu, su, wu) = make_weight(rt, rng, n, k), make_weight(rt, rng, n, k)
+        bound = rt.bind_gate_up("w8a16", counts, xr_, wg, wu, yr_, max_tokens)
+        g, u = o.dense_projection(xr, deq(qg, sg)), o.dense_projection(xr, deq(qu, su))
+        ref = o.silu_mul_array(g, u)
+        # an ulp of bf16 at |h| in [4, 8) is 0.03: allowed only where the
+        # two sides' summation bounds reach across a rounding midpoint
+        extra = dict(midpoint_tol=swiglu_midpoint_tol(g, u, abs_sum(xr, deq(qg, sg)), abs_sum(xr, deq(qu, su)), k))
+    else:
+        if op == "qkv":
+            nkv = n // 7 // 16 * 16 + (48 if n > 1000 else 0)
+            ws = [make_weight(rt, rng, r, k) for r in (n - 2 * nkv, nkv, nkv)]
+            bound = rt.bind_qkv("w8a16", counts, xr_, *(w for _, _, w in ws), yr_, max_tokens)
+        else:
+            ws = [make_weight(rt, rng, n, k)]
+            bound = rt.bind_dense("w8a16", counts, xr_, ws[0][2], yr_, max_tokens)
+        wr = deq(np.concatenate([q for q, _, _ in ws]), np.concatenate([s for _, s, _ in ws]))
+        ref = o.dense_projection(xr, wr)
+        extra = dict(k=k, s_abs=abs_sum(xr, wr))
+    sym = bound.steps[0].name
+    assert sym == f"lf_fp8_w8a16_{op}_m{max_tokens}", sym
+    ya.copy_from_host(np.full(max_tokens * n, 0x7FC1, np.uint16))
+    outs = []
+    for _ in range(3):
+        bound.launch(rt.stream, synchronous=True)
+        outs.append(ya.read(np.uint16, (max_tokens, n)))
+    for y in outs:
+        assert np.all(y[m:] == 0x7FC1), f"{sym}: rows past M written"
+        parity(y[:m], ref, label=f"{sym} n={n} k={k} m={m}", **extra)
+    assert all(np.array_equal(outs[0], y) for y in outs[1:]), f"{sym}: launches differ"
 
 
 @pytest.mark.parametrize("m,max_tokens,family", [(1, 16, "w8a16"), (13, 16, "w8a16"),
