@@ -5,6 +5,7 @@
 #include "w8a8_v3.h"
 #include "w8a8_v4.h"
 #include "w8a8_v5.h"
+#include "w8a8_v6.h"
 
 namespace {
 
@@ -1284,139 +1285,55 @@ LF_DEVICE void w8a8_b128_one_launch(const int32_t *counts, const uint16_t *x, co
 }
 
 // ---------------------------------------------------------------------------
-// Block-scaled W8A8 on 256 x 256 tiles (the eight-wave half-step loop of
-// w8a8_v4.h with swapped operands, as the block-scaled MoE GEMMs), which
-// the launch geometry picks for profiles of at least 192 such tiles (fewer:
-// the 128 x 128 form above keeps more CUs busy). The accumulators hold
-// acc / sigma_kt with sigma_kt = a[row][kt] w[block][kt] (each scale
-// sequence carries its last nonzero value forward, carry_ratio: a zero scale
-// belongs only to an all-zero group, whose products are zero); before
-// k-tile kt's first MFMA into a column fragment they are multiplied by
-// sigma_{kt-1} / sigma_kt, and the epilogue multiplies by the last sigma.
-// No table of all k-tiles fits beside the 128 KiB stage ring at these K
-// (32-112 k-tiles), so each stage also side-loads its k-tile's activation
-// scales of the tile's 256 rows into a two-slot LDS window, and the weight
-// scales are scalar loads.
+// Block-scaled W8A8 on 256-row bands (w8a8_v6.h: eight waves, each k-tile's
+// products folded into the sums with that k-tile's scales): 256 x 256 tiles
+// from 192 such tiles on, 256 x 128 tiles below that, as the launch geometry
+// picks. No table of all k-tiles' scales fits beside the stage ring (32-112
+// k-tiles), so each stage also side-loads its k-tile's activation scales of
+// the tile's 256 rows into an LDS window; the weight scales are scalar
+// loads. Both tiles compute the same sums bit for bit. Bound by the matrix
+// pipes at the clock the chip holds, and by the loads from L2 (32 bytes per
+// clock and CU at 256 x 256). Against the loop before (accumulators kept
+// divided by the current scale and multiplied by the ratio of successive
+// scales between MFMAs; kernel times, M = 2048, us): qkv 78.5 -> 72.4, o
+// 56.8 -> 50.5, GatedMlp 520 -> 461 (1.39 -> 1.56 PFLOP/s with both
+// quantizer steps inside).
 // ---------------------------------------------------------------------------
-using B128V4Tile = w8a8v4::Tile<256, 256, 4, 4, 2>;
-// 256 x 128 tiles: eight waves of 32 x 128 (each wave's columns still one
-// 128-column block), for launches with too few 256 x 256 tiles
-using B128V4TileN128 = w8a8v4::Tile<256, 128, 4, 8, 1>;
-constexpr int kB128V4BM = 256;
+// 256 x 256 (WIDE: 128 x 64 wave tiles, two stages) and 256 x 128 tiles (64 x
+// 64 wave tiles, three stages) of eight waves.
+template <bool WIDE>
+using B128Tile6 = std::conditional_t<WIDE, w8a8v6::Tile<256, 256, 2, 4, 2>, w8a8v6::Tile<256, 128, 4, 2, 3>>;
+constexpr int kB128WideBM = 256;
+// LDS scale window (floats)
+template <bool WIDE>
+constexpr int kB128Win6 = B128Tile6<WIDE>::kScaleSlots * kB128WideBM;
 
-// Side loads (w8a8v4 mainloop SIDE): stage s loads the 256 row scales of
-// k-tile s / 2 (1 KiB of scales_t[kt][m0 ..]) into window slot (s / 2) & 1;
-// both stages of a k-tile load the same bytes, so every stage has one load
-// per wave and the waits stay uniform. Wave w loads rows 64 (w % 4) .. + 63,
-// one dword per lane (waves w and w + 4 write the same bytes: a load with
-// only some lanes active, a branch inside the half-step, cost the loop 70-190
-// spilled registers). Slot reuse: k-tile kt + 2's first load is issued after
-// the block barrier of half-step 2 kt + 1, when every wave has read k-tile
-// kt's slot (at the start of half-step 2 kt); the second load of a k-tile
-// rewrites its slot with the same bytes.
-template <class T>
-struct B128V4Side {
-  static constexpr int kIns = 1;
-  const uint8_t *base;  // scales_t + m0 (wave-uniform)
-  uint64_t stride;      // bytes per k-tile: cap * 4
-  uint32_t win;         // LDS byte offset of the window [2][kBM] fp32
-  LF_DEVICE void issue(int s, int) const {
-    static_assert(T::kBM == 256 && T::kWaves == 8, "four waves cover the 256 rows");
-    const int lane = threadIdx.x & 63, part = (static_cast<int>(threadIdx.x) >> 6) & 3;
-    const int kt = s >> 1;
-    w8a8v3::dma4(w8a8v3::uniform_ptr(base + static_cast<uint64_t>(kt) * stride),
-                 static_cast<uint32_t>(64 * part + lane) * 4,
-                 win + static_cast<uint32_t>(kt & 1) * T::kBM * 4 + static_cast<uint32_t>(part) * 256);
-  }
-};
-
-// Rescale (w8a8v4 mainloop RESCALE, swapped layout: lane l holds row
-// row0 + 32 i of fragment i). Part 1: the up fragments of gate/up (column
-// fragments kFN / 2 ..), whose weight block scales are the up weight's.
-// The loop runs on a copy of the functor, so after the last k-tile's
-// begin() the final sigma factors go to LDS (last: the tile's 256 row
-// scales, then two per wave) for the epilogue.
-template <class T, int MODE>
-struct B128V4Rescale {
-  static constexpr int kParts = MODE == 2 ? 2 : 1;
-  typedef const __attribute__((address_space(3))) float *lds_ptr;
-  typedef __attribute__((address_space(3))) float *lds_wptr;
-  lds_ptr win;                 // [2][kBM] row scales (B128V4Side)
-  lds_wptr last;               // [kBM + 2 kWaves]: last nonzero row / block scales
-  int row0;                    // the lane's row of fragment 0 in the tile
-  int KT;
-  const float *sw[kParts];     // this wave's block scales [KT] per part (wave-uniform)
-  float prev_a[T::kFM];        // last nonzero row scale so far (1 before any)
-  float prev_w[kParts];
-  float m[kParts][T::kFM];     // this k-tile's multipliers
-  LF_DEVICE void begin(int kt) {
-    float rw[kParts];
-#pragma unroll
-    for (int p = 0; p < kParts; ++p) rw[p] = carry_ratio(sload(sw[p], kt), prev_w[p]);
-#pragma unroll
-    for (int i = 0; i < T::kFM; ++i) {
-      const float ra = carry_ratio(win[(kt & 1) * T::kBM + row0 + 32 * i], prev_a[i]);
-#pragma unroll
-      for (int p = 0; p < kParts; ++p) m[p][i] = kt == 0 ? 1.0f : ra * rw[p];
-    }
-    if (kt == KT - 1) {
-      // (lanes l and l + 32 hold the same rows: the same values)
-#pragma unroll
-      for (int i = 0; i < T::kFM; ++i) last[row0 + 32 * i] = prev_a[i];
-      const int wave = threadIdx.x >> 6;
-#pragma unroll
-      for (int p = 0; p < kParts; ++p) last[T::kBM + 2 * wave + p] = prev_w[p];
-    }
-  }
-  template <class A>
-  LF_DEVICE void apply(int o, A &acc) {
-    const int p = kParts == 2 && o >= T::kFN / 2 ? 1 : 0;
-#pragma unroll
-    for (int i = 0; i < T::kFM; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][o][e] *= m[p][i];
-  }
-};
-
-// The GEMM on one 256 x 256 tile of M live rows of a workspace sized for
-// cap rows (codes [cap, K], scales_t [K / 128][cap]); operand mapping and
-// gate as w8a8_b128_gemm; win: the block's LDS window (2 x 256 floats), then
-// kBM + 2 kWaves floats for the final scales.
-template <class T, int GROUP, int MODE, bool THROUGH = false, class Gate = Open>
-LF_DEVICE int w8a8_b128_v4_gemm(uint8_t *smem, float *win, int M, const uint8_t *xq, const float *scales_t,
-                                int cap, const uint8_t *w0, const uint8_t *w1, const uint8_t *w2, uint16_t *y,
-                                int bid, const Gate &gate) {
-  constexpr int BM = T::kBM, BN = T::kBN;
-  static_assert(T::kWaveN == 128 && BM == kB128V4BM, "a wave's columns are one 128-column block");
+// One tile (column block bx, rows m0 ..) of M live rows of a
+// workspace sized for cap rows (codes [cap, K], scales_t [K / 128][cap]);
+// operand mapping as w8a8_b128_gemm.
+template <class T, int MODE, bool THROUGH>
+LF_DEVICE void w8a8_b128_tile6(uint8_t *smem, float *win, int M, const uint8_t *xq, const float *scales_t, int cap,
+                               const uint8_t *w0, const uint8_t *w1, const uint8_t *w2, uint16_t *y, int ld, int bx,
+                               int m0) {
+  constexpr int BN = T::kBN;
+  constexpr int kParts = MODE == 2 ? 2 : 1;
   const WeightHeader &h0 = header_of(w0);
   const int K = static_cast<int>(h0.columns);
   const int KT = K >> 7;
   const int tq = static_cast<int>(h0.rows) >> 4;
   const int tk = MODE == 1 ? static_cast<int>(header_of(w1).rows) >> 4 : 0;
-  const int ld = dense_ld<MODE>(w0, w1, w2);
-  const int gx = dense_gx<MODE, BN>(ld);
-  int bx, by;
-  if (!w8a8v3::tile_of_block(bid, gx, (M + BM - 1) / BM, GROUP, bx, by)) return -1;
-  const int m0 = by * BM;
-  // 32-bit activation offsets (below 256 K) need K < 2^24
-  if (K >= (1 << 24)) {
-    poison_tile<MODE, BN>(y, ld, M, m0, BM, bx);
-    return by;
-  }
-  if (!gate(m0)) return -1;
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int wm = wave / T::kWgn, wn = wave % T::kWgn;
-
-  // Weight tile of block-local tile s (the mapping of w8a8_v4_kernel).
+  // Weight tile of block-local slot s; gate/up: each wave column's kFN slots
+  // are kFN / 2 gate tiles, then the up tiles of the same columns.
   auto slot = [&](int s, const uint8_t *&region, int &t, int &ocol) {
     if (MODE == 2) {
-      const int sw = s / (2 * T::kFN), f = s % (2 * T::kFN);
-      const bool up = f >= T::kFN;
-      const int col = bx * (BN / 2) + sw * (T::kWaveN / 2) + 16 * (up ? f - T::kFN : f);
+      const int sw = s / T::kFN, f = s % T::kFN;
+      const bool up = f >= T::kFN / 2;
+      ocol = bx * (BN / 2) + sw * (T::kWaveN / 2) + 16 * (up ? f - T::kFN / 2 : f);
       region = up ? w1 : w0;
-      t = col >> 4;
-      ocol = col;
+      t = ocol >> 4;
     } else {
       t = bx * (BN / 16) + s;
       ocol = t * 16;
@@ -1432,119 +1349,105 @@ LF_DEVICE int w8a8_b128_v4_gemm(uint8_t *smem, float *win, int M, const uint8_t 
       }
     }
   };
-
-  w8a8v4::Plan<T> plan;
+  w8a8v6::Plan<T> plan;
   plan.a_base = w8a8v3::uniform_ptr(xq + static_cast<uint64_t>(m0) * K);
 #pragma unroll
   for (int q = 0; q < T::kAIns; ++q) {
-    const int tr = w8a8v4::a_load_row<T>(wave, q, lane);
+    const int tr = w8a8v3::a_load_row<T>(wave, q, lane);
     const int row = m0 + tr < M ? tr : M - 1 - m0;
-    plan.a_off[q] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) + w8a8v4::a_load_slot(tr, lane) * 32;
+    plan.a_off[q] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) + w8a8v3::a_load_chunk(tr, lane) * 16;
   }
 #pragma unroll
   for (int q = 0; q < T::kBIns; ++q) {
+    const int half = w8a8v3::b_load_half<T>(wave, q);
     const uint8_t *region;
     int t, ocol;
-    slot(w8a8v4::b_load_tile<T>(wave, q), region, t, ocol);
-    plan.b_base[q] = w8a8v3::uniform_ptr(expert_tiles(region, 0) + static_cast<uint64_t>(t) * KT * kTileBytes);
+    slot(half >> 1, region, t, ocol);
+    plan.b_base[q] = w8a8v3::uniform_ptr(expert_tiles(region, 0) + static_cast<uint64_t>(t) * KT * kTileBytes +
+                                         (half & 1) * 1024);
   }
   plan.b_lane = lane * 16;
-
-  // This wave's 128-column block: (gate/up) its 64 gate and 64 up columns
-  // lie in one 128-row block of each weight; (dense, QKV) its 128 columns
-  // are one block of one region (every QKV width is a multiple of 128).
-  typedef const __attribute__((address_space(3))) float *lds_ptr;
-  typedef __attribute__((address_space(3))) float *lds_wptr;
-  float *last = win + 2 * BM;
-  B128V4Rescale<T, MODE> rs;
-  rs.win = (lds_ptr)(win);
-  rs.last = (lds_wptr)(last);
-  rs.row0 = wm * T::kWaveM + (lane & 31);
-  rs.KT = KT;
+  // A wave's columns (gate/up: of each weight) lie in one 128-row block.
+  w8a8v6::DenseScales<T, kParts> scales;
+  scales.base = w8a8v3::uniform_ptr(reinterpret_cast<const uint8_t *>(scales_t + m0));
+  scales.stride = static_cast<uint64_t>(cap) * 4;
+  scales.win = win;
+  scales.win_offset = w8a8v3::lds_offset_of(reinterpret_cast<uint8_t *>(win));
+  scales.row0 = wm * T::kWaveM + (lane & 15);
+  int col0 = 0;
 #pragma unroll
-  for (int p = 0; p < B128V4Rescale<T, MODE>::kParts; ++p) {
+  for (int p = 0; p < kParts; ++p) {
     const uint8_t *region;
     int t, ocol;
-    slot(wn * (T::kWaveN / 16) + p * T::kFN, region, t, ocol);
-    rs.sw[p] = reinterpret_cast<const float *>(w8a8v3::uniform_ptr(
-        reinterpret_cast<const uint8_t *>(expert_scales(region, 0) + static_cast<uint64_t>(t >> 3) * KT)));
-    rs.prev_w[p] = 1.0f;
+    slot(wn * T::kFN + p * (T::kFN / 2), region, t, ocol);
+    scales.sw[p] = uniform_f32(expert_scales(region, 0) + static_cast<uint64_t>(t >> 3) * KT);
+    if (p == 0) col0 = __builtin_amdgcn_readfirstlane(ocol);
   }
-#pragma unroll
-  for (int i = 0; i < T::kFM; ++i) rs.prev_a[i] = 1.0f;
-  const B128V4Side<T> side{w8a8v3::uniform_ptr(reinterpret_cast<const uint8_t *>(scales_t + m0)),
-                           static_cast<uint64_t>(cap) * 4,
-                           w8a8v3::lds_offset_of(reinterpret_cast<uint8_t *>(win))};
-  w8a8v4::f32x16 acc[T::kFM][T::kFN];
-  w8a8v4::mainloop<T, false, B128V4Rescale<T, MODE>, true, B128V4Side<T>>(plan, KT, smem, acc, T::kFM, rs,
-                                                                         true, side);
-  // the final sigma factors (this lane wrote its rows' and its wave's)
-  float sa_last[T::kFM], sw_last[B128V4Rescale<T, MODE>::kParts];
-#pragma unroll
-  for (int i = 0; i < T::kFM; ++i) sa_last[i] = last[rs.row0 + 32 * i];
-#pragma unroll
-  for (int p = 0; p < B128V4Rescale<T, MODE>::kParts; ++p) sw_last[p] = last[BM + 2 * wave + p];
+  f32x4 acc[T::kFM][T::kFN];
+  w8a8v6::mainloop<T, w8a8v6::DenseScales<T, kParts>>(plan, KT, smem, acc, scales);
 
-  // Epilogue (swapped layout: element 4 g + q of fragment j is column
-  // 32 j + 8 g + 4 (lane / 32) + q): times the last sigma, staged through
-  // LDS one 32-row fragment at a time in 16-byte row chunks.
-  const int rl = lane & 31, c4 = 4 * (lane >> 5);
+  // Epilogue: element q of fragment (i, j) is row 16 i + lane % 16, column
+  // 16 j + 4 (lane / 16) + q of the wave tile; staged through LDS.
   constexpr int kCols = MODE == 2 ? T::kWaveN / 2 : T::kWaveN;
-  using Stage = w8a8v4::StageTile<uint16_t, 32, kCols>;
+  constexpr int kRows = 64;  // staged at a time
+  using Stage = w8a8v4::StageTile<uint16_t, kRows, kCols>;
   static_assert(Stage::kBytes * T::kWaves <= T::kSmem, "staging fits the stage ring");
-  int col0;
-  {
-    const uint8_t *region;
-    int t;
-    slot(wn * (T::kWaveN / 16), region, t, col0);
-  }
-  col0 = __builtin_amdgcn_readfirstlane(col0);
   w8a8v4::epilogue_barrier();
   const Stage st{reinterpret_cast<uint16_t *>(smem + wave * Stage::kBytes)};
 #pragma unroll
   for (int i = 0; i < T::kFM; ++i) {
-    const float sa = sa_last[i];
-    if constexpr (MODE == 2) {
+    constexpr int kOut = MODE == 2 ? T::kFN / 2 : T::kFN;
 #pragma unroll
-      for (int j = 0; j < T::kFN / 2; ++j)
+    for (int j = 0; j < kOut; ++j) {
+      uint32_t b[4];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          uint32_t b[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float gv = acc[i][j][4 * g + q] * sa * sw_last[0];
-            const float uv = acc[i][j + T::kFN / 2][4 * g + q] * sa * sw_last[B128V4Rescale<T, MODE>::kParts - 1];
-            b[q] = f32_to_bf16(silu_mul(gv, uv));
-          }
-          st.put4(rl, 32 * j + 8 * g + c4, b);
-        }
-    } else {
-#pragma unroll
-      for (int j = 0; j < T::kFN; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          uint32_t b[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) b[q] = f32_to_bf16(acc[i][j][4 * g + q] * sa * sw_last[0]);
-          st.put4(rl, 32 * j + 8 * g + c4, b);
-        }
+      for (int q = 0; q < 4; ++q) {
+        const float v = acc[i][j][q];
+        b[q] = f32_to_bf16(MODE == 2 ? silu_mul(v, acc[i][j + T::kFN - kOut][q]) : v);
+      }
+      st.put4(16 * i % kRows + (lane & 15), 16 * j + 4 * (lane >> 4), b);
     }
-    const int mw = m0 + wm * T::kWaveM + 32 * i;
-    st.template flush<THROUGH>(lane, [&](int row) -> uint16_t * {
-      return mw + row < M ? y + static_cast<uint64_t>(mw + row) * ld + col0 : nullptr;
-    });
+    if (16 * (i + 1) % kRows == 0) {
+      const int mw = m0 + wm * T::kWaveM + 16 * (i + 1) - kRows;
+      st.template flush<THROUGH>(lane, [&](int row) -> uint16_t * {
+        return mw + row < M ? y + static_cast<uint64_t>(mw + row) * ld + col0 : nullptr;
+      });
+    }
   }
+}
+
+// The GEMM on one block's tile: gate and the returned band as in
+// w8a8_b128_gemm.
+template <bool WIDE, int GROUP, int MODE, bool THROUGH = false, class Gate = Open>
+LF_DEVICE int w8a8_b128_wide_gemm(uint8_t *smem, float *win, int M, const uint8_t *xq, const float *scales_t,
+                                  int cap, const uint8_t *w0, const uint8_t *w1, const uint8_t *w2, uint16_t *y,
+                                  int bid, const Gate &gate) {
+  using T = B128Tile6<WIDE>;
+  constexpr int BM = T::kBM, BN = T::kBN;
+  const int K = static_cast<int>(header_of(w0).columns);
+  const int ld = dense_ld<MODE>(w0, w1, w2);
+  int bx, by;
+  if (!w8a8v3::tile_of_block(bid, dense_gx<MODE, BN>(ld), (M + BM - 1) / BM, GROUP, bx, by)) return -1;
+  const int m0 = by * BM;
+  // 32-bit activation offsets (below 256 K) need K < 2^24
+  if (K >= (1 << 24)) {
+    poison_tile<MODE, BN>(y, ld, M, m0, BM, bx);
+    return by;
+  }
+  if (!gate(m0)) return -1;
+  w8a8_b128_tile6<T, MODE, THROUGH>(smem, win, M, xq, scales_t, cap, w0, w1, w2, y, ld, bx, m0);
   return by;
 }
 
 // The block-scaled operations in one launch on the 256 x 256 (or 256 x 128)
 // form: as w8a8_b128_one_launch with 256-row bands (cap = bands x 256).
-template <class T, int MODE>
-LF_DEVICE void w8a8_b128_v4_one_launch(const int32_t *counts, const uint16_t *x, const uint8_t *w0,
+template <bool WIDE, int MODE>
+LF_DEVICE void w8a8_b128_wide_one_launch(const int32_t *counts, const uint16_t *x, const uint8_t *w0,
                                        const uint8_t *w1, const uint8_t *w2, uint16_t *y, uint8_t *ws) {
-  constexpr int BM = kB128V4BM;
+  using T = B128Tile6<WIDE>;
+  constexpr int BM = kB128WideBM;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[T::kSmem];
-  __shared__ __attribute__((aligned(16))) float win[2 * BM + BM + 2 * T::kWaves];
+  __shared__ __attribute__((aligned(16))) float win[kB128Win6<WIDE>];
   __shared__ phase::Flag flag;
   if (!dense_regions_ok<MODE, kScaleBlock128>(w0, w1, w2)) return;
   const int K = static_cast<int>(header_of(w0).columns);
@@ -1565,7 +1468,7 @@ LF_DEVICE void w8a8_b128_v4_one_launch(const int32_t *counts, const uint16_t *x,
     const int band = m0 / BM;
     return phase::wait_for(sync, sync.band(0, band), chunks_in_band(M, band, BM), flag);
   };
-  w8a8_b128_v4_gemm<T, 4, MODE>(smem, win, M, rows.codes, rows.scales_t, cap, w0, w1, w2, y,
+  w8a8_b128_wide_gemm<WIDE, 4, MODE>(smem, win, M, rows.codes, rows.scales_t, cap, w0, w1, w2, y,
                                 b - kQuantBlocks, gate);
   phase::finish(sync, blocks, 1, flag);
 }
@@ -1579,19 +1482,17 @@ LF_DEVICE void w8a8_b128_v4_one_launch(const int32_t *counts, const uint16_t *x,
 template <int FORM>
 struct B128Form {
   static_assert(FORM == 0 || FORM == 2, "GatedMlp tile forms");
-  using T = std::conditional_t<FORM == 2, B128V4Tile, std::conditional_t<FORM == 1, B128V4TileN128, B128Tile>>;
-  static constexpr int kBM = FORM ? kB128V4BM : kB128BM, kBN = FORM == 2 ? 256 : 128;
-  // LDS scale window: (256-row forms) two k-tile slots, then the final
-  // scales; (128 x 128) one slot per stage
-  static constexpr int kWin = FORM ? 3 * kBM + 2 * T::kWaves : T::kStages * kBM;
+  using T = std::conditional_t<FORM != 0, B128Tile6<true>, B128Tile>;
+  static constexpr int kBM = FORM ? kB128WideBM : kB128BM, kBN = FORM == 2 ? 256 : 128;
+  static constexpr int kWin = FORM ? kB128Win6<true> : T::kStages * kBM;  // LDS scale window
 };
 
 template <int FORM, int MODE, bool THROUGH, class Gate>
 LF_DEVICE int w8a8_b128_form_gemm(uint8_t *smem, float *win, int M, const B128Rows &rows, int cap,
                                   const uint8_t *w0, const uint8_t *w1, uint16_t *out, int bid, const Gate &gate) {
   if constexpr (FORM != 0) {
-    return w8a8_b128_v4_gemm<typename B128Form<FORM>::T, 4, MODE, THROUGH>(smem, win, M, rows.codes, rows.scales_t,
-                                                                          cap, w0, w1, w1, out, bid, gate);
+    return w8a8_b128_wide_gemm<FORM == 2, 4, MODE, THROUGH>(smem, win, M, rows.codes, rows.scales_t, cap, w0, w1,
+                                                            w1, out, bid, gate);
   } else {
     return w8a8_b128_gemm<B128Tile, 4, MODE, THROUGH>(smem, win, M, rows.codes, rows.scales_t, cap, w0, w1, w1,
                                                       out, bid, gate);
@@ -1826,36 +1727,36 @@ __global__ __launch_bounds__(256) void lf_fp8_w8a8_gate_up_b128(const int32_t *c
 // such tiles (lunaflux_fp8_launch_geometry picks the form).
 __global__ __launch_bounds__(512) void lf_fp8_w8a8_dense_b128_t256(const int32_t *counts, const uint16_t *x,
                                                                    const uint8_t *w, uint16_t *y, uint8_t *ws) {
-  w8a8_b128_v4_one_launch<B128V4Tile, 0>(counts, x, w, w, w, y, ws);
+  w8a8_b128_wide_one_launch<true, 0>(counts, x, w, w, w, y, ws);
 }
 __global__ __launch_bounds__(512) void lf_fp8_w8a8_qkv_b128_t256(const int32_t *counts, const uint16_t *x,
                                                                  const uint8_t *wq, const uint8_t *wk,
                                                                  const uint8_t *wv, uint16_t *y, uint8_t *ws) {
-  w8a8_b128_v4_one_launch<B128V4Tile, 1>(counts, x, wq, wk, wv, y, ws);
+  w8a8_b128_wide_one_launch<true, 1>(counts, x, wq, wk, wv, y, ws);
 }
 __global__ __launch_bounds__(512) void lf_fp8_w8a8_gate_up_b128_t256(const int32_t *counts, const uint16_t *x,
                                                                      const uint8_t *wg, const uint8_t *wu,
                                                                      uint16_t *h, uint8_t *ws) {
-  w8a8_b128_v4_one_launch<B128V4Tile, 2>(counts, x, wg, wu, wu, h, ws);
+  w8a8_b128_wide_one_launch<true, 2>(counts, x, wg, wu, wu, h, ws);
 }
 // The same on 256 x 128 tiles (eight waves of 32 x 128), where 256 x 256
 // tiles would be too few.
 __global__ __launch_bounds__(512) void lf_fp8_w8a8_dense_b128_t256x128(const int32_t *counts,
                                                                        const uint16_t *x, const uint8_t *w,
                                                                        uint16_t *y, uint8_t *ws) {
-  w8a8_b128_v4_one_launch<B128V4TileN128, 0>(counts, x, w, w, w, y, ws);
+  w8a8_b128_wide_one_launch<false, 0>(counts, x, w, w, w, y, ws);
 }
 __global__ __launch_bounds__(512) void lf_fp8_w8a8_qkv_b128_t256x128(const int32_t *counts, const uint16_t *x,
                                                                      const uint8_t *wq, const uint8_t *wk,
                                                                      const uint8_t *wv, uint16_t *y,
                                                                      uint8_t *ws) {
-  w8a8_b128_v4_one_launch<B128V4TileN128, 1>(counts, x, wq, wk, wv, y, ws);
+  w8a8_b128_wide_one_launch<false, 1>(counts, x, wq, wk, wv, y, ws);
 }
 __global__ __launch_bounds__(512) void lf_fp8_w8a8_gate_up_b128_t256x128(const int32_t *counts,
                                                                          const uint16_t *x, const uint8_t *wg,
                                                                          const uint8_t *wu, uint16_t *h,
                                                                          uint8_t *ws) {
-  w8a8_b128_v4_one_launch<B128V4TileN128, 2>(counts, x, wg, wu, wu, h, ws);
+  w8a8_b128_wide_one_launch<false, 2>(counts, x, wg, wu, wu, h, ws);
 }
 __global__ __launch_bounds__(256) void lf_fp8_w8a8_gated_mlp_b128(const int32_t *counts, const uint16_t *x,
                                                                   const uint8_t *wg, const uint8_t *wu,
