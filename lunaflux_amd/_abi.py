@@ -136,6 +136,7 @@ SIGNATURES = {
     "lunaflux_fp8_moe_sync_offset": (_i64, [_vp, _i32]),
     "lunaflux_fp8_moe_workspace_layout": (_i32, [_vp, _i32, _i64p]),
     "lunaflux_fp8_moe_launch_geometry": (_i32, [_i32, _vp, _i32, _i32p, ctypes.c_char_p]),
+    "lunaflux_fp8_moe_step_geometry": (_i32, [_i32, _vp, _i32, _i32p, ctypes.c_char_p]),
 }
 
 MOE_ROUTE, MOE_SORT, MOE_QUANT_TOKENS, MOE_GATE_UP, MOE_QUANT_HIDDEN, MOE_DOWN, MOE_COMBINE = range(1, 8)

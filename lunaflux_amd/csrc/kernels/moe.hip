@@ -1130,6 +1130,197 @@ __device__ __forceinline__ void grouped_gemm_t256(const int32_t *counts, const M
   }
 }
 
+// Grouped GEMM on 128 x 256 tiles (w8a8_v6.h: eight 64 x 64 waves, three
+// stages, one block per CU) over the 128-row tiles of all experts, for
+// block-scaled weights. STAGE 0: 128 h-columns per block; STAGE 1: 256
+// columns. QUANT (gate/up): the epilogue quantizes the block's 128
+// h-columns, which are one scale group, as grouped_gemm_t256's does, and h is
+// not stored. The activation scales of the tile's rows sit in an LDS table
+// [KT][128] (K <= 128 kT128x256MaxKT).
+// Why this tile: an expert's last tile is half of one on average, and at a
+// few hundred rows per expert 256-row tiles spend a third of their rows on
+// that; 256 columns keep two stages of 32 KiB of weights in flight per CU,
+// which streams the weights of experts with few rows (60 tokens, 64
+// experts: 4.0 TB/s against 2.0 on 128 x 128 tiles with one 16 KiB stage
+// ahead in each of two blocks). The sizes measured are at the rule
+// (csrc/pack.cpp, moe_t128x256).
+using GemmTile128x256 = w8a8v6::Tile<128, 256, 2, 4, 3>;
+constexpr int kT128x256MaxKT = 24;
+
+struct GroupedScales {
+  static constexpr bool kFold = true;
+  static constexpr int kIns = 0, kParts = 2;
+  typedef const __attribute__((address_space(3))) float *lds_ptr;
+  lds_ptr sa;          // [KT][128]
+  const float *sw[2];  // this wave's block scales [KT] of the gate and up (STAGE 1: of all) fragments
+  int row0;            // this lane's row of fragment 0
+  LF_DEVICE void issue(int) const {}
+  LF_DEVICE float row(int kt, int i) const { return sa[kt * w8a8::kBM + row0 + 16 * i]; }
+  LF_DEVICE float block(int kt, int p) const { return sload(sw[p], kt); }
+};
+
+template <int STAGE, bool QUANT>
+__device__ __forceinline__ void grouped_gemm_t128x256(const int32_t *counts, const MoeDesc &d, const uint8_t *w0,
+                                                      const uint8_t *w1, uint8_t *ws) {
+  static_assert(!QUANT || STAGE == 0, "the fused quantizer is the gate/up's");
+  using T = GemmTile128x256;
+  constexpr int BM = T::kBM;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[T::kSmem];
+  __shared__ __attribute__((aligned(16))) float scale_lds[kT128x256MaxKT * BM];
+  const int Tn = live_rows(counts, 1 << 30);
+  if (Tn == 0) return;
+  const MoeLayout L(d, Tn);
+  const int E = d.experts;
+  const int32_t *tiles = at<int32_t>(ws, L.tiles);
+  const WeightHeader &h0 = header_of(w0);
+  const int K = static_cast<int>(h0.columns);
+  const int KT = K >> 7;
+  const int N = static_cast<int>(h0.rows);
+  // what the launch geometry checks: 32-bit activation offsets, the table
+  const uint64_t a_rows = STAGE == 0 ? static_cast<uint64_t>(Tn) : static_cast<uint64_t>(Tn) * d.top_k;
+  if (a_rows * static_cast<uint64_t>(K) >= (uint64_t(1) << 32) || KT > kT128x256MaxKT) return;
+  const int gx = STAGE == 0 ? N / (T::kBN / 2) : N / T::kBN;
+  int bx, by;
+  if (!w8a8v3::tile_of_block(gx, tiles[E], tiles[E], bx, by)) return;
+  const TileExpert te = find_tile_expert(tiles, at<int32_t>(ws, L.offsets), E, by);
+  const int e = te.e;
+  const int p0 = te.row_begin + (by - te.first_tile) * BM;
+  const int pend = te.row_end;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int wm = wave / T::kWgn, wn = wave % T::kWgn;
+  const int32_t *sorted = at<int32_t>(ws, L.sorted);
+  auto src_row = [&](int p) { return STAGE == 0 ? sorted[p] / d.top_k : p; };
+  // Weight tile of block-local slot s.
+  auto slot = [&](int s, const uint8_t *&region, int &col) {
+    if (STAGE == 0) {
+      const int sw = s / T::kFN, f = s % T::kFN;
+      const bool up = f >= T::kFN / 2;
+      col = bx * (T::kBN / 2) + sw * (T::kWaveN / 2) + 16 * (up ? f - T::kFN / 2 : f);
+      region = up ? w1 : w0;
+    } else {
+      col = bx * T::kBN + 16 * s;
+      region = w0;
+    }
+  };
+
+  w8a8v6::Plan<T> plan;
+  plan.a_base = w8a8v3::uniform_ptr(at<uint8_t>(ws, STAGE == 0 ? L.xq : L.hq));
+#pragma unroll
+  for (int q = 0; q < T::kAIns; ++q) {
+    const int tr = w8a8v3::a_load_row<T>(wave, q, lane);
+    const int p = p0 + tr < pend ? p0 + tr : p0;  // dead rows re-read the first row
+    plan.a_off[q] = static_cast<uint32_t>(src_row(p)) * static_cast<uint32_t>(K) +
+                    w8a8v3::a_load_chunk(tr, lane) * 16;
+  }
+#pragma unroll
+  for (int q = 0; q < T::kBIns; ++q) {
+    const int half = w8a8v3::b_load_half<T>(wave, q);
+    const uint8_t *region;
+    int col;
+    slot(half >> 1, region, col);
+    plan.b_base[q] = w8a8v3::uniform_ptr(expert_tiles(region, e) + static_cast<uint64_t>(col >> 4) * KT * kTileBytes +
+                                         (half & 1) * 1024);
+  }
+  plan.b_lane = lane * 16;
+
+  const int live_rows_wave = pend - (p0 + wm * T::kWaveM);
+  const int live_fm = live_rows_wave <= 0 ? 0 : live_rows_wave >= T::kWaveM ? T::kFM : (live_rows_wave + 15) / 16;
+  f32x4 acc[T::kFM][T::kFN];
+  const int tid = static_cast<int>(threadIdx.x);
+  {
+    // thread: row tid % 128, k-tiles tid / 128, + 4, ... (all loads in flight)
+    const float *ascales = at<float>(ws, STAGE == 0 ? L.xs : L.hs);
+    const int row = tid & (BM - 1), k0 = tid / BM;
+    constexpr int kStep = T::kThreads / BM, kPer = kT128x256MaxKT / kStep;
+    const float *sr = ascales + static_cast<uint64_t>(src_row(p0 + row < pend ? p0 + row : p0)) * KT;
+    float sv[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) sv[i] = k0 + i * kStep < KT ? sr[k0 + i * kStep] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) scale_lds[(k0 + i * kStep) * BM + row] = sv[i];
+  }
+  GroupedScales scales;
+  scales.sa = (GroupedScales::lds_ptr)scale_lds;
+  scales.row0 = wm * T::kWaveM + (lane & 15);
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const uint8_t *region;
+    int col;
+    slot(wn * T::kFN + p * (T::kFN / 2), region, col);
+    scales.sw[p] = uniform_ptr(expert_scales(region, e) + static_cast<uint64_t>(col >> 7) * KT);
+  }
+  __syncthreads();
+  w8a8v6::mainloop_live<T, GroupedScales>(plan, KT, smem, acc, scales, live_fm);
+  w8a8v4::epilogue_barrier();
+
+  // Element q of fragment (i, j): row 16 i + lane % 16, column 16 j + 4 (lane
+  // / 16) + q of the wave tile.
+  const int r = lane & 15, c4 = 4 * (lane >> 4);
+  constexpr int kOut = STAGE == 0 ? T::kFN / 2 : T::kFN;       // output fragments per row
+  constexpr int kCols = STAGE == 0 ? T::kWaveN / 2 : T::kWaveN;
+  auto out4 = [&](int i, int j, uint32_t (&b)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float v = acc[i][j][q];
+      b[q] = f32_to_bf16(STAGE == 0 ? silu_mul(v, acc[i][j + T::kFN - kOut][q]) : v);
+    }
+  };
+  if constexpr (QUANT) {
+    constexpr int kPitch = T::kBN / 2 + 8;  // staged bf16 per row: 128 + pad
+    static_assert(BM * kPitch * 2 <= T::kSmem, "the h tile fits the stage ring");
+    uint16_t *tile = reinterpret_cast<uint16_t *>(smem);
+#pragma unroll
+    for (int i = 0; i < T::kFM; ++i)
+#pragma unroll
+      for (int j = 0; j < kOut; ++j) {
+        uint32_t b[4];
+        out4(i, j, b);
+        *reinterpret_cast<uint2 *>(tile + (wm * T::kWaveM + 16 * i + r) * kPitch + wn * kCols + 16 * j + c4) =
+            uint2{b[0] | (b[1] << 16), b[2] | (b[3] << 16)};
+      }
+    __syncthreads();
+    uint8_t *hq = at<uint8_t>(ws, L.hq);
+    float *hs = at<float>(ws, L.hs);
+    const int groups = N >> 7, hcol0 = bx * (T::kBN / 2);
+    const int ch = lane & 15;
+    constexpr int kRowsPerWave = BM / T::kWaves;
+#pragma unroll
+    for (int it = 0; it < kRowsPerWave / 4; ++it) {
+      const int row = wave * kRowsPerWave + 4 * it + (lane >> 4);
+      const uint4 v = *reinterpret_cast<const uint4 *>(tile + row * kPitch + ch * 8);
+      float amax = bf16x8_amax(v, 0.0f);
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+      const bool zero = amax == 0.0f;
+      const float ratio = zero ? 0.0f : 448.0f / amax;
+      const int p = p0 + row;
+      if (p < pend) {
+        *reinterpret_cast<uint2 *>(hq + static_cast<uint64_t>(p) * N + hcol0 + ch * 8) = bf16x8_encode(v, ratio, zero);
+        if (ch == 0) hs[static_cast<uint64_t>(p) * groups + bx] = zero ? 0.0f : amax / 448.0f;
+      }
+    }
+  } else {
+    using Stage = w8a8v4::StageTile<uint16_t, T::kWaveM, kCols>;
+    static_assert(Stage::kBytes * T::kWaves <= T::kSmem, "staging fits the stage ring");
+    const Stage st{reinterpret_cast<uint16_t *>(smem + wave * Stage::kBytes)};
+#pragma unroll
+    for (int i = 0; i < T::kFM; ++i)
+#pragma unroll
+      for (int j = 0; j < kOut; ++j) {
+        uint32_t b[4];
+        out4(i, j, b);
+        st.put4(16 * i + r, 16 * j + c4, b);
+      }
+    uint16_t *out = at<uint16_t>(ws, STAGE == 0 ? L.h : L.y);
+    const int pw = p0 + wm * T::kWaveM;
+    const int col0 = bx * (STAGE == 0 ? T::kBN / 2 : T::kBN) + wn * kCols;
+    st.flush(lane, [&](int row) -> uint16_t * {
+      return pw + row < pend ? out + static_cast<uint64_t>(pw + row) * N + col0 : nullptr;
+    });
+  }
+}
+
 // Per-channel profiles on the 256-row tiles (e.g. Mixtral): the hidden
 // quantizer as the first counted step of the down launch
 // (lf_moe_down_t256_aq), so the plan has no lf_moe_quant_hidden launch. Per-
@@ -1745,6 +1936,29 @@ __global__ __launch_bounds__(512) void lf_moe_down_t256_b128(const int32_t *coun
   grouped_gemm_t256<1, true>(counts, d, wd, wd, ws);
 }
 
+// Block-scaled profiles on 128 x 256 tiles (lunaflux_fp8_moe_step_geometry);
+// _q: the hidden quantizer in the gate/up epilogue. The form without it
+// stores bf16 h for inspection.
+__global__ __launch_bounds__(512) void lf_moe_gate_up_t128x256_b128(const int32_t *counts, const int32_t *desc,
+                                                                    const uint8_t *wg, const uint8_t *wu,
+                                                                    uint8_t *ws) {
+  const MoeDesc d = desc_of(desc);
+  if (!desc_ok(d) || d.group != 128 || header_of(wg).magic != kWeightMagic) return;
+  grouped_gemm_t128x256<0, false>(counts, d, wg, wu, ws);
+}
+__global__ __launch_bounds__(512) void lf_moe_gate_up_t128x256_b128_q(const int32_t *counts, const int32_t *desc,
+                                                                      const uint8_t *wg, const uint8_t *wu,
+                                                                      uint8_t *ws) {
+  const MoeDesc d = desc_of(desc);
+  if (!desc_ok(d) || d.group != 128 || header_of(wg).magic != kWeightMagic) return;
+  grouped_gemm_t128x256<0, true>(counts, d, wg, wu, ws);
+}
+__global__ __launch_bounds__(512) void lf_moe_down_t128x256_b128(const int32_t *counts, const int32_t *desc,
+                                                                 const uint8_t *wd, uint8_t *ws) {
+  const MoeDesc d = desc_of(desc);
+  if (!desc_ok(d) || d.group != 128 || header_of(wd).magic != kWeightMagic) return;
+  grouped_gemm_t128x256<1, false>(counts, d, wd, wd, ws);
+}
 // Small profiles (at most 32 tokens): the grouped GEMV form, either scale
 // mode (the descriptor's group).
 __global__ __launch_bounds__(256) void lf_moe_gate_up_gemv(const int32_t *counts,

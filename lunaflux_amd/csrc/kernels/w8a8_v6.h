@@ -65,18 +65,24 @@ struct Plan {
 };
 
 // SCALES (the block's scales):
+//   kFold: false where the scales do not change with k (per-channel weights,
+//     per-token activations): the MFMAs then accumulate into acc, and the
+//     rest of SCALES is not used
 //   kIns: side loads per wave and stage; issue(kt): issues stage kt's
 //   row(kt, i): the scale of this lane's row of fragment row i (an LDS read)
 //   block(kt, p): the weight scale of part p (wave-uniform); p = 1: the up
 //     fragments of a gate/up block (kParts == 2: j >= kFN / 2)
 // The scales of k-tile kt are read until its last fragment row, when stage
 // kt + NS may already be landing.
-template <class T, class SCALES>
+// LIVE: the wave's fragment rows that hold a live row (the others' sums stay
+// zero and are never stored); its loads and barriers are those of every wave.
+template <class T, class SCALES, int LIVE = T::kFM>
 LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)[T::kFM][T::kFN],
                         const SCALES &scales) {
   constexpr int NS = T::kStages, FM = T::kFM, FN = T::kFN, R = T::kRing, P = SCALES::kParts;
   constexpr int kBarrierRow = FM - R;
   constexpr int kIns = T::kAIns + T::kBIns + SCALES::kIns;
+  constexpr bool FOLD = SCALES::kFold;
   static_assert((NS - 1) * kIns < 64, "vmcnt range");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
@@ -134,17 +140,19 @@ LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)
   float f[P];          // their factors
   float sa, sw[P];     // the next row's scale, this k-tile's block scales
 #pragma unroll
-  for (int i = 0; i < R; ++i) read_a(0, i, a[i]);
+  for (int i = 0; i < (R < LIVE ? R : LIVE); ++i) read_a(0, i, a[i]);
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
-    read_b(0, j, b[j]);
+    if (LIVE > 0) read_b(0, j, b[j]);
     part[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  sa = scales.row(0, 0);
+  if constexpr (FOLD) {
+    sa = scales.row(0, 0);
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    sw[p] = scales.block(0, p);
-    f[p] = 0.0f;
+    for (int p = 0; p < P; ++p) {
+      sw[p] = scales.block(0, p);
+      f[p] = 0.0f;
+    }
   }
   auto fold = [&](int i, int j) {
 #pragma unroll
@@ -160,21 +168,30 @@ LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)
     float nsw[P];
     static_for<FM>([&](auto ii) {
       constexpr int i = decltype(ii)::value;
-      const float sa_row = sa;
-      if constexpr (i + 1 < FM) {
-        sa = scales.row(kt, i + 1);
-      } else if constexpr (NEXT) {
-        sa = scales.row(kt + 1, 0);
+      [[maybe_unused]] const float sa_row = sa;
+      if constexpr (FOLD && i < LIVE) {
+        if constexpr (i + 1 < LIVE) {
+          sa = scales.row(kt, i + 1);
+        } else if constexpr (NEXT) {
+          sa = scales.row(kt + 1, 0);
+        }
       }
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
-        fold((i + FM - 1) % FM, j);
-        part[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b[j].v, a[i % R].v, f32x4{0.f, 0.f, 0.f, 0.f}, 0,
-                                                                   0, 0, 127, 0, 127);
-        if constexpr (NEXT && i == FM - 1) read_b(kt + 1, j, b[j]);
+        if constexpr (FOLD && i < LIVE) {
+          fold((i + LIVE - 1) % LIVE, j);
+          part[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b[j].v, a[i % R].v, f32x4{0.f, 0.f, 0.f, 0.f}, 0,
+                                                                     0, 0, 127, 0, 127);
+        } else if constexpr (i < LIVE) {
+          acc[i][j] =
+              __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b[j].v, a[i % R].v, acc[i][j], 0, 0, 0, 127, 0, 127);
+        }
+        if constexpr (LIVE > 0 && NEXT && i == FM - 1) read_b(kt + 1, j, b[j]);
       }
+      if constexpr (FOLD && i < LIVE) {
 #pragma unroll
-      for (int p = 0; p < P; ++p) f[p] = sa_row * sw[p];
+        for (int p = 0; p < P; ++p) f[p] = sa_row * sw[p];
+      }
       if constexpr (NEXT && i == kBarrierRow) {
         __builtin_amdgcn_sched_barrier(0);
         // stage kt + 1 visible (at most the NS - 2 stages after it are
@@ -189,18 +206,20 @@ LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (FOLD) {
 #pragma unroll
-        for (int p = 0; p < P; ++p) nsw[p] = scales.block(kt + 1, p);
+          for (int p = 0; p < P; ++p) nsw[p] = scales.block(kt + 1, p);
+        }
       }
       if constexpr (MORE && i > kBarrierRow) issue(kt + NS, i - kBarrierRow - 1, R - 1);
       if constexpr (i < kBarrierRow) {
-        read_a(kt, i + R, a[i % R]);
-      } else if constexpr (NEXT) {
+        if constexpr (i + R < LIVE) read_a(kt, i + R, a[i % R]);
+      } else if constexpr (NEXT && i - kBarrierRow < LIVE) {
         read_a(kt + 1, i - kBarrierRow, a[i % R]);
       }
       __builtin_amdgcn_sched_barrier(0);
     });
-    if constexpr (NEXT) {
+    if constexpr (FOLD && NEXT) {
 #pragma unroll
       for (int p = 0; p < P; ++p) sw[p] = nsw[p];
     }
@@ -209,9 +228,36 @@ LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)
   for (; kt + NS < KT; ++kt) step(kt, std::true_type{}, std::true_type{});
   for (; kt + 1 < KT; ++kt) step(kt, std::false_type{}, std::true_type{});
   step(kt, std::false_type{}, std::false_type{});
+  if constexpr (FOLD && LIVE > 0) {
 #pragma unroll
-  for (int j = 0; j < FN; ++j) fold(FM - 1, j);
+    for (int j = 0; j < FN; ++j) fold(LIVE - 1, j);
+  }
 }
+
+// The main loop of a wave with live_fm live fragment rows (wave-uniform).
+template <class T, class SCALES>
+LF_DEVICE void mainloop_live(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)[T::kFM][T::kFN],
+                             const SCALES &scales, int live_fm) {
+  const int live = __builtin_amdgcn_readfirstlane(live_fm);
+  if (live <= 0) {
+    mainloop<T, SCALES, 0>(plan, KT, smem, acc, scales);
+  } else if (live == 1) {
+    mainloop<T, SCALES, 1>(plan, KT, smem, acc, scales);
+  } else if (live == 2) {
+    mainloop<T, SCALES, 2>(plan, KT, smem, acc, scales);
+  } else {
+    mainloop<T, SCALES>(plan, KT, smem, acc, scales);
+  }
+}
+
+// Scales that do not change with k.
+struct NoScales {
+  static constexpr bool kFold = false;
+  static constexpr int kIns = 0, kParts = 1;
+  LF_DEVICE void issue(int) const {}
+  LF_DEVICE float row(int, int) const { return 1.0f; }
+  LF_DEVICE float block(int, int) const { return 1.0f; }
+};
 
 // Row scales of a dense tile, k-tile-major in memory ([K / 128][cap], the
 // tile's at base): each stage side-loads its k-tile's BM scales into a slot
@@ -220,6 +266,7 @@ LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)
 // wave has the same loads to count). The block scales are scalar loads.
 template <class T, int PARTS>
 struct DenseScales {
+  static constexpr bool kFold = true;
   static constexpr int kIns = 1, kParts = PARTS;
   const uint8_t *base;     // scales_t + m0 (wave-uniform)
   uint64_t stride;         // bytes per k-tile

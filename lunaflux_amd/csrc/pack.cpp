@@ -1089,9 +1089,24 @@ int64_t lunaflux_fp8_moe_sync_offset(const lf_fp8_moe_desc *d, int32_t max_token
   return offsets[12];
 }
 
-int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d,
-                                         int32_t max_tokens, int32_t dims[7],
-                                         char symbol[LF_FP8_SYMBOL_BYTES]) {
+// Block-scaled profiles above the GEMV form's 32 tokens: 128 x 256 tiles
+// (kernels/moe.hip, grouped_gemm_t128x256), where both K fit its scale table
+// and its 32-bit activation offsets. Against the forms moe_geometry gives
+// below, gate/up + down (+ hidden quantizer) of 64 experts of 2048 x 1408,
+// top 6, us: 60 tokens 153 -> 82, 250 tokens 211 -> 114, 900 tokens 323 ->
+// 154, 1500 tokens 432 -> 192 (all 128 x 128 tiles before), 4096 tokens 369
+// -> 355 (256 x 256). Per-channel profiles stay on their forms: 8 experts of
+// 4096 x 14336, top 2, gate/up + down 60 tokens 271 -> 264, 250 tokens 297 ->
+// 289, but 1024 tokens 497 -> 513 us.
+static bool moe_t128x256(const lf_fp8_moe_desc *d, int64_t T) {
+  constexpr int64_t kMaxK = 128 * 24;  // kT128x256MaxKT
+  return d->group == 128 && !moe_gemv(d, T) && d->hidden % 256 == 0 && d->hidden <= kMaxK && d->inter <= kMaxK &&
+         T * d->top_k * std::max<int64_t>(d->hidden, d->inter) < (int64_t(1) << 32);
+}
+
+// step: the forms lunaflux_fp8_moe_step_geometry gives.
+static int32_t moe_geometry(int32_t entry, const lf_fp8_moe_desc *d, int32_t max_tokens, bool step,
+                            int32_t dims[7], char symbol[LF_FP8_SYMBOL_BYTES]) {
   if (!moe_desc_ok(d) || max_tokens <= 0 || dims == nullptr || symbol == nullptr) {
     return LF_INVALID_ARGUMENT;
   }
@@ -1116,6 +1131,13 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d
   // per-channel 256-row tiles: the hidden quantizer is the down launch's
   // first step (kQuantBlocks blocks ahead of its tiles)
   const bool down_aq = moe_down_aq(d, T);
+  const bool t128x256 = step && moe_t128x256(d, T);
+  // The one-block router also sorts and quantizes, in about 0.3-0.5 us a
+  // token (16 us at 32 tokens); the four launches it stands for take 20 us
+  // at any of these sizes (whole operation, 64 experts, 60 tokens 187 -> 177
+  // us on the four; 8 experts of 4096, 60 / 250 tokens 321 -> 300, 443 ->
+  // 328 us).
+  const bool one_block = A <= 1024 && (!step || T <= 32);
   const int64_t kGemvBlocks = 1024;
   int64_t gx = 1, gy = 1;
   int32_t bx = 256;
@@ -1128,7 +1150,7 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d
     // two sort steps and the token quantizer then launch nothing (empty
     // symbol, zero dims).
     case LF_FP8_MOE_ROUTE:
-      if (A <= 1024) {
+      if (one_block) {
         name = "lf_moe_route_sort";
         bx = 1024;
         break;
@@ -1139,7 +1161,7 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d
     // The sort: one 1024-thread block per chunk of 1024 assignments.
     case LF_FP8_MOE_SORT_COUNT:
     case LF_FP8_MOE_SORT:
-      if (A <= 1024) {
+      if (one_block) {
         std::memset(dims, 0, 7 * sizeof(int32_t));
         std::memset(symbol, 0, LF_FP8_SYMBOL_BYTES);
         return LF_OK;
@@ -1149,7 +1171,7 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d
       bx = 1024;
       break;
     case LF_FP8_MOE_QUANT_TOKENS:
-      if (A <= 1024) {  // quantized by lf_moe_route_sort
+      if (one_block) {  // quantized by lf_moe_route_sort
         std::memset(dims, 0, 7 * sizeof(int32_t));
         std::memset(symbol, 0, LF_FP8_SYMBOL_BYTES);
         return LF_OK;
@@ -1166,6 +1188,12 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d
       // 1-D grid over (64 h-column block, 128-row tile); blocks past the
       // live tile count return.
       // (block scales: the epilogue also quantizes h, see QUANT_HIDDEN)
+      if (t128x256) {
+        name = "lf_moe_gate_up_t128x256_b128_q";
+        gx = d->inter / 128 * tiles;
+        bx = 512;
+        break;
+      }
       if (t256) {
         name = b128 ? "lf_moe_gate_up_t256_b128_q" : "lf_moe_gate_up_t256";
         gx = d->inter / 128 * tiles256;
@@ -1176,7 +1204,7 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d
       gx = d->inter / 64 * tiles;
       break;
     case LF_FP8_MOE_QUANT_HIDDEN:
-      if ((t256 && b128 && !gemv) || down_aq) {
+      if (t128x256 || (t256 && b128 && !gemv) || down_aq) {
         // fused into the gate/up epilogue (block scales) or run as the down
         // launch's first step (per-token): no launch (empty symbol, zero dims)
         std::memset(dims, 0, 7 * sizeof(int32_t));
@@ -1190,6 +1218,12 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d
       if (gemv) {
         name = "lf_moe_down_gemv";
         gx = std::min<int64_t>(std::min<int64_t>(d->experts, A) * (d->hidden / 64), kGemvBlocks);
+        break;
+      }
+      if (t128x256) {
+        name = "lf_moe_down_t128x256_b128";
+        gx = d->hidden / 256 * tiles;
+        bx = 512;
         break;
       }
       if (t256) {
@@ -1215,6 +1249,18 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d
   std::memset(symbol, 0, LF_FP8_SYMBOL_BYTES);
   std::strncpy(symbol, name, LF_FP8_SYMBOL_BYTES - 1);
   return LF_OK;
+}
+
+int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry, const lf_fp8_moe_desc *d,
+                                         int32_t max_tokens, int32_t dims[7],
+                                         char symbol[LF_FP8_SYMBOL_BYTES]) {
+  return moe_geometry(entry, d, max_tokens, false, dims, symbol);
+}
+
+int32_t lunaflux_fp8_moe_step_geometry(int32_t entry, const lf_fp8_moe_desc *d,
+                                       int32_t max_tokens, int32_t dims[7],
+                                       char symbol[LF_FP8_SYMBOL_BYTES]) {
+  return moe_geometry(entry, d, max_tokens, true, dims, symbol);
 }
 
 }  // extern "C"

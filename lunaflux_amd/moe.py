@@ -70,10 +70,18 @@ def workspace_layout(desc: MoeDescriptor, tokens: int) -> dict:
 
 
 def launch_geometry(entry: int, desc: MoeDescriptor, max_tokens: int):
+    return _geometry("lunaflux_fp8_moe_launch_geometry", entry, desc, max_tokens)
+
+
+def step_geometry(entry: int, desc: MoeDescriptor, max_tokens: int):
+    """The forms bind_moe takes (lunaflux_fp8_moe_step_geometry)."""
+    return _geometry("lunaflux_fp8_moe_step_geometry", entry, desc, max_tokens)
+
+
+def _geometry(function: str, entry: int, desc: MoeDescriptor, max_tokens: int):
     dims = (ctypes.c_int32 * 7)()
     symbol = ctypes.create_string_buffer(128)
-    _check("moe_launch_geometry", _abi.lib().lunaflux_fp8_moe_launch_geometry(
-        entry, ctypes.byref(desc), max_tokens, dims, symbol))
+    _check(function, getattr(_abi.lib(), function)(entry, ctypes.byref(desc), max_tokens, dims, symbol))
     return (KernelLaunchDimensions.new(tuple(dims[0:3]), tuple(dims[3:6]), dims[6]),
             symbol.value.decode("ascii"))
 
@@ -93,7 +101,7 @@ def bind_moe(rt: ProjectionRuntime, counts, desc: MoeDescriptor, desc_region: Ke
     the workspace's counter area as a fifth operand and its error word read
     after a synchronous launch) runs it, and the two sort steps and the
     token quantizer when the route step's kernel (lf_moe_route_sort,
-    profiles of at most 1024 assignments) does their work."""
+    profiles of at most 32 tokens and 1024 assignments) does their work."""
     e, h, i = desc.experts, desc.hidden, desc.inter
     mode = _abi.LF_FP8_SCALE_BLOCK128 if desc.group == 128 else _abi.LF_FP8_SCALE_PER_CHANNEL
     for w, rows, cols in ((wg, i, h), (wu, i, h), (wd, h, i)):
@@ -111,7 +119,7 @@ def bind_moe(rt: ProjectionRuntime, counts, desc: MoeDescriptor, desc_region: Ke
     c = _region(counts, COUNTS_BYTES, alignment=4)
 
     def step(entry, operands):
-        dims, symbol = launch_geometry(entry, desc, max_tokens)
+        dims, symbol = step_geometry(entry, desc, max_tokens)
         if not symbol:
             return None
         return LaunchStep(rt.function(symbol), dims, KernelArguments(operands), symbol)

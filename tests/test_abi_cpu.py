@@ -577,6 +577,41 @@ def test_golden_config1_reproduces_from_seed():
     np.testing.assert_array_equal(y, g["y32"])
 
 
+@pytest.mark.parametrize("group", [0, 128])
+@pytest.mark.parametrize("hidden,inter", [(256, 128), (2048, 1408), (384, 256), (3072, 3072), (3328, 1024), (4096, 4096)])
+def test_moe_step_geometry_forms(group, hidden, inter):
+    """The forms a binding takes against the recorded-plan ones: the four
+    routing launches above 32 tokens, 128 x 256 tiles (and no hidden quantizer)
+    for block scales where both K are at most 24 k-tiles and the hidden width
+    is a multiple of 256; every other step the same, and what one refuses the
+    other does too."""
+    from lunaflux_amd import moe
+    desc = moe.moe_descriptor(16, 4, 1, hidden, inter, group)
+    for t in (1, 32, 33, 100, 256, 257, 1024, 5000, 1 << 20):
+        wide = group == 128 and t > 32 and hidden % 256 == 0 and max(hidden, inter) <= 3072 and (
+            t * 4 * max(hidden, inter) < 1 << 32)
+        tiles = t * 4 // 128 + 16
+        for entry in range(1, 9):
+            old, new = moe.launch_geometry(entry, desc, t), moe.step_geometry(entry, desc, t)
+            if wide and entry == _abi.MOE_GATE_UP:
+                assert new[1] == "lf_moe_gate_up_t128x256_b128_q"
+                assert new[0].grid == (inter // 128 * tiles, 1, 1) and new[0].block == (512, 1, 1)
+            elif wide and entry == _abi.MOE_DOWN:
+                assert new[1] == "lf_moe_down_t128x256_b128"
+                assert new[0].grid == (hidden // 256 * tiles, 1, 1) and new[0].block == (512, 1, 1)
+            elif wide and entry == _abi.MOE_QUANT_HIDDEN:
+                assert new[1] == ""
+            elif 32 < t <= 256 and entry in (_abi.MOE_ROUTE, _abi.MOE_SORT_COUNT, _abi.MOE_SORT, _abi.MOE_QUANT_TOKENS):
+                name = {_abi.MOE_ROUTE: "route", _abi.MOE_SORT_COUNT: "sort_count", _abi.MOE_SORT: "sort",
+                        _abi.MOE_QUANT_TOKENS: "quant_tokens"}[entry]
+                assert new[1] == "lf_moe_" + name and old[1] in ("", "lf_moe_route_sort")
+            else:
+                assert old == new, (entry, t)
+    for entry, tokens in ((0, 16), (9, 16), (4, 0), (4, -1)):
+        with pytest.raises(fp8.DeviceError):
+            moe.step_geometry(entry, desc, tokens)
+
+
 def test_moe_descriptor_layout_and_geometry():
     from lunaflux_amd import moe
     d = moe.moe_descriptor(8, 2, 0, 4096, 14336, 0)
