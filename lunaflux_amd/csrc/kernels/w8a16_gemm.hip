@@ -289,8 +289,17 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
   struct Frags {
     uint4 bq[T::kFN][2];
     bf16x8 af[4][T::kFM];
+    float sb[BLOCK ? T::kFN : 1];
   };
   auto read_frags = [&](int k, Frags &f) {
+    // The k-step's block scales (scalar loads) are requested with its
+    // fragments, a k-step before their use: requested at the use, their wait
+    // (which cannot tell scalar loads from LDS reads) also waited for the
+    // next step's fragments.
+    if constexpr (BLOCK) {
+#pragma unroll
+      for (int j = 0; j < T::kFN; ++j) f.sb[j] = sload(bs[j], ktile(k));
+    }
     const uint8_t *a = smem + (k % NSA) * T::kAStage;
     const uint8_t *b = smem + NSA * T::kAStage + (k % NSB) * T::kBStage;
 #pragma unroll
@@ -325,14 +334,9 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
       if (k + NSB < nkt) issue_b(k + NSB);
     }
   };
-  auto compute = [&](int k, const Frags &f) {
+  auto compute = [&](const Frags &f) {
     // BLOCK: this k-step's products, scaled into acc after its MFMAs
     f32x4 part[BLOCK ? T::kFM : 1][T::kFN];
-    float sb[BLOCK ? T::kFN : 1];
-    if constexpr (BLOCK) {
-#pragma unroll
-      for (int j = 0; j < T::kFN; ++j) sb[j] = bs[j][ktile(k)];
-    }
 #pragma unroll
     for (int step = 0; step < 4; ++step) {
 #pragma unroll
@@ -354,7 +358,7 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
       for (int j = 0; j < T::kFN; ++j)
 #pragma unroll
         for (int i = 0; i < T::kFM; ++i) {
-          acc[i][j] += part[i][j] * sb[j];
+          acc[i][j] += part[i][j] * f.sb[j];
           // keeps these reads of the MFMA results in the MFMAs' basic block
           // (a read sunk past a branch has been issued without the wait
           // states an MFMA result needs: w8a16.hip, BLOCK)
@@ -387,18 +391,18 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
   for (; k + 2 < nkt; k += 2) {
     advance(k);
     read_frags(k + 1, f1);
-    compute(k, f0);
+    compute(f0);
     advance(k + 1);
     read_frags(k + 2, f0);
-    compute(k + 1, f1);
+    compute(f1);
   }
   if (k + 1 < nkt) {
     advance(k);
     read_frags(k + 1, f1);
-    compute(k, f0);
-    compute(k + 1, f1);
+    compute(f0);
+    compute(f1);
   } else {
-    compute(k, f0);
+    compute(f0);
   }
 
   // Epilogue. Lane element (i, j, e) is row wm * kWaveM + 16 i + 4 g + e of
