@@ -248,6 +248,22 @@ enum lf_fp8_entry {
 #define LF_FP8_AQ_ERROR_OFFSET 0
 int64_t lunaflux_fp8_w8a8_workspace_bytes(int32_t entry, int64_t n, int64_t k, int32_t max_tokens);
 
+/* The split W8A8 form, a GEMM over rows already quantized, for profiles of at
+ * most 2048 rows whose 128 x 256 tiles number at most 256 (N a multiple of
+ * 256, gate/up of 128; 2048 <= K < 2^24):
+ *  lf_fp8_w8a8_{dense,qkv,gate_up}_t128x256_sk (counts, xq, w..., y, ws)
+ * operands as the GEMM-only entries plus ws, the partial tiles of the K
+ * split and their arrival counters (lunaflux_fp8_w8a8_split_workspace_bytes,
+ * zero-filled once when allocated; its counters return to zero at the end of
+ * every launch; launches sharing one ws must not overlap). Grid: column
+ * blocks x slices x row bands. entry: LF_FP8_ENTRY_W8A8_DENSE / _QKV (N the
+ * packed width) / _GATE_UP. LF_UNSUPPORTED (-1 bytes) where the form does not
+ * take the shape or profile: the operation then runs the forms of
+ * lunaflux_fp8_launch_geometry. */
+int32_t lunaflux_fp8_w8a8_split_geometry(int32_t entry, int64_t n, int64_t k, int32_t max_tokens,
+                                         int32_t dims[7], char symbol[LF_FP8_SYMBOL_BYTES]);
+int64_t lunaflux_fp8_w8a8_split_workspace_bytes(int32_t entry, int64_t n, int64_t k, int32_t max_tokens);
+
 /* Admission of one weight operand's region before an operation is bound,
  * the FP8 counterpart of the exact BF16 size check engine/device_plan applies
  * to every weight region (build.mbt:149-203). region_head: the region's

@@ -124,6 +124,8 @@ SIGNATURES = {
     "lunaflux_fp8_w8a16_workspace_bytes": (_i64, [_i32, _i64, _i64, _i32]),
     "lunaflux_fp8_w8a8_workspace_bytes": (_i64, [_i32, _i64, _i64, _i32]),
     "lunaflux_fp8_launch_geometry": (_i32, [_i32, _i64, _i64, _i32, _i32p, ctypes.c_char_p]),
+    "lunaflux_fp8_w8a8_split_geometry": (_i32, [_i32, _i64, _i64, _i32, _i32p, ctypes.c_char_p]),
+    "lunaflux_fp8_w8a8_split_workspace_bytes": (_i64, [_i32, _i64, _i64, _i32]),
     "lunaflux_fp8_gated_mlp_geometry": (_i32, [_i32, _i64, _i64, _i32, _i32p, ctypes.c_char_p]),
     "lunaflux_fp8_gated_mlp_workspace_bytes": (_i64, [_i32, _i64, _i64, _i32]),
     "lunaflux_fp8_qkv_launch_geometry": (_i32, [_i32, _i64, _i64, _i64, _i32, _i32p,

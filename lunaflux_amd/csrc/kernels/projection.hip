@@ -1572,6 +1572,203 @@ LF_DEVICE void w8a8_b128_gated_mlp(const int32_t *counts, const uint16_t *x, con
 }
 
 // ---------------------------------------------------------------------------
+// Per-channel W8A8 GEMM on 128 x 256 tiles with a K split (w8a8_v6.h without
+// the fold: eight 64 x 64 waves, three stages, one block per CU), over rows
+// already quantized: operands (counts, xq, w..., y, ws). For launches whose
+// tiles alone leave CUs idle: grid = slices x tiles (tiles of the profile's
+// bands x column blocks). The fp32 partial tiles of a split meet as in the
+// W8A16 forms: each block stores its tile's fragments through the XCD's L2,
+// counts itself into its tile's counter, and the last to arrive sums the
+// slices in order (deterministic), runs the epilogue and resets the counter.
+// Nothing waits for another block. Workspace: fragments [slice][tile][wave][i][j][64
+// lanes x 4], then one counter per tile; zero-filled once.
+// ---------------------------------------------------------------------------
+using SplitTile = w8a8v6::Tile<128, 256, 2, 4, 3>;
+
+template <int MODE>
+LF_DEVICE void w8a8_split_gemm(const int32_t *counts, const uint8_t *xq, const uint8_t *w0, const uint8_t *w1,
+                               const uint8_t *w2, uint16_t *y, uint8_t *ws) {
+  using T = SplitTile;
+  constexpr int BM = T::kBM, BN = T::kBN;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[T::kSmem];
+  __shared__ __attribute__((aligned(16))) float scale_lds[BM + BN];
+  __shared__ int last_block;
+  if (!dense_regions_ok<MODE>(w0, w1, w2)) return;
+  const WeightHeader &h0 = header_of(w0);
+  const int K = static_cast<int>(h0.columns);
+  const int KT = K >> 7;
+  const int tq = static_cast<int>(h0.rows) >> 4;
+  const int tk = MODE == 1 ? static_cast<int>(header_of(w1).rows) >> 4 : 0;
+  const int ld = dense_ld<MODE>(w0, w1, w2);
+  const int gx = dense_gx<MODE, BN>(ld);
+  // profile bands x slices: the grid's z and y (x: column blocks)
+  const int S = static_cast<int>(gridDim.y), bands = static_cast<int>(gridDim.z);
+  if (gx != static_cast<int>(gridDim.x) || S > KT || K >= (1 << 24)) return;  // not a grid of this entry's geometry
+  const int M = live_rows(counts, bands * BM);
+  const int live_bands = (M + BM - 1) / BM;
+  // Block order: slices, then column blocks, then the bands innermost, dealt
+  // so that each XCD (block index mod 8) takes a contiguous range: the bands
+  // that share a weight strip, then the strips of one K-slice.
+  const int linear =
+      (static_cast<int>(blockIdx.z) * S + static_cast<int>(blockIdx.y)) * gx + static_cast<int>(blockIdx.x);
+  const int work = gx * S * live_bands;
+  if (linear >= work) return;
+  const int xcd = linear & 7, local = linear >> 3, base = work >> 3, extra = work & 7;
+  const int t = xcd * base + (xcd < extra ? xcd : extra) + local;
+  const int by = t % live_bands, bx = t / live_bands % gx, s = t / (live_bands * gx);
+  const int m0 = by * BM;
+  const int kt0 = KT * s / S, kt1 = KT * (s + 1) / S;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int wm = wave / T::kWgn, wn = wave % T::kWgn;
+
+  auto slot = [&](int sl, const uint8_t *&region, int &tile, int &ocol) {
+    if (MODE == 2) {
+      const int sw = sl / T::kFN, f = sl % T::kFN;
+      const bool up = f >= T::kFN / 2;
+      ocol = bx * (BN / 2) + sw * (T::kWaveN / 2) + 16 * (up ? f - T::kFN / 2 : f);
+      region = up ? w1 : w0;
+      tile = ocol >> 4;
+    } else {
+      tile = bx * (BN / 16) + sl;
+      ocol = tile * 16;
+      region = w0;
+      if (MODE == 1) {
+        if (tile >= tq + tk) {
+          region = w2;
+          tile -= tq + tk;
+        } else if (tile >= tq) {
+          region = w1;
+          tile -= tq;
+        }
+      }
+    }
+  };
+  w8a8v6::Plan<T> plan;
+  plan.a_base = w8a8v3::uniform_ptr(xq + static_cast<uint64_t>(m0) * K + static_cast<uint64_t>(kt0) * 128);
+#pragma unroll
+  for (int q = 0; q < T::kAIns; ++q) {
+    const int tr = w8a8v3::a_load_row<T>(wave, q, lane);
+    const int row = m0 + tr < M ? tr : M - 1 - m0;
+    plan.a_off[q] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) + w8a8v3::a_load_chunk(tr, lane) * 16;
+  }
+#pragma unroll
+  for (int q = 0; q < T::kBIns; ++q) {
+    const int half = w8a8v3::b_load_half<T>(wave, q);
+    const uint8_t *region;
+    int tile, ocol;
+    slot(half >> 1, region, tile, ocol);
+    plan.b_base[q] = w8a8v3::uniform_ptr(expert_tiles(region, 0) +
+                                         (static_cast<uint64_t>(tile) * KT + kt0) * kTileBytes + (half & 1) * 1024);
+  }
+  plan.b_lane = lane * 16;
+  // Row scales, then the block's 256 column scales: loaded before the main
+  // loop, parked in LDS after it.
+  const int tid = static_cast<int>(threadIdx.x);
+  float sa_mine = 0.0f, sw_mine = 0.0f;
+  if (tid < BM) {
+    const float *ascale = reinterpret_cast<const float *>(xq + align256(static_cast<uint64_t>(M) * K));
+    sa_mine = ascale[m0 + tid < M ? m0 + tid : M - 1];
+  }
+  if (tid < BN) {
+    const uint8_t *region;
+    int tile, ocol;
+    slot(tid >> 4, region, tile, ocol);
+    sw_mine = expert_scales(region, 0)[tile * 16 + (tid & 15)];
+  }
+  const int live_rows_wave = M - (m0 + wm * T::kWaveM);
+  const int live_fm = live_rows_wave <= 0 ? 0 : live_rows_wave >= T::kWaveM ? T::kFM : (live_rows_wave + 15) / 16;
+  f32x4 acc[T::kFM][T::kFN];
+  w8a8v6::mainloop_live<T, w8a8v6::NoScales>(plan, kt1 - kt0, smem, acc, w8a8v6::NoScales{}, live_fm);
+  if (tid < BM) scale_lds[tid] = sa_mine;
+  if (tid < BN) scale_lds[BM + tid] = sw_mine;
+
+  if (S > 1) {
+    const int tiles = gx * live_bands, tile = bx * live_bands + by;
+    auto frag_at = [&](int slice, int i, int j) {
+      return ws + (((static_cast<uint64_t>(slice) * tiles + tile) * T::kWaves + wave) * T::kFM * T::kFN +
+                   i * T::kFN + j) * 1024 + lane * 16;
+    };
+#pragma unroll
+    for (int i = 0; i < T::kFM; ++i) {
+      if (i >= live_fm) continue;
+#pragma unroll
+      for (int j = 0; j < T::kFN; ++j) phase::store16_through(frag_at(s, i, j), __builtin_bit_cast(u32x4, acc[i][j]));
+    }
+    // (the counters follow the partials of the profile's tiles)
+    int *arrivals = reinterpret_cast<int *>(ws + static_cast<uint64_t>(S) * gx * bands * T::kWaves * T::kFM *
+                                                     T::kFN * 1024) + tile;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      const int before = __hip_atomic_fetch_add(arrivals, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last_block = before == S - 1 ? 1 : 0;
+      if (before == S - 1) phase::store_agent(arrivals, 0);
+    }
+    __syncthreads();
+    if (last_block == 0) return;
+    // the S partials in slice order, this block's own from its registers
+    for (int slice = 0; slice < S; ++slice) {
+      if (slice == s) continue;
+      uint64_t v[T::kFM][T::kFN][2];
+#pragma unroll
+      for (int i = 0; i < T::kFM; ++i)
+#pragma unroll
+        for (int j = 0; j < T::kFN; ++j)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            v[i][j][h] = i < live_fm ? __hip_atomic_load(reinterpret_cast<uint64_t *>(frag_at(slice, i, j)) + h,
+                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                     : 0;
+          }
+#pragma unroll
+      for (int i = 0; i < T::kFM; ++i)
+#pragma unroll
+        for (int j = 0; j < T::kFN; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            acc[i][j][e] += __uint_as_float(static_cast<uint32_t>(v[i][j][e >> 1] >> (32 * (e & 1))));
+          }
+    }
+  }
+  w8a8v4::epilogue_barrier();
+  // Element q of fragment (i, j): row 16 i + lane % 16, column 16 j + 4 (lane
+  // / 16) + q of the wave tile. Column scale of block slot column c at BM + c.
+  const int r = lane & 15, c4 = 4 * (lane >> 4);
+  constexpr int kOut = MODE == 2 ? T::kFN / 2 : T::kFN;
+  constexpr int kCols = 16 * kOut;
+  using Stage = w8a8v4::StageTile<uint16_t, T::kWaveM, kCols>;
+  static_assert(Stage::kBytes * T::kWaves <= T::kSmem, "staging fits the stage ring");
+  const Stage st{reinterpret_cast<uint16_t *>(smem + wave * Stage::kBytes)};
+#pragma unroll
+  for (int i = 0; i < T::kFM; ++i) {
+    const float sa = scale_lds[wm * T::kWaveM + 16 * i + r];
+#pragma unroll
+    for (int j = 0; j < kOut; ++j) {
+      uint32_t b[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int c = BM + wn * T::kWaveN + 16 * j + c4 + q;
+        const float v = acc[i][j][q] * sa * scale_lds[c];
+        if constexpr (MODE == 2) {
+          b[q] = f32_to_bf16(silu_mul(v, acc[i][j + T::kFN - kOut][q] * sa * scale_lds[c + 16 * kOut]));
+        } else {
+          b[q] = f32_to_bf16(v);
+        }
+      }
+      st.put4(16 * i + r, 16 * j + c4, b);
+    }
+  }
+  const uint8_t *region;
+  int tile0, col0;
+  slot(wn * T::kFN, region, tile0, col0);
+  const int mw = m0 + wm * T::kWaveM;
+  st.flush(lane, [&](int row) -> uint16_t * {
+    return mw + row < M ? y + static_cast<uint64_t>(mw + row) * ld + col0 : nullptr;
+  });
+}
+
+// ---------------------------------------------------------------------------
 // W8A8 GatedMlp in one launch (model/plan/plan.mbt:47-59;
 // kernels/reference/mlp.mbt:4-39): x -> xq (per token) -> gate/up + SwiGLU ->
 // h (bf16) -> hq (per token) -> down -> y, the same arithmetic as the
@@ -1706,6 +1903,22 @@ LF_W8A8_ENTRIES(t128, GemmT128)
 LF_W8A8_GATED_MLP(t256_t256, GemmT256S, GemmT256S)
 LF_W8A8_GATED_MLP(t256_t256x128, GemmT256S, GemmT256x128S)
 LF_W8A8_GATED_MLP(t128_t128, GemmT128S, GemmT128S)
+
+// Per-channel, 128 x 256 tiles with a K split: (counts, xq, w..., y, ws).
+__global__ __launch_bounds__(512) void lf_fp8_w8a8_dense_t128x256_sk(const int32_t *counts, const uint8_t *xq,
+                                                                     const uint8_t *w, uint16_t *y, uint8_t *ws) {
+  w8a8_split_gemm<0>(counts, xq, w, w, w, y, ws);
+}
+__global__ __launch_bounds__(512) void lf_fp8_w8a8_qkv_t128x256_sk(const int32_t *counts, const uint8_t *xq,
+                                                                   const uint8_t *wq, const uint8_t *wk,
+                                                                   const uint8_t *wv, uint16_t *y, uint8_t *ws) {
+  w8a8_split_gemm<1>(counts, xq, wq, wk, wv, y, ws);
+}
+__global__ __launch_bounds__(512) void lf_fp8_w8a8_gate_up_t128x256_sk(const int32_t *counts, const uint8_t *xq,
+                                                                       const uint8_t *wg, const uint8_t *wu,
+                                                                       uint16_t *h, uint8_t *ws) {
+  w8a8_split_gemm<2>(counts, xq, wg, wu, wu, h, ws);
+}
 
 // Block-scaled (128 x 128 weight blocks, 128-column activation groups) W8A8
 // operations, one launch each: (counts, x, w..., y, ws).

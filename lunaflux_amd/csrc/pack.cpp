@@ -748,6 +748,68 @@ int64_t lunaflux_fp8_w8a8_workspace_bytes(int32_t entry, int64_t n, int64_t k, i
   return sync_bytes(1, t.bands) + quantized_rows_bytes(t.bands * t.bm, k);
 }
 
+// The split W8A8 form (kernels/projection.hip, w8a8_split_gemm): 128 x 256
+// tiles (gate/up: 128 h-columns) where the profile has at most one per CU,
+// K cut into the most slices that keep 14 k-tiles each and one block per CU,
+// up to four. Measured on the Llama-3-8B shapes, whole and as one of two
+// tensor-parallel ranks, act-quant launch and GEMM against the one-launch
+// forms of w8a8_tiles (us, M = 130 / 256 / 509 / 1000 / 2000):
+//   4096 x 14336: 118.0 / 124.6 / 124.2 / 104.4 / 129.1 -> 41.5 / 47.6 (4
+//     slices) / 50.3 (4) / 73.5 (2) / 124.2 (1); 2, 6 and 8 slices at 256
+//     rows 62.6, 47.6, 49.9
+//   6144 x 4096: 30.2 / 31.8 / 33.8 / 43.3 -> 24.2 (2) / 26.0 (2) / 30.9 (2) /
+//     38.2 (1); past 256 tiles (2000 rows, 384) 60.7 -> 70.2, so not there
+//   4096 x 4096: 29.3 / 30.2 / 32.3 / 40.1 / 46.2 -> 24.0 / 26.8 / 28.5 /
+//     35.1 / 42.4
+//   4096 x 2048: 20.0 / 20.6 / 21.8 / 27.2 / 31.5 -> 18.3 / 18.7 / 20.0 /
+//     23.2 / 28.7 (1 slice; 2 slices 18.5 / 20.7 / 23.4 / 29.1)
+//   gate/up 14336 x 4096, 130 / 256 rows: 44.0 / 50.6 -> 36.9 / 42.6; past
+//     256 tiles (509 rows, 448) 67.2 -> 73.8, so not there
+// Shorter K and profiles above 2048 rows are not measured and keep their
+// forms.
+struct W8a8SplitForm {
+  int64_t gx, split, bands;
+};
+constexpr int64_t kSplitTileBytes = 128 * 256 * 4;
+static bool w8a8_split(int32_t entry, int64_t n, int64_t k, int32_t max_tokens, W8a8SplitForm *out) {
+  if (entry != LF_FP8_ENTRY_W8A8_DENSE && entry != LF_FP8_ENTRY_W8A8_QKV && entry != LF_FP8_ENTRY_W8A8_GATE_UP) {
+    return false;
+  }
+  const int64_t cols = entry == LF_FP8_ENTRY_W8A8_GATE_UP ? 128 : 256, kt = k / 128;
+  if (n <= 0 || n > kMaxDim || n % cols != 0 || k < 2048 || k >= (int64_t(1) << 24) || k % 128 != 0 ||
+      max_tokens <= 0 || max_tokens > 2048) {
+    return false;
+  }
+  out->gx = n / cols;
+  out->bands = (max_tokens + 127) / 128;
+  const int64_t tiles = out->gx * out->bands;
+  if (tiles > 256) return false;
+  out->split = std::max<int64_t>(1, std::min<int64_t>(4, std::min(256 / tiles, kt / 14)));
+  return true;
+}
+
+int32_t lunaflux_fp8_w8a8_split_geometry(int32_t entry, int64_t n, int64_t k, int32_t max_tokens,
+                                         int32_t dims[7], char symbol[LF_FP8_SYMBOL_BYTES]) {
+  if (dims == nullptr || symbol == nullptr) return LF_INVALID_ARGUMENT;
+  W8a8SplitForm f;
+  if (!w8a8_split(entry, n, k, max_tokens, &f)) return LF_UNSUPPORTED;
+  const int32_t values[7] = {static_cast<int32_t>(f.gx), static_cast<int32_t>(f.split),
+                             static_cast<int32_t>(f.bands), 512, 1, 1, 0};
+  std::memcpy(dims, values, sizeof(values));
+  std::memset(symbol, 0, LF_FP8_SYMBOL_BYTES);
+  std::snprintf(symbol, LF_FP8_SYMBOL_BYTES, "lf_fp8_w8a8_%s_t128x256_sk",
+                entry == LF_FP8_ENTRY_W8A8_QKV ? "qkv" : entry == LF_FP8_ENTRY_W8A8_GATE_UP ? "gate_up" : "dense");
+  return LF_OK;
+}
+
+int64_t lunaflux_fp8_w8a8_split_workspace_bytes(int32_t entry, int64_t n, int64_t k, int32_t max_tokens) {
+  W8a8SplitForm f;
+  if (!w8a8_split(entry, n, k, max_tokens, &f)) return -1;
+  if (f.split == 1) return 256;
+  const int64_t tiles = f.gx * f.bands;
+  return f.split * tiles * kSplitTileBytes + align_up(tiles * 4, 256);
+}
+
 int32_t lunaflux_fp8_gated_mlp_geometry(int32_t entry, int64_t hidden, int64_t inter,
                                         int32_t max_tokens, int32_t dims[7],
                                         char symbol[LF_FP8_SYMBOL_BYTES]) {

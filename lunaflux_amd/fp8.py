@@ -159,6 +159,20 @@ def launch_geometry(entry: int, n: int, k: int, max_tokens: int,
             symbol.value.decode("ascii"))
 
 
+def w8a8_split_geometry(entry: int, n: int, k: int, max_tokens: int):
+    """(dims, symbol, workspace bytes) of the split W8A8 form of a GEMM-only
+    entry for the shape and profile, or None where it takes neither."""
+    dims = (ctypes.c_int32 * 7)()
+    symbol = ctypes.create_string_buffer(128)
+    status = _abi.lib().lunaflux_fp8_w8a8_split_geometry(entry, n, k, max_tokens, dims, symbol)
+    if status == _abi.LF_UNSUPPORTED:
+        return None
+    _check("w8a8_split_geometry", status)
+    return (KernelLaunchDimensions.new(tuple(dims[0:3]), tuple(dims[3:6]), dims[6]),
+            symbol.value.decode("ascii"),
+            _abi.lib().lunaflux_fp8_w8a8_split_workspace_bytes(entry, n, k, max_tokens))
+
+
 def gated_mlp_geometry(hidden: int, inter: int, max_tokens: int,
                        entry: int = _abi.ENTRY_W8A16_GATED_MLP):
     """(dims, symbol) of the one-launch GatedMlp entry (W8A16 or W8A8) for the
@@ -339,6 +353,34 @@ class ProjectionRuntime:
         step = self._step(entry, n, k, max_tokens, operands + [_region(ws, alignment=256)], qkv_split)
         return BoundOperation([step], workspace=ws, error_offset=_abi.LF_FP8_AQ_ERROR_OFFSET)
 
+    def _split_step(self, entry: int, n: int, k: int, max_tokens: int, operands):
+        """The split W8A8 GEMM over quantized rows (its workspace zero-filled
+        once here and held by the step), or None where the form does not take
+        the shape and profile."""
+        geometry = w8a8_split_geometry(entry, n, k, max_tokens)
+        if geometry is None:
+            return None
+        dims, symbol, nbytes = geometry
+        ws = self.context.allocate(nbytes)
+        ws.copy_from_host(np.zeros(nbytes, np.uint8))
+        return LaunchStep(self.function(symbol), dims,
+                          KernelArguments(operands + [_region(ws, alignment=256)]), symbol)
+
+    def _w8a8_split(self, entry: int, weights, n: int, counts: Allocation, x: KernelArgument,
+                    y: KernelArgument, max_tokens: int):
+        """A W8A8 operation as the act-quant launch and the split GEMM, or
+        None where the form does not take it."""
+        k = weights[0].columns
+        if w8a8_split_geometry(entry, n, k, max_tokens) is None:
+            return None
+        xq_alloc = self.context.allocate(act_quant_bytes(max_tokens, k))
+        xq = _region(xq_alloc, alignment=256)
+        return BoundOperation([
+            self.bind_act_quant(counts, x, weights[0], xq, max_tokens),
+            self._split_step(entry, n, k, max_tokens, [_region(counts, COUNTS_BYTES, alignment=4), xq,
+                                                       *(w.region for w in weights), y]),
+        ], workspace=xq_alloc)
+
     # -- binding plan operations to launch steps ---------------------------
     def bind_act_quant(self, counts: Allocation, x: KernelArgument, w: Fp8Weight,
                        xq: KernelArgument, max_tokens: int) -> LaunchStep:
@@ -358,8 +400,13 @@ class ProjectionRuntime:
     def bind_dense_quantized(self, counts: Allocation, xq: KernelArgument, w: Fp8Weight,
                              y: KernelArgument, max_tokens: int) -> LaunchStep:
         """The W8A8 dense GEMM alone, over rows already quantized (by
-        bind_rms_norm_quant or bind_act_quant)."""
+        bind_rms_norm_quant or bind_act_quant); the split form where it takes
+        the shape and profile."""
         w.admit(_abi.ENTRY_W8A8_DENSE)
+        split = self._split_step(_abi.ENTRY_W8A8_DENSE, w.rows, w.columns, max_tokens,
+                                 [_region(counts, COUNTS_BYTES, alignment=4), xq, w.region, y])
+        if split is not None:
+            return split
         return self._step(_abi.ENTRY_W8A8_DENSE, w.rows, w.columns, max_tokens,
                           [_region(counts, COUNTS_BYTES, alignment=4), xq, w.region, y])
 
@@ -380,8 +427,10 @@ class ProjectionRuntime:
     def bind_dense(self, family: str, counts: Allocation, x: KernelArgument, w: Fp8Weight,
                    y: KernelArgument, max_tokens: int, one_launch: bool = True) -> BoundOperation:
         """OutputProjection / down / the vocabulary head. W8A8: one launch
-        (the _aq entry quantizes x inside it); one_launch=False binds the
-        act-quant launch and the GEMM-only launch instead (same outputs).
+        (the _aq entry quantizes x inside it), or the act-quant launch and
+        the split GEMM where that form takes the shape and profile
+        (w8a8_split_geometry); one_launch=False binds the act-quant launch
+        and the GEMM-only launch instead (the one launch's outputs).
         A weight with 128 x 128 block scales binds the family's _B128 entry
         (one launch in both families, whatever one_launch says)."""
         _family(family, max_tokens)
@@ -394,6 +443,9 @@ class ProjectionRuntime:
             return self._w8a16(_abi.ENTRY_W8A16_DENSE, w.rows, w.columns, max_tokens,
                                [c, x, w.region, y])
         if one_launch:
+            split = self._w8a8_split(_abi.ENTRY_W8A8_DENSE, [w], w.rows, counts, x, y, max_tokens)
+            if split is not None:
+                return split
             w.admit(_abi.ENTRY_W8A8_DENSE_AQ)
             return self._w8a8_one_launch(_abi.ENTRY_W8A8_DENSE_AQ, w.rows, w.columns, max_tokens,
                                          [c, x, w.region, y])
@@ -423,6 +475,9 @@ class ProjectionRuntime:
                                [c, x, wq.region, wk.region, wv.region, y],
                                qkv_split=(wq.rows, wk.rows))
         if one_launch:
+            split = self._w8a8_split(_abi.ENTRY_W8A8_QKV, [wq, wk, wv], n, counts, x, y, max_tokens)
+            if split is not None:
+                return split
             return self._w8a8_one_launch(_abi.ENTRY_W8A8_QKV_AQ, n, wq.columns, max_tokens,
                                          [c, x, wq.region, wk.region, wv.region, y],
                                          qkv_split=(wq.rows, wk.rows))
@@ -450,6 +505,9 @@ class ProjectionRuntime:
             return self._w8a16(_abi.ENTRY_W8A16_GATE_UP, wg.rows, wg.columns, max_tokens,
                                [c, x, wg.region, wu.region, h])
         if one_launch:
+            split = self._w8a8_split(_abi.ENTRY_W8A8_GATE_UP, [wg, wu], wg.rows, counts, x, h, max_tokens)
+            if split is not None:
+                return split
             return self._w8a8_one_launch(_abi.ENTRY_W8A8_GATE_UP_AQ, wg.rows, wg.columns, max_tokens,
                                          [c, x, wg.region, wu.region, h])
         ws = self.context.allocate(act_quant_bytes(max_tokens, wg.columns))
@@ -487,8 +545,16 @@ class ProjectionRuntime:
             entry = None
         else:
             entry = _abi.ENTRY_W8A16_GATED_MLP if family == "w8a16" else _abi.ENTRY_W8A8_GATED_MLP
+        # W8A8 where the down projection takes the split form: the gate/up
+        # and the down operation in turn. In the one launch both GEMMs share
+        # a band height, and down has a tile for a quarter of the CUs at 509
+        # rows (Llama-3-8B layer, us, one launch -> two operations: 200 rows
+        # 264 -> 144, 509 rows 242 -> 181, 900 rows 287 -> 243, 1800 rows 416
+        # -> 403).
+        split_down = (entry == _abi.ENTRY_W8A8_GATED_MLP and one_launch and
+                      w8a8_split_geometry(_abi.ENTRY_W8A8_DENSE, wd.rows, wd.columns, max_tokens) is not None)
         geometry = (gated_mlp_geometry(wg.columns, wg.rows, max_tokens, entry)
-                    if one_launch and entry is not None else None)
+                    if one_launch and entry is not None and not split_down else None)
         if geometry is not None:
             for w in (wg, wu, wd):
                 w.admit(entry)

@@ -258,6 +258,30 @@ def test_w8a16_any_shape_grid_holds_the_kernels_slices(entry, cols, k):
                 assert fp8.w8a16_workspace_bytes(entry, n, k, m) >= need + blocks * 4
 
 
+def test_w8a8_split_geometry():
+    """The split W8A8 form: at most 256 tiles of 128 x 256, K from 2048, at
+    most 2048 rows; slices of at least 14 k-tiles, at most four, at most 256
+    blocks; the workspace holds every slice's tiles and a counter per tile."""
+    for entry, cols in ((_abi.ENTRY_W8A8_DENSE, 256), (_abi.ENTRY_W8A8_QKV, 256), (_abi.ENTRY_W8A8_GATE_UP, 128)):
+        for n in (128, 256, 1000, 1536, 4096, 6144, 14336, 65536):
+            for k in (1920, 2048, 2064, 4096, 14336, 1 << 24):
+                for m in (1, 128, 129, 509, 2048, 2049):
+                    tiles = n // cols * -(-m // 128)
+                    got = fp8.w8a8_split_geometry(entry, n, k, m)
+                    fits = n % cols == 0 and k % 128 == 0 and 2048 <= k < 1 << 24 and m <= 2048 and tiles <= 256
+                    assert (got is not None) == fits, (entry, n, k, m)
+                    if not fits:
+                        assert _abi.lib().lunaflux_fp8_w8a8_split_workspace_bytes(entry, n, k, m) == -1
+                        continue
+                    dims, sym, nbytes = got
+                    gx, s, bands = dims.grid
+                    assert (gx, bands) == (n // cols, -(-m // 128)) and dims.block == (512, 1, 1)
+                    assert s == max(1, min(4, 256 // tiles, k // 128 // 14)) and s * tiles <= 256
+                    assert nbytes >= (s * tiles * 128 * 256 * 4 + tiles * 4 if s > 1 else 1)
+    assert fp8.w8a8_split_geometry(_abi.ENTRY_W8A8_DENSE_AQ, 4096, 4096, 256) is None
+    assert fp8.w8a8_split_geometry(_abi.ENTRY_W8A8_DENSE, 4096, 4096, 0) is None
+
+
 def test_one_launch_w8a8_geometry_and_workspace():
     """The _aq entries: the GEMM-only entry's tile form, 256 quantizer blocks
     ahead of its tiles, workspace = sync area (128 B + one counter per row

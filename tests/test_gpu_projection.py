@@ -586,6 +586,64 @@ def test_w8a16_gemm_form_any_width(rt, op, n, k, m, max_tokens):
     assert all(np.array_equal(outs[0], y) for y in outs[1:]), f"{sym}: launches differ"
 
 
+@pytest.mark.parametrize("op,n,k,max_tokens,ms,slices", [
+    ("dense", 256, 2048, 129, (129, 128, 1, 0), 1),             # one column block, no split
+    ("dense", 512, 3584, 300, (300, 257, 16, 17), 2),           # 28 k-tiles in two slices
+    ("dense", 768, 7296, 512, (512, 449, 63), 4),               # 57 k-tiles: slices of 14 and 15
+    ("qkv", 1280, 7168, 200, (200, 65), 4),                     # 992 + 144 + 144: boundaries inside blocks
+    ("gate_up", 256, 3584, 160, (160, 129, 2), 2),              # two blocks of 128 h-columns
+    ("gate_up", 14336, 2048, 256, (256, 193), 1),               # 224 tiles
+])
+def test_w8a8_split_form(rt, op, n, k, max_tokens, ms, slices):
+    """The split W8A8 form (act-quant launch, then 128 x 256 tiles with K cut
+    into slices) as the bindings take it: ragged live rows on one workspace,
+    two launches bit for bit, rows past M untouched, against the oracle over
+    a column sample (the quantized rows are the act-quant launch's)."""
+    from lunaflux_amd import _abi, fp8
+    from lunaflux_amd.fp8 import _region
+    rng = np.random.default_rng(9300 + n + k)
+    entry = {"dense": _abi.ENTRY_W8A8_DENSE, "qkv": _abi.ENTRY_W8A8_QKV, "gate_up": _abi.ENTRY_W8A8_GATE_UP}[op]
+    dims, sym, nbytes = fp8.w8a8_split_geometry(entry, n, k, max_tokens)
+    assert dims.grid == (n // (128 if op == "gate_up" else 256), slices, -(-max_tokens // 128)), dims.grid
+    sizes = {"dense": [n], "qkv": [n - 288, 144, 144], "gate_up": [n, n]}[op]
+    ws = [make_weight(rt, rng, r, k) for r in sizes]
+    xa = rt.context.allocate(max_tokens * k * 2)
+    ya = rt.context.allocate(max_tokens * n * 2)
+    xr_, yr_ = _region(xa, alignment=256), _region(ya, alignment=256)
+    cols = np.sort(rng.choice(n, min(n, 192), replace=False))
+    counts = rt.step_counts(max_tokens, decode=False)
+    args = [w for _, _, w in ws]
+    bound = {"dense": rt.bind_dense, "qkv": rt.bind_qkv, "gate_up": rt.bind_gate_up}[op](
+        "w8a8", counts, xr_, *args, yr_, max_tokens)
+    assert [s.name for s in bound.steps] == ["lf_fp8_act_quant_rows", sym]
+    for m in ms:
+        counts.copy_from_host(np.array([1, 0, 1, m, 0], np.int32))
+        x = synth.activations(rng, max_tokens, k)
+        xa.copy_from_host(x)
+        outs = []
+        for _ in range(2):
+            ya.copy_from_host(np.full(max_tokens * n, 0x7FC1, np.uint16))
+            bound.launch(rt.stream, synchronous=True)
+            outs.append(ya.read(np.uint16, (max_tokens, n)))
+            assert np.all(outs[-1][m:] == 0x7FC1), f"{sym} m={m}: rows past M written"
+        assert np.array_equal(outs[0], outs[1]), f"{sym} m={m}: launches differ"
+        if m == 0:
+            continue
+        rows = np.unique(np.concatenate([[0, m - 1], rng.integers(0, m, 24)]))
+        xq, xs = o.quantize_rows(o.bf16_decode(x[rows]))
+        xr = o.dequantize(xq, xs)
+        got = outs[0][rows][:, cols]
+        if op == "gate_up":
+            (qg, sg, _), (qu, su, _) = ws
+            wg, wu = deq(qg[cols], sg[cols]), deq(qu[cols], su[cols])
+            g, u = o.dense_projection(xr, wg), o.dense_projection(xr, wu)
+            parity(got, o.silu_mul_array(g, u), label=f"{sym} m={m}",
+                   midpoint_tol=swiglu_midpoint_tol(g, u, abs_sum(xr, wg), abs_sum(xr, wu), k))
+        else:
+            wc = deq(np.concatenate([q for q, _, _ in ws])[cols], np.concatenate([s for _, s, _ in ws])[cols])
+            parity(got, o.dense_projection(xr, wc), k=k, s_abs=abs_sum(xr, wc), label=f"{sym} m={m}")
+
+
 @pytest.mark.parametrize("m,max_tokens,family", [(1, 16, "w8a16"), (13, 16, "w8a16"),
                                                 (32, 32, "w8a16"), (100, 128, "w8a16"),
                                                 (256, 256, "w8a8")])
