@@ -484,9 +484,11 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry,
 /* The same for a caller that binds every step of an operation together
  * (workspace, operands and steps as above): the faster forms where the
  * geometry above, which recorded plans name, has kept an older one. Profiles
- * of more than 32 tokens run the four routing launches, and block-scaled
- * ones with K <= 3072 in both GEMMs and a hidden width that is a multiple of
- * 256
+ * of more than 32 tokens run the four routing launches, block-scaled ones of
+ * at most 32 (and 1024 assignments)
+ *  lf_moe_route_sort_q (counts, desc, logits, x, ws) in place of
+ * lf_moe_route_sort, and block-scaled ones with K <= 3072 in both GEMMs and a
+ * hidden width that is a multiple of 256
  *  lf_moe_gate_up_t128x256_b128_q (counts, desc, wg, wu, ws)
  *  lf_moe_down_t128x256_b128      (counts, desc, wd, ws)
  * (128 x 256 tiles; the gate/up epilogue quantizes h, so there is no hidden

@@ -423,6 +423,9 @@ LF_DEVICE void sort_assignments(const int32_t *counts, const MoeDesc &d, uint8_t
 // kSortThreads assignments in order, each chunk's positions starting where
 // the previous chunk's rows of each expert ended. Outputs equal those of the
 // four launches for any number of tokens.
+// QUANT false: other blocks quantize the tokens, and every wave routes (group
+// 128 only: the per-token form needs the scales after the sort).
+template <bool QUANT>
 LF_DEVICE void route_sort_block(const int32_t *counts, const MoeDesc &d, const float *logits,
                                 const uint16_t *x, uint8_t *ws) {
   __shared__ __attribute__((aligned(16))) int64_t sk[kSortWaves][256];
@@ -439,11 +442,11 @@ LF_DEVICE void route_sort_block(const int32_t *counts, const MoeDesc &d, const f
   // runs the token quantizer (codes and token scales need no routing; the
   // per-token form's expert-order copies of the scales are written after the
   // sort).
-  constexpr int kRouteWaves = kSortWaves / 2;
+  constexpr int kRouteWaves = QUANT ? kSortWaves / 2 : kSortWaves;
   if (wave < kRouteWaves) {
     // A wave's tokens are taken in batches of 4 whose logits are all loaded
     // before the first is ranked (one load latency per batch, not per token).
-    constexpr int kBatch = 4;
+    constexpr int kBatch = QUANT ? 4 : 2;
     for (int t0 = wave; t0 < T; t0 += kBatch * kRouteWaves) {
       TokenLogits lg[kBatch];
 #pragma unroll
@@ -497,7 +500,7 @@ LF_DEVICE void route_sort_block(const int32_t *counts, const MoeDesc &d, const f
   // Per-token form: each token's scale also goes to its assignments'
   // positions in expert order (the positions written above are visible to
   // the block after the last barrier).
-  if (d.group == 0) {
+  if (QUANT && d.group == 0) {
     const float *xs = at<float>(ws, L.xs);
     const int32_t *pos = at<int32_t>(ws, L.pos);
     float *hs = at<float>(ws, L.hs);
@@ -535,6 +538,34 @@ LF_DEVICE void quant_rows(const uint16_t *src, int K, int group, uint8_t *dst, f
 struct TileExpert {
   int e, first_tile, row_begin, row_end;
 };
+// This thread's expert's bounds, for a block that looks its tile up later:
+// loaded with the tile count, before the tile index is known.
+struct ExpertBounds {
+  int lo, hi, o0, o1;
+};
+LF_DEVICE ExpertBounds expert_bounds(const int32_t *tiles, const int32_t *offsets, int E) {
+  const int t = threadIdx.x < E ? static_cast<int>(threadIdx.x) : 0;
+  return {tiles[t], tiles[t + 1], offsets[t], offsets[t + 1]};
+}
+LF_DEVICE TileExpert find_tile_expert(const ExpertBounds &b, int E, int j) {
+  __shared__ int found[4];
+  const int t = threadIdx.x;
+  if (t == 0) {
+    found[0] = 0;
+    found[1] = j;
+    found[2] = 0;
+    found[3] = 0;
+  }
+  __syncthreads();
+  if (t < E && b.lo <= j && j < b.hi) {
+    found[0] = t;
+    found[1] = b.lo;
+    found[2] = b.o0;
+    found[3] = b.o1;
+  }
+  __syncthreads();
+  return {found[0], found[1], found[2], found[3]};
+}
 LF_DEVICE TileExpert find_tile_expert(const int32_t *tiles, const int32_t *offsets, int E, int j) {
   __shared__ int found[4];
   const int t = threadIdx.x;
@@ -1172,6 +1203,7 @@ __device__ __forceinline__ void grouped_gemm_t128x256(const int32_t *counts, con
   const MoeLayout L(d, Tn);
   const int E = d.experts;
   const int32_t *tiles = at<int32_t>(ws, L.tiles);
+  const ExpertBounds bounds = expert_bounds(tiles, at<int32_t>(ws, L.offsets), E);
   const WeightHeader &h0 = header_of(w0);
   const int K = static_cast<int>(h0.columns);
   const int KT = K >> 7;
@@ -1182,7 +1214,7 @@ __device__ __forceinline__ void grouped_gemm_t128x256(const int32_t *counts, con
   const int gx = STAGE == 0 ? N / (T::kBN / 2) : N / T::kBN;
   int bx, by;
   if (!w8a8v3::tile_of_block(gx, tiles[E], tiles[E], bx, by)) return;
-  const TileExpert te = find_tile_expert(tiles, at<int32_t>(ws, L.offsets), E, by);
+  const TileExpert te = find_tile_expert(bounds, E, by);
   const int e = te.e;
   const int p0 = te.row_begin + (by - te.first_tile) * BM;
   const int pend = te.row_end;
@@ -1829,9 +1861,27 @@ __global__ __launch_bounds__(1024) void lf_moe_route_sort(const int32_t *counts,
                                                          uint8_t *ws) {
   const MoeDesc d = desc_of(desc);
   if (!desc_ok(d) || blockDim.x != kSortThreads) return;
-  route_sort_block(counts, d, logits, x, ws);
+  route_sort_block<true>(counts, d, logits, x, ws);
 }
 
+// Block 0 routes and sorts with all its waves, the others quantize the
+// tokens (per 128-column group). One block for both took 15.7 us at 32 tokens
+// of 2048 and 64 experts (route and quantizer halves ~10 us each, then the
+// sort); so 10.5 us.
+__global__ __launch_bounds__(1024) void lf_moe_route_sort_q(const int32_t *counts, const int32_t *desc,
+                                                            const float *logits, const uint16_t *x, uint8_t *ws) {
+  const MoeDesc d = desc_of(desc);
+  if (!desc_ok(d) || d.group == 0) return;
+  if (blockIdx.x == 0) {
+    route_sort_block<false>(counts, d, logits, x, ws);
+    return;
+  }
+  const int T = live_rows(counts, 1 << 30);
+  const MoeLayout L(d, T);
+  quantize_groups_wave(x, d.hidden, T, at<uint8_t>(ws, L.xq), at<float>(ws, L.xs),
+                       (static_cast<int>(blockIdx.x) - 1) * kSortWaves + (static_cast<int>(threadIdx.x) >> 6),
+                       (static_cast<int>(gridDim.x) - 1) * kSortWaves);
+}
 __global__ __launch_bounds__(256) void lf_moe_quant_tokens(const int32_t *counts,
                                                            const int32_t *desc,
                                                            const uint16_t *x, uint8_t *ws) {

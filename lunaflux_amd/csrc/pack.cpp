@@ -1151,18 +1151,19 @@ int64_t lunaflux_fp8_moe_sync_offset(const lf_fp8_moe_desc *d, int32_t max_token
   return offsets[12];
 }
 
-// Block-scaled profiles above the GEMV form's 32 tokens: 128 x 256 tiles
-// (kernels/moe.hip, grouped_gemm_t128x256), where both K fit its scale table
-// and its 32-bit activation offsets. Against the forms moe_geometry gives
+// Block-scaled profiles: 128 x 256 tiles (kernels/moe.hip,
+// grouped_gemm_t128x256), where both K fit its scale table and its 32-bit
+// activation offsets. Against the forms moe_geometry gives
 // below, gate/up + down (+ hidden quantizer) of 64 experts of 2048 x 1408,
-// top 6, us: 60 tokens 153 -> 82, 250 tokens 211 -> 114, 900 tokens 323 ->
+// top 6, us: whole operation on the GEMV form 4 tokens 49.0 -> 47.6, 12 tokens
+// 63.9 -> 58.3, 32 tokens 93.1 -> 91.8 (no hidden quantizer launch); 60 tokens 153 -> 82, 250 tokens 211 -> 114, 900 tokens 323 ->
 // 154, 1500 tokens 432 -> 192 (all 128 x 128 tiles before), 4096 tokens 369
 // -> 355 (256 x 256). Per-channel profiles stay on their forms: 8 experts of
 // 4096 x 14336, top 2, gate/up + down 60 tokens 271 -> 264, 250 tokens 297 ->
 // 289, but 1024 tokens 497 -> 513 us.
 static bool moe_t128x256(const lf_fp8_moe_desc *d, int64_t T) {
   constexpr int64_t kMaxK = 128 * 24;  // kT128x256MaxKT
-  return d->group == 128 && !moe_gemv(d, T) && d->hidden % 256 == 0 && d->hidden <= kMaxK && d->inter <= kMaxK &&
+  return d->group == 128 && d->hidden % 256 == 0 && d->hidden <= kMaxK && d->inter <= kMaxK &&
          T * d->top_k * std::max<int64_t>(d->hidden, d->inter) < (int64_t(1) << 32);
 }
 
@@ -1213,7 +1214,9 @@ static int32_t moe_geometry(int32_t entry, const lf_fp8_moe_desc *d, int32_t max
     // symbol, zero dims).
     case LF_FP8_MOE_ROUTE:
       if (one_block) {
-        name = "lf_moe_route_sort";
+        // step, group 128: blocks beside it quantize the tokens
+        name = step && b128 ? "lf_moe_route_sort_q" : "lf_moe_route_sort";
+        gx = step && b128 ? 9 : 1;
         bx = 1024;
         break;
       }
@@ -1242,7 +1245,7 @@ static int32_t moe_geometry(int32_t entry, const lf_fp8_moe_desc *d, int32_t max
       gx = b128 ? group_quant_blocks(T * (d->hidden / 128)) : (T + 3) / 4;
       break;
     case LF_FP8_MOE_GATE_UP:
-      if (gemv) {
+      if (gemv && !t128x256) {
         name = "lf_moe_gate_up_gemv";
         gx = std::min<int64_t>(std::min<int64_t>(d->experts, A) * (d->inter / 64), kGemvBlocks);
         break;
@@ -1277,7 +1280,7 @@ static int32_t moe_geometry(int32_t entry, const lf_fp8_moe_desc *d, int32_t max
       gx = b128 ? group_quant_blocks(A * (d->inter / 128)) : (A + 3) / 4;
       break;
     case LF_FP8_MOE_DOWN:
-      if (gemv) {
+      if (gemv && !t128x256) {
         name = "lf_moe_down_gemv";
         gx = std::min<int64_t>(std::min<int64_t>(d->experts, A) * (d->hidden / 64), kGemvBlocks);
         break;

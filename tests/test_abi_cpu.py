@@ -605,14 +605,15 @@ def test_golden_config1_reproduces_from_seed():
 @pytest.mark.parametrize("hidden,inter", [(256, 128), (2048, 1408), (384, 256), (3072, 3072), (3328, 1024), (4096, 4096)])
 def test_moe_step_geometry_forms(group, hidden, inter):
     """The forms a binding takes against the recorded-plan ones: the four
-    routing launches above 32 tokens, 128 x 256 tiles (and no hidden quantizer)
+    routing launches above 32 tokens, the token quantizer on blocks of its own
+    up to there with block scales, 128 x 256 tiles (and no hidden quantizer)
     for block scales where both K are at most 24 k-tiles and the hidden width
     is a multiple of 256; every other step the same, and what one refuses the
     other does too."""
     from lunaflux_amd import moe
     desc = moe.moe_descriptor(16, 4, 1, hidden, inter, group)
     for t in (1, 32, 33, 100, 256, 257, 1024, 5000, 1 << 20):
-        wide = group == 128 and t > 32 and hidden % 256 == 0 and max(hidden, inter) <= 3072 and (
+        wide = group == 128 and hidden % 256 == 0 and max(hidden, inter) <= 3072 and (
             t * 4 * max(hidden, inter) < 1 << 32)
         tiles = t * 4 // 128 + 16
         for entry in range(1, 9):
@@ -625,6 +626,9 @@ def test_moe_step_geometry_forms(group, hidden, inter):
                 assert new[0].grid == (hidden // 256 * tiles, 1, 1) and new[0].block == (512, 1, 1)
             elif wide and entry == _abi.MOE_QUANT_HIDDEN:
                 assert new[1] == ""
+            elif t <= 32 and group == 128 and entry == _abi.MOE_ROUTE:
+                assert new[1] == "lf_moe_route_sort_q" and old[1] == "lf_moe_route_sort"
+                assert new[0].grid == (9, 1, 1) and new[0].block == old[0].block
             elif 32 < t <= 256 and entry in (_abi.MOE_ROUTE, _abi.MOE_SORT_COUNT, _abi.MOE_SORT, _abi.MOE_QUANT_TOKENS):
                 name = {_abi.MOE_ROUTE: "route", _abi.MOE_SORT_COUNT: "sort_count", _abi.MOE_SORT: "sort",
                         _abi.MOE_QUANT_TOKENS: "quant_tokens"}[entry]

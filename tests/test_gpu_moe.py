@@ -313,6 +313,32 @@ def test_moe_t256_row_boundaries(rt, block):
     check_output(x, weights, ex, w, out, block, f"moe t256 row boundaries block={block}", st)
 
 
+@pytest.mark.parametrize("t,e,k,mode,hidden", [(32, 64, 6, 1, 256), (1, 8, 2, 0, 128), (17, 129, 5, 1, 640),
+                                               (0, 8, 2, 0, 256), (63, 256, 16, 0, 384)])
+def test_route_sort_q_equals_route_sort(rt, t, e, k, mode, hidden):
+    """lf_moe_route_sort_q (the token quantizer on blocks of its own) against
+    lf_moe_route_sort: the whole workspace up to the quantized tokens' scales,
+    byte for byte."""
+    from lunaflux_amd import moe
+    from lunaflux_amd.device import KernelArguments, KernelLaunchDimensions
+    from lunaflux_amd.fp8 import LaunchStep, _region
+    rng = np.random.default_rng(980 + t + e)
+    desc = moe.moe_descriptor(e, k, mode, hidden, 128, 128)
+    ctx, prof = rt.context, max(t, 1)
+    xa, la = ctx.upload(synth.activations(rng, prof, hidden)), ctx.upload(rng.standard_normal((prof, e)).astype(np.float32))
+    da, counts, nbytes = ctx.upload(desc.as_bytes()), rt.step_counts(t, decode=False), moe.workspace_bytes(desc, prof)
+    end = moe.workspace_layout(desc, t)["h"]
+    got = []
+    for name, grid in (("lf_moe_route_sort", 1), ("lf_moe_route_sort_q", 9), ("lf_moe_route_sort_q", 2)):
+        ws = ctx.allocate(nbytes)
+        ws.copy_from_host(np.zeros(nbytes, np.uint8))
+        args = [_region(counts, 20, alignment=4), _region(da, 32, alignment=4), _region(la), _region(xa), _region(ws)]
+        LaunchStep(rt.function(name), KernelLaunchDimensions.new((grid,), (1024,)), KernelArguments(args),
+                   name).launch(rt.stream)
+        got.append(ws.read(np.uint8, (end,)))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
 @pytest.mark.parametrize("rows,k,hidden,inter,zero", [
     # rows per expert around the 16-row fragments, the 64-row wave halves and
     # the 128-row tiles; two and one k-tiles
@@ -320,6 +346,7 @@ def test_moe_t256_row_boundaries(rt, block):
     ([40, 3, 0, 21], 1, 3072, 256, False),      # the most k-tiles of gate/up, two of down
     ([140, 0, 9, 5], 1, 256, 3072, True),       # the most of down; all-zero groups and blocks
     ([90, 70, 200, 12, 64, 33], 2, 768, 384, True),
+    ([1, 0, 0, 17, 2], 1, 256, 256, False),     # a decode step
 ])
 def test_moe_t128x256(rt, rows, k, hidden, inter, zero):
     """Block-scaled profiles above 32 tokens on 128 x 256 tiles: exact rows
@@ -332,7 +359,8 @@ def test_moe_t128x256(rt, rows, k, hidden, inter, zero):
     desc = moe.moe_descriptor(e, k, 1, hidden, inter, 128)
     names = [moe.step_geometry(s, desc, t)[1] for s in (_abi.MOE_ROUTE, _abi.MOE_GATE_UP, _abi.MOE_QUANT_HIDDEN,
                                                         _abi.MOE_DOWN)]
-    assert names == ["lf_moe_route", "lf_moe_gate_up_t128x256_b128_q", "", "lf_moe_down_t128x256_b128"]
+    assert names == ["lf_moe_route" if t > 32 else "lf_moe_route_sort_q", "lf_moe_gate_up_t128x256_b128_q", "",
+                     "lf_moe_down_t128x256_b128"]
     rng = np.random.default_rng(970 + total + hidden)
     logits = (0.1 * rng.standard_normal((t, e))).astype(np.float32)
     if k == 1:
