@@ -1707,9 +1707,24 @@ LF_DEVICE void w8a8_split_gemm(const int32_t *counts, const uint8_t *xq, const u
     }
     __syncthreads();
     if (last_block == 0) return;
-    // the S partials in slice order, this block's own from its registers
+    // the S partials in slice order, this block's own from its registers (the
+    // sum's order must not depend on which block came last)
+    f32x4 own[T::kFM][T::kFN];
+#pragma unroll
+    for (int i = 0; i < T::kFM; ++i)
+#pragma unroll
+      for (int j = 0; j < T::kFN; ++j) {
+        own[i][j] = acc[i][j];
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
     for (int slice = 0; slice < S; ++slice) {
-      if (slice == s) continue;
+      if (slice == s) {
+#pragma unroll
+        for (int i = 0; i < T::kFM; ++i)
+#pragma unroll
+          for (int j = 0; j < T::kFN; ++j) acc[i][j] += own[i][j];
+        continue;
+      }
       uint64_t v[T::kFM][T::kFN][2];
 #pragma unroll
       for (int i = 0; i < T::kFM; ++i)

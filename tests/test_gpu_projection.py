@@ -597,8 +597,9 @@ def test_w8a16_gemm_form_any_width(rt, op, n, k, m, max_tokens):
 def test_w8a8_split_form(rt, op, n, k, max_tokens, ms, slices):
     """The split W8A8 form (act-quant launch, then 128 x 256 tiles with K cut
     into slices) as the bindings take it: ragged live rows on one workspace,
-    two launches bit for bit, rows past M untouched, against the oracle over
-    a column sample (the quantized rows are the act-quant launch's)."""
+    eight launches bit for bit (whichever slice arrives last), rows past M
+    untouched, against the oracle over a column sample (the quantized rows are
+    the act-quant launch's)."""
     from lunaflux_amd import _abi, fp8
     from lunaflux_amd.fp8 import _region
     rng = np.random.default_rng(9300 + n + k)
@@ -621,12 +622,12 @@ def test_w8a8_split_form(rt, op, n, k, max_tokens, ms, slices):
         x = synth.activations(rng, max_tokens, k)
         xa.copy_from_host(x)
         outs = []
-        for _ in range(2):
+        for _ in range(8):
             ya.copy_from_host(np.full(max_tokens * n, 0x7FC1, np.uint16))
             bound.launch(rt.stream, synchronous=True)
             outs.append(ya.read(np.uint16, (max_tokens, n)))
             assert np.all(outs[-1][m:] == 0x7FC1), f"{sym} m={m}: rows past M written"
-        assert np.array_equal(outs[0], outs[1]), f"{sym} m={m}: launches differ"
+        assert all(np.array_equal(outs[0], y) for y in outs[1:]), f"{sym} m={m}: launches differ"
         if m == 0:
             continue
         rows = np.unique(np.concatenate([[0, m - 1], rng.integers(0, m, 24)]))
