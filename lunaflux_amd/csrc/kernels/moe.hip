@@ -1782,31 +1782,29 @@ LF_DEVICE void grouped_gemv(const int32_t *counts, const MoeDesc &d, const uint8
 }
 
 // --- combine -------------------------------------------------------------------
-LF_DEVICE void combine(const int32_t *counts, const MoeDesc &d, uint8_t *ws, uint16_t *out) {
-  const int T = live_rows(counts, 1 << 30);
-  const int t = blockIdx.x;
-  if (t >= T) return;
-  const MoeLayout L(d, T);
-  const int H = d.hidden;
-  const float *w = at<float>(ws, L.topk_w) + static_cast<uint64_t>(t) * d.top_k;
-  const int32_t *pos = at<int32_t>(ws, L.pos) + static_cast<uint64_t>(t) * d.top_k;
-  const uint16_t *y = at<uint16_t>(ws, L.y);
+// A block per token: its k rows of y read, its row of out written. Bound by
+// HBM for many tokens and by the chain counts -> position -> row for few.
+// K > 0: top_k is K, so the positions and weights come in a few wide scalar
+// loads, all k rows are in flight together and the registers are those of k
+// rows (4096 tokens of 2048, top 6, 116 MB: 28.9 -> 18.9 us, 6.1 TB/s; 32
+// tokens 5.1 -> 4.6); K = 0: any top_k, each term behind its own branch.
+template <int K>
+LF_DEVICE void combine_row(const float *w, const int32_t *pos, const uint16_t *y, int k, int H, uint16_t *out) {
   // eight columns per thread (H % 128 == 0); the k rows' loads are all
   // issued before the sum, whose terms are added in slot order j
-  constexpr int kMaxK = 16;  // desc_ok bounds top_k
-  const int k = d.top_k;
+  constexpr int kSlots = K > 0 ? K : 16;  // desc_ok bounds top_k
   for (int c = 8 * threadIdx.x; c < H; c += 8 * blockDim.x) {
-    u32x4 v[kMaxK];
-    static_for<kMaxK>([&](auto j) {
-      if (j < k) v[j] = *reinterpret_cast<const u32x4 *>(y + static_cast<uint64_t>(pos[j]) * H + c);
+    u32x4 v[kSlots];
+    static_for<kSlots>([&](auto j) {
+      if (K > 0 || j < k) v[j] = *reinterpret_cast<const u32x4 *>(y + static_cast<uint64_t>(pos[j]) * H + c);
     });
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    static_for<kMaxK>([&](auto j) {
+    static_for<kSlots>([&](auto j) {
       // product and sum each rounded (no fused multiply-add), as the combine
       // is defined: the output is then bit-identical to that definition for
       // the same y and weights
 #pragma clang fp contract(off)
-      if (j < k) {
+      if (K > 0 || j < k) {
         const float wj = w[j];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
@@ -1819,7 +1817,30 @@ LF_DEVICE void combine(const int32_t *counts, const MoeDesc &d, uint8_t *ws, uin
     u32x4 packed;
 #pragma unroll
     for (int q = 0; q < 4; ++q) packed[q] = f32_to_bf16(acc[2 * q]) | (f32_to_bf16(acc[2 * q + 1]) << 16);
-    *reinterpret_cast<u32x4 *>(out + static_cast<uint64_t>(t) * H + c) = packed;
+    *reinterpret_cast<u32x4 *>(out + c) = packed;
+  }
+}
+
+LF_DEVICE void combine(const int32_t *counts, const MoeDesc &d, uint8_t *ws, uint16_t *out) {
+  const int T = live_rows(counts, 1 << 30);
+  const int t = blockIdx.x;
+  if (t >= T) return;
+  const MoeLayout L(d, T);
+  const int H = d.hidden, k = d.top_k;
+  const float *w = at<float>(ws, L.topk_w) + static_cast<uint64_t>(t) * k;
+  const int32_t *pos = at<int32_t>(ws, L.pos) + static_cast<uint64_t>(t) * k;
+  const uint16_t *y = at<uint16_t>(ws, L.y);
+  uint16_t *row = out + static_cast<uint64_t>(t) * H;
+  switch (k) {
+    case 1: return combine_row<1>(w, pos, y, k, H, row);
+    case 2: return combine_row<2>(w, pos, y, k, H, row);
+    case 3: return combine_row<3>(w, pos, y, k, H, row);
+    case 4: return combine_row<4>(w, pos, y, k, H, row);
+    case 5: return combine_row<5>(w, pos, y, k, H, row);
+    case 6: return combine_row<6>(w, pos, y, k, H, row);
+    case 7: return combine_row<7>(w, pos, y, k, H, row);
+    case 8: return combine_row<8>(w, pos, y, k, H, row);
+    default: return combine_row<0>(w, pos, y, k, H, row);
   }
 }
 

@@ -339,6 +339,17 @@ def test_route_sort_q_equals_route_sort(rt, t, e, k, mode, hidden):
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16])
+def test_moe_combine_every_top_k(rt, k):
+    """The combine's body per top_k (1 to 8) and its general one, on a width
+    of more than one pass of a block: bit for bit on the device's y."""
+    rng = np.random.default_rng(990 + k)
+    t, e, hidden, inter = 5, 16, 2176, 128
+    x, logits, weights, out, st = run_case(rt, rng, t, e, k, hidden, inter, 1)
+    ex, w = check_routing(logits, k, 1, st)
+    check_output(x, weights, ex, w, out, False, f"moe combine k={k}", st)
+
+
 @pytest.mark.parametrize("rows,k,hidden,inter,zero", [
     # rows per expert around the 16-row fragments, the 64-row wave halves and
     # the 128-row tiles; two and one k-tiles
