@@ -345,7 +345,7 @@ def test_moe_combine_every_top_k(rt, k):
     of more than one pass of a block: bit for bit on the device's y."""
     rng = np.random.default_rng(990 + k)
     t, e, hidden, inter = 5, 16, 2176, 128
-    x, logits, weights, out, st = run_case(rt, rng, t, e, k, hidden, inter, 1)
+    x, logits, weights, out, st = run_case(rt, rng, t, e, k, hidden, inter, 1, block=False)
     ex, w = check_routing(logits, k, 1, st)
     check_output(x, weights, ex, w, out, False, f"moe combine k={k}", st)
 
