@@ -487,7 +487,9 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry,
  * of more than 32 tokens run the four routing launches, block-scaled ones of
  * at most 32 (and 1024 assignments)
  *  lf_moe_route_sort_q (counts, desc, logits, x, ws) in place of
- * lf_moe_route_sort, and block-scaled ones with K <= 3072 in both GEMMs and a
+ * lf_moe_route_sort, larger block-scaled ones
+ *  lf_moe_route_q (counts, desc, logits, x, ws)
+ * in place of lf_moe_route and lf_moe_quant_tokens, and block-scaled ones with K <= 3072 in both GEMMs and a
  * hidden width that is a multiple of 256
  *  lf_moe_gate_up_t128x256_b128_q (counts, desc, wg, wu, ws)
  *  lf_moe_down_t128x256_b128      (counts, desc, wd, ws)

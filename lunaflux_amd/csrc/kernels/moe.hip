@@ -1865,8 +1865,8 @@ __global__ __launch_bounds__(256) void lf_moe_route(const int32_t *counts, const
 
 // The router and, in the grid's second row, the per-128-column token
 // quantizer, which needs no routing: profiles above the one-block router's.
-// Each is a few us of latency; as launches of their own they took 5.6 and 9.1
-// us for 4096 tokens of 2048.
+// Each is a few us of latency: launches of their own took 5.6 and 9.1 us for
+// 4096 tokens of 2048, this one 10.3.
 __global__ __launch_bounds__(256) void lf_moe_route_q(const int32_t *counts, const int32_t *desc,
                                                       const float *logits, const uint16_t *x, uint8_t *ws) {
   const MoeDesc d = desc_of(desc);

@@ -1222,6 +1222,11 @@ static int32_t moe_geometry(int32_t entry, const lf_fp8_moe_desc *d, int32_t max
       }
       name = "lf_moe_route";
       gx = (T + 3) / 4;
+      if (step && b128) {  // the second grid row quantizes the tokens
+        name = "lf_moe_route_q";
+        gx = std::max(gx, group_quant_blocks(T * (d->hidden / 128)));
+        gy = 2;
+      }
       break;
     // The sort: one 1024-thread block per chunk of 1024 assignments.
     case LF_FP8_MOE_SORT_COUNT:
@@ -1236,7 +1241,7 @@ static int32_t moe_geometry(int32_t entry, const lf_fp8_moe_desc *d, int32_t max
       bx = 1024;
       break;
     case LF_FP8_MOE_QUANT_TOKENS:
-      if (one_block) {  // quantized by lf_moe_route_sort
+      if (one_block || (step && b128)) {  // quantized by the route step's launch
         std::memset(dims, 0, 7 * sizeof(int32_t));
         std::memset(symbol, 0, LF_FP8_SYMBOL_BYTES);
         return LF_OK;

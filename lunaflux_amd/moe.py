@@ -101,7 +101,9 @@ def bind_moe(rt: ProjectionRuntime, counts, desc: MoeDescriptor, desc_region: Ke
     the workspace's counter area as a fifth operand and its error word read
     after a synchronous launch) runs it, and the two sort steps and the
     token quantizer when the route step's kernel (lf_moe_route_sort,
-    profiles of at most 32 tokens and 1024 assignments) does their work."""
+    profiles of at most 32 tokens and 1024 assignments) does their work;
+    with block scales the token quantizer also runs beside the router above
+    32 tokens (lf_moe_route_q)."""
     e, h, i = desc.experts, desc.hidden, desc.inter
     mode = _abi.LF_FP8_SCALE_BLOCK128 if desc.group == 128 else _abi.LF_FP8_SCALE_PER_CHANNEL
     for w, rows, cols in ((wg, i, h), (wu, i, h), (wd, h, i)):

@@ -629,6 +629,12 @@ def test_moe_step_geometry_forms(group, hidden, inter):
             elif t <= 32 and group == 128 and entry == _abi.MOE_ROUTE:
                 assert new[1] == "lf_moe_route_sort_q" and old[1] == "lf_moe_route_sort"
                 assert new[0].grid == (9, 1, 1) and new[0].block == old[0].block
+            elif t > 32 and group == 128 and entry == _abi.MOE_ROUTE:
+                quant = min(1024, -(-t * (hidden // 128) // 16))
+                assert new[1] == "lf_moe_route_q" and new[0].block == (256, 1, 1)
+                assert new[0].grid == (max(-(-t // 4), quant), 2, 1)
+            elif t > 32 and group == 128 and entry == _abi.MOE_QUANT_TOKENS:
+                assert new[1] == ""
             elif 32 < t <= 256 and entry in (_abi.MOE_ROUTE, _abi.MOE_SORT_COUNT, _abi.MOE_SORT, _abi.MOE_QUANT_TOKENS):
                 name = {_abi.MOE_ROUTE: "route", _abi.MOE_SORT_COUNT: "sort_count", _abi.MOE_SORT: "sort",
                         _abi.MOE_QUANT_TOKENS: "quant_tokens"}[entry]

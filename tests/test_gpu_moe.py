@@ -339,6 +339,36 @@ def test_route_sort_q_equals_route_sort(rt, t, e, k, mode, hidden):
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("t,prof,e,k,mode,hidden", [(33, 33, 64, 6, 1, 256), (250, 256, 129, 5, 1, 3968),
+                                                    (0, 64, 8, 2, 0, 256), (1, 40, 256, 16, 0, 128)])
+def test_route_q_equals_two_launches(rt, t, prof, e, k, mode, hidden):
+    """lf_moe_route_q on the profile's grid and on a smaller one against
+    lf_moe_route and lf_moe_quant_tokens: the whole workspace up to the
+    quantized tokens' scales, byte for byte, live tokens below the profile's."""
+    from lunaflux_amd import _abi, moe
+    from lunaflux_amd.device import KernelArguments, KernelLaunchDimensions
+    from lunaflux_amd.fp8 import LaunchStep, _region
+    rng = np.random.default_rng(985 + t + e)
+    desc = moe.moe_descriptor(e, k, mode, hidden, 128, 128)
+    ctx = rt.context
+    xa, la = ctx.upload(synth.activations(rng, prof, hidden)), ctx.upload(rng.standard_normal((prof, e)).astype(np.float32))
+    da, counts, nbytes = ctx.upload(desc.as_bytes()), rt.step_counts(t, decode=False), moe.workspace_bytes(desc, prof)
+    end = moe.workspace_layout(desc, t)["h"]
+    grid = moe.step_geometry(_abi.MOE_ROUTE, desc, prof)[0].grid
+    routes = -(-prof // 4)
+    got = []
+    for launches in ([("lf_moe_route", (routes,), True), ("lf_moe_quant_tokens", (7,), False)],
+                     [("lf_moe_route_q", grid[:2], True)], [("lf_moe_route_q", (routes, 2), True)]):
+        ws = ctx.allocate(nbytes)
+        ws.copy_from_host(np.zeros(nbytes, np.uint8))
+        for name, g, routed in launches:
+            args = [_region(counts, 20, alignment=4), _region(da, 32, alignment=4)] + ([_region(la)] if routed else [])
+            LaunchStep(rt.function(name), KernelLaunchDimensions.new(g, (256,)),
+                       KernelArguments(args + [_region(xa), _region(ws)]), name).launch(rt.stream)
+        got.append(ws.read(np.uint8, (end,)))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16])
 def test_moe_combine_every_top_k(rt, k):
     """The combine's body per top_k (1 to 8) and its general one, on a width
@@ -370,7 +400,7 @@ def test_moe_t128x256(rt, rows, k, hidden, inter, zero):
     desc = moe.moe_descriptor(e, k, 1, hidden, inter, 128)
     names = [moe.step_geometry(s, desc, t)[1] for s in (_abi.MOE_ROUTE, _abi.MOE_GATE_UP, _abi.MOE_QUANT_HIDDEN,
                                                         _abi.MOE_DOWN)]
-    assert names == ["lf_moe_route" if t > 32 else "lf_moe_route_sort_q", "lf_moe_gate_up_t128x256_b128_q", "",
+    assert names == ["lf_moe_route_q" if t > 32 else "lf_moe_route_sort_q", "lf_moe_gate_up_t128x256_b128_q", "",
                      "lf_moe_down_t128x256_b128"]
     rng = np.random.default_rng(970 + total + hidden)
     logits = (0.1 * rng.standard_normal((t, e))).astype(np.float32)
