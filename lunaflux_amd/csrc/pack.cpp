@@ -1154,13 +1154,13 @@ int64_t lunaflux_fp8_moe_sync_offset(const lf_fp8_moe_desc *d, int32_t max_token
 // Block-scaled profiles: 128 x 256 tiles (kernels/moe.hip,
 // grouped_gemm_t128x256), where both K fit its scale table and its 32-bit
 // activation offsets. Against the forms moe_geometry gives
-// below, gate/up + down (+ hidden quantizer) of 64 experts of 2048 x 1408,
-// top 6, us: whole operation on the GEMV form 4 tokens 49.0 -> 47.6, 12 tokens
-// 63.9 -> 58.3, 32 tokens 93.1 -> 91.8 (no hidden quantizer launch); 60 tokens 153 -> 82, 250 tokens 211 -> 114, 900 tokens 323 ->
-// 154, 1500 tokens 432 -> 192 (all 128 x 128 tiles before), 4096 tokens 369
-// -> 355 (256 x 256). Per-channel profiles stay on their forms: 8 experts of
-// 4096 x 14336, top 2, gate/up + down 60 tokens 271 -> 264, 250 tokens 297 ->
-// 289, but 1024 tokens 497 -> 513 us.
+// below, 64 experts of 2048 x 1408, top 6, us: whole operation on the GEMV
+// form 4 tokens 49.0 -> 47.6, 12 tokens 63.9 -> 58.3, 32 tokens 93.1 -> 91.8
+// (no hidden quantizer launch); gate/up + down 60 tokens 153 -> 82, 250 tokens
+// 211 -> 114, 900 tokens 323 -> 154, 1500 tokens 432 -> 192 (all 128 x 128
+// tiles before), 4096 tokens 369 -> 355 (256 x 256). Per-channel profiles stay
+// on their forms: 8 experts of 4096 x 14336, top 2, gate/up + down 60 tokens
+// 271 -> 264, 250 tokens 297 -> 289, but 1024 tokens 497 -> 513 us.
 static bool moe_t128x256(const lf_fp8_moe_desc *d, int64_t T) {
   constexpr int64_t kMaxK = 128 * 24;  // kT128x256MaxKT
   return d->group == 128 && d->hidden % 256 == 0 && d->hidden <= kMaxK && d->inter <= kMaxK &&
