@@ -150,7 +150,9 @@ int32_t lunaflux_fp8_unpack_weight(const uint8_t *region, int64_t region_bytes,
 int64_t lunaflux_fp8_act_quant_bytes(int64_t max_rows, int64_t columns);
 /* Split-K workspace of a W8A16 entry for (N, K, max_query_tokens): fp32
  * partial tiles plus one arrival counter per column group; -1 if the shape
- * is not supported (N % 16, K % 128, max > 128). */
+ * is not supported (N % 16, K % 128, max > 128). QKV entries: N is the packed
+ * width, and the size covers whichever entry of that width the geometry picks
+ * once it is given the Q / K-V split. */
 int64_t lunaflux_fp8_w8a16_workspace_bytes(int32_t entry, int64_t n, int64_t k,
                                            int32_t max_tokens);
 
@@ -213,9 +215,7 @@ enum lf_fp8_entry {
  *  W8A16 shape-specialized (Llama-3-8B widths, profiles of <= 32 rows, as
  *      the per-channel ones): lf_fp8_w8a16_{dense,gate_up}_b128_k{K}_mM,
  *      lf_fp8_w8a16_qkv_b128_k4096_q4096_kv1024_mM (picked by
- *      lunaflux_fp8_qkv_launch_geometry; without the split,
- *      lunaflux_fp8_w8a16_workspace_bytes sizes the QKV_B128 workspace for
- *      every entry of that width). W8A16 GatedMlp in one launch with
+ *      lunaflux_fp8_qkv_launch_geometry). W8A16 GatedMlp in one launch with
  *      LF_FP8_ENTRY_W8A16_GATED_MLP_B128 (the per-channel one-launch forms:
  *      lf_fp8_w8a16_gated_mlp_b128_h4096_i14336_m{16,32} and
  *      lf_fp8_w8a16_gated_mlp_b128_m128_n128_n{64,128}; workspace and error

@@ -645,6 +645,20 @@ int64_t lunaflux_fp8_act_quant_bytes(int64_t max_rows, int64_t columns) {
   return align_up(max_rows * columns, 256) + align_up(max_rows * 4, 256);
 }
 
+// A QKV size asked for without the Q / K-V split (nq = 0) also covers the
+// specialized entries of that width, one of which the geometry, given the
+// split, may pick; 0 for every other call.
+static int64_t w8a16_unknown_split_workspace(int32_t entry, int64_t n, int64_t k, int64_t nq, int32_t max_tokens) {
+  int64_t need = 0;
+  if ((entry != LF_FP8_ENTRY_W8A16_QKV && entry != LF_FP8_ENTRY_W8A16_QKV_B128) || nq != 0) return need;
+  for (const W8a16Fixed &f : kW8a16Fixed) {
+    if (f.entry == entry && n == f.nq + 2 * f.nkv && w8a16_fixed(entry, n, k, f.nq, f.nkv, max_tokens) == &f) {
+      need = std::max(need, w8a16_fixed_workspace(f, n));
+    }
+  }
+  return need;
+}
+
 static int64_t w8a16_workspace(int32_t entry, int64_t n, int64_t k, int64_t nq, int64_t nkv,
                                int32_t max_tokens) {
   if (w8a16_b128_entry(entry)) {
@@ -659,21 +673,10 @@ static int64_t w8a16_workspace(int32_t entry, int64_t n, int64_t k, int64_t nq, 
       return w8a16_fixed_workspace(*f, n);
     }
     const int64_t nw = entry == LF_FP8_ENTRY_W8A16_GATE_UP_B128 ? 2 : 1;
-    int64_t need = sp.split == 1 ? 256
-                                 : align_up(sp.split * (n / 16) * nw * sp.mt * 1024, 256) +
-                                       align_up(sp.groups * 4, 256);
-    // QKV without its Q / K-V split: also room for the workspace of any
-    // specialized entry of this width (the geometry, given the split, may
-    // pick one)
-    if (entry == LF_FP8_ENTRY_W8A16_QKV_B128 && nq == 0) {
-      for (const W8a16Fixed &f : kW8a16Fixed) {
-        if (f.entry == entry && n == f.nq + 2 * f.nkv &&
-            w8a16_fixed(entry, n, k, f.nq, f.nkv, max_tokens) == &f) {
-          need = std::max(need, w8a16_fixed_workspace(f, n));
-        }
-      }
-    }
-    return need;
+    const int64_t need = sp.split == 1 ? 256
+                                       : align_up(sp.split * (n / 16) * nw * sp.mt * 1024, 256) +
+                                             align_up(sp.groups * 4, 256);
+    return std::max(need, w8a16_unknown_split_workspace(entry, n, k, nq, max_tokens));
   }
   if (entry != LF_FP8_ENTRY_W8A16_DENSE && entry != LF_FP8_ENTRY_W8A16_QKV &&
       entry != LF_FP8_ENTRY_W8A16_GATE_UP) {
@@ -689,13 +692,15 @@ static int64_t w8a16_workspace(int32_t entry, int64_t n, int64_t k, int64_t nq, 
   if (const W8a16Fixed *f = w8a16_fixed(entry, n, k, nq, nkv, max_tokens)) {
     return w8a16_fixed_workspace(*f, n);
   }
-  if (sp.split == 1) return 256;
   // One 1 KiB fp32 accumulator fragment per (slice, 16-column tile, weight,
   // 16-row tile), then one arrival counter per column group. The GEMM form
   // (mt 2, 4) stores whole blocks of tiles.
   const int64_t nw = entry == LF_FP8_ENTRY_W8A16_GATE_UP ? 2 : 1;
   const int64_t tiles = sp.mt == 8 ? n / 16 : sp.groups * kW16Waves;
-  return align_up(sp.split * tiles * nw * sp.mt * 1024, 256) + align_up(sp.groups * 4, 256);
+  const int64_t need = sp.split == 1 ? 256
+                                     : align_up(sp.split * tiles * nw * sp.mt * 1024, 256) +
+                                           align_up(sp.groups * 4, 256);
+  return std::max(need, w8a16_unknown_split_workspace(entry, n, k, nq, max_tokens));
 }
 
 int64_t lunaflux_fp8_w8a16_workspace_bytes(int32_t entry, int64_t n, int64_t k,

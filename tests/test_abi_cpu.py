@@ -258,6 +258,25 @@ def test_w8a16_any_shape_grid_holds_the_kernels_slices(entry, cols, k):
                 assert fp8.w8a16_workspace_bytes(entry, n, k, m) >= need + blocks * 4
 
 
+@pytest.mark.parametrize("entry", [_abi.ENTRY_W8A16_QKV, _abi.ENTRY_W8A16_QKV_B128])
+def test_w8a16_qkv_size_without_the_split_covers_every_entry(entry):
+    """The plain workspace size of a packed QKV width is enough for whichever
+    entry the geometry picks once it is given the split."""
+    for k in (2048, 4096, 8192):
+        for m in (1, 16, 17, 32, 33, 64, 65, 128):
+            plain = fp8.w8a16_workspace_bytes(entry, 6144, k, m)
+            for split in ((4096, 1024), (2048, 2048), (5120, 512)):
+                dims, sym = fp8.launch_geometry(entry, 6144, k, m, qkv_split=split)
+                if entry == _abi.ENTRY_W8A16_QKV:
+                    need = fp8.w8a16_workspace_bytes(entry, 6144, k, m, split)
+                elif "_k4096_" in sym:  # 8 tiles a block at 32 rows, else unsplit
+                    slices = dims.grid[0] * 8 // 384 if m > 16 else 1
+                    need = slices * 384 * 2 * 1024 + 256 if slices > 1 else 256
+                else:
+                    need = plain
+                assert plain >= need, (k, m, split, sym, plain, need)
+
+
 def test_w8a8_split_geometry():
     """The split W8A8 form: at most 256 tiles of 128 x 256, K from 2048, at
     most 2048 rows; slices of at least 14 k-tiles, at most four, at most 256
