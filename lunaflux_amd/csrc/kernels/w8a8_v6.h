@@ -72,8 +72,9 @@ struct Plan {
 //   row(kt, i): the scale of this lane's row of fragment row i (an LDS read)
 //   block(kt, p): the weight scale of part p (wave-uniform); p = 1: the up
 //     fragments of a gate/up block (kParts == 2: j >= kFN / 2)
-// The scales of k-tile kt are read until its last fragment row, when stage
-// kt + NS may already be landing.
+// The scales of k-tile kt are read after the barrier that publishes its stage
+// (scales an issue() loads land with it) and until its last fragment row, when
+// stage kt + NS may already be landing.
 // LIVE: the wave's fragment rows that hold a live row (the others' sums stay
 // zero and are never stored); its loads and barriers are those of every wave.
 template <class T, class SCALES, int LIVE = T::kFM>
@@ -83,6 +84,9 @@ LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)
   constexpr int kBarrierRow = FM - R;
   constexpr int kIns = T::kAIns + T::kBIns + SCALES::kIns;
   constexpr bool FOLD = SCALES::kFold;
+  // the row at which the next k-tile's first row scale is read: the last live
+  // row, or the barrier's (after it) where the live rows end before that
+  constexpr int kNextScaleRow = LIVE - 1 > kBarrierRow ? LIVE - 1 : kBarrierRow;
   static_assert((NS - 1) * kIns < 64, "vmcnt range");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
@@ -172,7 +176,7 @@ LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)
       if constexpr (FOLD && i < LIVE) {
         if constexpr (i + 1 < LIVE) {
           sa = scales.row(kt, i + 1);
-        } else if constexpr (NEXT) {
+        } else if constexpr (NEXT && i == kNextScaleRow && i > kBarrierRow) {
           sa = scales.row(kt + 1, 0);
         }
       }
@@ -207,6 +211,7 @@ LF_DEVICE void mainloop(const Plan<T> &plan, int KT, uint8_t *smem, f32x4 (&acc)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (FOLD) {
+          if constexpr (LIVE > 0 && i == kNextScaleRow) sa = scales.row(kt + 1, 0);
 #pragma unroll
           for (int p = 0; p < P; ++p) nsw[p] = scales.block(kt + 1, p);
         }
