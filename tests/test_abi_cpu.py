@@ -868,3 +868,24 @@ def test_block_scaled_weights_bind_their_own_entries():
     with pytest.raises(fp8.DeviceError) as err:
         fp8.ProjectionRuntime.bind_dense_quantized(None, None, None, w, None, 16)
     assert err.value.status == _abi.LF_UNSUPPORTED
+
+
+@pytest.mark.parametrize("n,k,max_tokens", [(6144, 4096, 512), (3072, 4096, 128), (2048, 2048, 2048), (1024, 1024, 64)])
+def test_dense_quantized_step_holds_no_state(n, k, max_tokens):
+    """The GEMM over quantized rows is one launch of (counts, xq, w, y), also
+    where the split form takes the shape: no workspace, so nothing is
+    allocated and launches of one step may overlap."""
+    from types import SimpleNamespace
+    region = lambda: SimpleNamespace(byte_count=256, ptr=None)
+    head = fp8.pack_weight(np.zeros((16, 128), np.uint8), np.ones(16, np.float32))[:256].copy()
+    w = fp8.Fp8Weight(region(), n, k, 1, fp8.PER_CHANNEL, head)
+    w.admit = lambda entry: None
+    rt = fp8.ProjectionRuntime.__new__(fp8.ProjectionRuntime)
+    rt.function = lambda symbol: symbol
+    rt.context = None                      # (any allocation would fail)
+    arg = lambda: fp8.KernelArgument.device_region(region(), 0, 256, 256)
+    xq, y = arg(), arg()
+    step = rt.bind_dense_quantized(region(), xq, w, y, max_tokens)
+    dims, symbol = fp8.launch_geometry(_abi.ENTRY_W8A8_DENSE, n, k, max_tokens)
+    assert step.name == symbol and step.dims == dims
+    assert step.args.arguments[1:] == [xq, w.region, y]
