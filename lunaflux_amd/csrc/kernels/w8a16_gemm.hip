@@ -145,8 +145,7 @@ __device__ __forceinline__ void w8a16_gemm_kernel(uint8_t *smem, const int32_t *
   const int nb = nblocks < 0 ? static_cast<int>(gridDim.x) : nblocks;
   const int block = bid < 0 ? static_cast<int>(blockIdx.x) : bid;
   // K-slices. Forms below 128 rows: at most w16_slices of them (the rule
-  // and its measurements: there); the geometry's grid may hold more, whose
-  // blocks end here.
+  // and its measurements: there), which is what the geometry launches.
   const int S = T::kPartial ? min(nb / blocks_n, w16_slices(blocks_n, KT)) : nb / blocks_n;
   // A grid whose split is not 1..KT (the geometry rules it out) stores
   // nothing in any block: an empty K-slice would never arrive, and its

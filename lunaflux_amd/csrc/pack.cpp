@@ -62,17 +62,12 @@ inline int64_t swizzled_offset(int64_t n, int64_t k, int64_t columns) {
 // profiles: kW16Waves 16-column tiles per block (gate/up: of both weights),
 // K cut into `split` slices across blocks, partial tiles reduced through the
 // workspace. 17..64 rows (mt 2, 4; block-scaled also mt 1) run the LDS-tiled
-// GEMM of w8a16_gemm.hip, which cuts K into w16_slices slices. Up to
-// kW16DirectK the grid and workspace are sized for about 512 blocks all the
-// same, as they were for the column-group kernels (two blocks per CU): those
-// past the GEMM's slices end at once, on CUs its at most 256 blocks leave
-// free. Wider K runs exactly the GEMM's blocks (a block's LDS rings fill a
-// CU there, so spare blocks would queue behind the others: 4096 x 14336 at
-// M = 61 21.9 us). 65..128 rows of a width that is no multiple of 64 run the
-// column-group form of w8a16.hip on about 512 blocks.
+// GEMM of w8a16_gemm.hip, which cuts K into w16_slices slices: exactly those
+// blocks are launched, as a block's LDS rings leave room for one or two per
+// CU and a spare block costs its start. 65..128 rows of a width that is no
+// multiple of 64 run the column-group form of w8a16.hip on about 512 blocks.
 constexpr int kW16Waves = 4;
 constexpr int kW16TileWaves = 8;
-constexpr int64_t kW16DirectK = 2048;
 // kernels/w8a16_gemm.hip, w16_slices
 int64_t w16_slices(int64_t blocks_n, int64_t kt) {
   return std::max<int64_t>(1, std::min<int64_t>(256 / blocks_n, kt / 8));
@@ -96,10 +91,8 @@ bool w8a16_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
     return tiles <= INT32_MAX;
   }
   const int64_t groups = (tiles + kW16Waves - 1) / kW16Waves;
-  int64_t split = (512 + groups / 2) / groups;
-  if (split < 1) split = 1;
-  if (split > kt) split = kt;
-  if (mt != 8 && k > kW16DirectK) split = w16_slices(groups, kt);
+  const int64_t split = mt == 8 ? std::min(kt, std::max<int64_t>(1, (512 + groups / 2) / groups))
+                                : w16_slices(groups, kt);
   if (groups * split > INT32_MAX) return false;
   out->groups = groups;
   out->split = split;
@@ -110,9 +103,10 @@ bool w8a16_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
 // LDS-tiled GEMM form with the per-channel entries' tile and split
 // (w8a16_gemm below, the _b128_m128_n{BN} symbols; every block-scaled width
 // is a multiple of 128, so a 16-column fragment lies in one 128-row scale
-// block); every other profile (also <= 16 rows) the GEMM form's _b128_m16 /
-// _m32 / _m64 entries, the grid sized as above and for slices of at most 128
-// k-tiles.
+// block), except vocabulary-wide dense shapes, which keep the column-group
+// form (its block scales of a slice are staged in LDS: at most 128 k-tiles);
+// every other profile (also <= 16 rows) the GEMM form's _b128_m16 / _m32 /
+// _m64 entries, the grid as above.
 bool w8a16_b128_entry(int32_t e) {
   return e == LF_FP8_ENTRY_W8A16_DENSE_B128 || e == LF_FP8_ENTRY_W8A16_QKV_B128 ||
          e == LF_FP8_ENTRY_W8A16_GATE_UP_B128;
@@ -129,11 +123,9 @@ bool w8a16_b128_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out)
   if (out->one_tile) {  // <= 16 rows: the GEMM form too
     out->one_tile = false;
     out->groups = (tiles + kW16Waves - 1) / kW16Waves;
-    out->split = k > kW16DirectK
-                     ? w16_slices(out->groups, kt)
-                     : std::min<int64_t>(kt, std::max<int64_t>(1, (512 + out->groups / 2) / out->groups));
+    out->split = w16_slices(out->groups, kt);
   }
-  out->split = std::max<int64_t>(out->split, (kt + 127) / 128);
+  if (out->mt == 8) out->split = std::max<int64_t>(out->split, (kt + 127) / 128);
   return out->groups * out->split <= INT32_MAX;
 }
 

@@ -109,22 +109,24 @@ def test_region_size_validation():
 
 def test_launch_geometry():
     # W8A16 generic forms, max rows <= 16: one 16-column tile per 8-wave
-    # block, K split across its waves. Larger profiles: 4 column tiles per
-    # 4-wave block, K cut into about 512 / groups slices across blocks.
+    # block, K split across its waves. Up to 64 rows: 4 column tiles per
+    # block, K cut into min(256 / groups, k-tiles / 8) slices across blocks.
     dims, sym = fp8.launch_geometry(_abi.ENTRY_W8A16_DENSE, 4096, 2048, 32)
-    assert sym == "lf_fp8_w8a16_dense_m32" and dims.grid == (64 * 8, 1, 1) and dims.block == (256, 1, 1)
+    assert sym == "lf_fp8_w8a16_dense_m32" and dims.grid == (64 * 2, 1, 1) and dims.block == (256, 1, 1)
     dims, sym = fp8.launch_geometry(_abi.ENTRY_W8A16_QKV, 6144, 4096, 1)
     assert sym == "lf_fp8_w8a16_qkv_m16_t1" and dims.grid == (384, 1, 1) and dims.block == (512, 1, 1)
     dims, sym = fp8.launch_geometry(_abi.ENTRY_W8A16_GATE_UP, 14336, 2048, 32)
-    assert sym == "lf_fp8_w8a16_gate_up_m32" and dims.grid == (224 * 2, 1, 1)
-    # 65..128 rows, N not a multiple of 64: the generic column-group form
+    assert sym == "lf_fp8_w8a16_gate_up_m32" and dims.grid == (224, 1, 1)
+    # 65..128 rows, N not a multiple of 64: the generic column-group form, K
+    # cut into about 512 / groups slices
     dims, sym = fp8.launch_geometry(_abi.ENTRY_W8A16_QKV, 6160, 4096, 128)
     assert sym == "lf_fp8_w8a16_qkv_m128" and dims.grid == (97 * 5, 1, 1)
     # split-K workspace: S x (N / 16) x NW x MT 1 KiB fragments + one counter
     # per column group; 256 bytes (unused) without a split
-    assert fp8.w8a16_workspace_bytes(_abi.ENTRY_W8A16_DENSE, 4096, 2048, 32) == 8 * 256 * 2 * 1024 + 256
+    assert fp8.w8a16_workspace_bytes(_abi.ENTRY_W8A16_DENSE, 4096, 2048, 32) == 2 * 256 * 2 * 1024 + 256
     assert fp8.w8a16_workspace_bytes(_abi.ENTRY_W8A16_QKV, 6144, 4096, 1) == 256
-    assert fp8.w8a16_workspace_bytes(_abi.ENTRY_W8A16_GATE_UP, 14336, 2048, 32) == 2 * 896 * 2 * 2 * 1024 + 1024
+    assert fp8.w8a16_workspace_bytes(_abi.ENTRY_W8A16_GATE_UP, 14336, 2048, 32) == 256
+    assert fp8.w8a16_workspace_bytes(_abi.ENTRY_W8A16_GATE_UP, 4096, 2048, 64) == 2 * 256 * 2 * 4 * 1024 + 256
     assert fp8.w8a16_workspace_bytes(_abi.ENTRY_W8A16_QKV, 6144, 4096, 128) == 2 * 96 * 8 * 4 * 1024 + 512
     # Shape-specialized (Llama-3-8B) entries for profiles of <= 32 rows.
     dims, sym = fp8.launch_geometry(_abi.ENTRY_W8A16_DENSE, 4096, 14336, 32)
@@ -241,9 +243,9 @@ def test_launch_geometry():
 @pytest.mark.parametrize("k", [128, 1024, 2048, 2176, 7168, 28672])
 def test_w8a16_any_shape_grid_holds_the_kernels_slices(entry, cols, k):
     """Profiles of 17..64 rows: the kernel cuts K into max(1, min(256 /
-    blocks, k-tiles / 8)) slices of 64-column blocks; the grid is whole
-    slices, at least that many, and the workspace holds their partial tiles
-    and a counter per block."""
+    blocks, k-tiles / 8)) slices of 64-column blocks; the grid is exactly
+    those, and the workspace holds their partial tiles and a counter per
+    block."""
     for n in (16, 48, 64, 1040, 4096, 7184, 16384, 40000):
         for m in (17, 32, 33, 64):
             dims, sym = fp8.launch_geometry(entry, n, k, m)
@@ -251,7 +253,7 @@ def test_w8a16_any_shape_grid_holds_the_kernels_slices(entry, cols, k):
                 continue
             rows, blocks = (32 if m <= 32 else 64), -(-n // 64)
             slices = max(1, min(256 // blocks, k // 128 // 8))
-            assert dims.grid[0] % blocks == 0 and dims.grid[0] // blocks >= slices
+            assert dims.grid[0] == blocks * slices
             assert dims.block[0] == (256 if rows == 32 else 512)
             if slices > 1:
                 need = slices * blocks * 64 * cols * rows * 4

@@ -533,7 +533,7 @@ def lm_head_weight(rt, rng, vocab, k):
 @pytest.mark.parametrize("op,n,k,m,max_tokens", [
     ("dense", 16, 128, 17, 32),        # one fragment of a block's four, one k-tile
     ("dense", 80, 384, 32, 32),        # a partial second block, three k-tiles
-    ("dense", 4096, 2048, 1, 32),      # two slices of a grid sized for eight
+    ("dense", 4096, 2048, 1, 32),      # two slices
     ("dense", 1072, 4224, 33, 64),     # four slices of 33 k-tiles, partial block
     ("qkv", 112, 1024, 29, 32),        # 80 + 16 + 16: three weights in two blocks
     ("qkv", 1584, 4096, 64, 64),       # 1040 + 272 + 272, boundaries inside blocks

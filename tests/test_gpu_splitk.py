@@ -1,10 +1,12 @@
 """The W8A16 split-K exchange on every form that splits K across blocks:
 the shape-specialized column-group entries of the Llama-3-8B decode layer
-(down K = 14336 and QKV at 32 rows, four slices), the generic column-group
-form (eight slices, the last block loading seven partials in two batches;
-gate/up with sixteen, two weights per tile), and the 128-row GEMM form
-(four slices at BN 64, and six at BN 128: a width the launch geometry no
-longer splits, launched directly, as a caller of the entry may). Every
+(down K = 14336 and QKV at 32 rows, four slices), the any-width GEMM form of
+17..64 rows (two slices, four, and sixteen where columns are few and K is
+large; gate/up with two weights per tile), the column-group form of a width
+that is no multiple of 64 at 128 rows (seven slices, the last block loading
+six partials in two batches), and the 128-row GEMM form (four slices at BN 64,
+and six at BN 128: a width the launch geometry does not split, launched
+directly, as a caller of the entry may). Every
 block stores its partial tile and counts
 itself; the last to arrive sums the S partials in slice order and resets
 the counter. So every launch must match the oracle, be bit-identical to the
@@ -39,8 +41,11 @@ def weight(rt, rng, n, k):
 CASES = [
     ("dense", 4096, 14336, 32, 32, "lf_fp8_w8a16_dense_k14336_m32", 4),
     ("qkv", 6144, 4096, 32, 27, "lf_fp8_w8a16_qkv_k4096_q4096_kv1024_m32", 4),
-    ("dense", 4096, 2048, 32, 17, "lf_fp8_w8a16_dense_m32", 8),
-    ("gate_up", 1024, 2048, 32, 30, "lf_fp8_w8a16_gate_up_m32", 16),
+    ("dense", 4096, 2048, 32, 17, "lf_fp8_w8a16_dense_m32", 2),
+    ("gate_up", 4096, 8192, 32, 30, "lf_fp8_w8a16_gate_up_m32", 4),
+    ("dense", 256, 16384, 64, 61, "lf_fp8_w8a16_dense_m64", 16),
+    ("gate_up", 128, 16384, 32, 25, "lf_fp8_w8a16_gate_up_m32", 16),
+    ("dense", 4624, 2048, 128, 90, "lf_fp8_w8a16_dense_m128", 7),
     ("dense", 4096, 4096, 128, 128, "lf_fp8_w8a16_dense_m128_n64", 4),
     ("dense", 4096, 14336, 128, 77, "lf_fp8_w8a16_dense_m128_n64", 4),
     ("dense", 4096, 14336, 128, 77, "lf_fp8_w8a16_dense_m128_n128", 6),
