@@ -96,12 +96,18 @@ LF_DEVICE void wait_ring(int later) {
 }
 
 // K-slices of the forms below 128 rows: as many as keep 8 k-tiles per slice
-// and one block per CU (256), as the 128-row geometry. Measured (us, M = 24
-// dense 4096 x 2048: 1 / 2 / 3 / 4 / 8 slices 8.8 / 8.1 / 7.9 / 8.0 / 10.0;
-// 4096 x 1024: 1 / 2 / 4 5.7 / 6.2 / 6.8; M = 61 4096 x 7168: 3 / 4 15.7 /
-// 14.8; gate/up 7168 x 4096: 1 / 2 21.2 / 18.7). csrc/pack.cpp holds the
+// and one block per CU (256), as the 128-row geometry; 4 k-tiles where blocks
+// and k-tiles are few, as a block's latency is the whole time there. Measured
+// (us, M = 24 dense 4096 x 2048: 1 / 2 / 3 / 4 / 8 slices 8.8 / 8.1 / 7.9 /
+// 8.0 / 10.0; 4096 x 1024: 1 / 2 / 4 5.7 / 6.2 / 6.8; M = 61 4096 x 7168: 3 /
+// 4 15.7 / 14.8; gate/up 7168 x 4096: 1 / 2 21.2 / 18.7; slices of 8 / 4
+// k-tiles, block-scaled, M = 32: 256 x 1536 7.1 / 6.0 (column groups, before:
+// 6.4), 1024 x 2048 7.4 / 7.0, 2048 x 3072 8.2 / 8.6). csrc/pack.cpp holds the
 // same rule.
-LF_DEVICE int w16_slices(int blocks_n, int kt) { return max(1, min(256 / blocks_n, kt / 8)); }
+LF_DEVICE int w16_slices(int blocks_n, int kt) {
+  const int least = blocks_n <= 32 && kt <= 16 ? 4 : 8;
+  return max(1, min(256 / blocks_n, kt / least));
+}
 
 // MODE 0: dense, 1: QKV (three weights, packed Q|K|V output), 2: gate/up
 // (each wave column's fragments: kFN / 2 gate tiles, then the up tiles of the

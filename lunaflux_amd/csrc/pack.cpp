@@ -70,7 +70,8 @@ constexpr int kW16Waves = 4;
 constexpr int kW16TileWaves = 8;
 // kernels/w8a16_gemm.hip, w16_slices
 int64_t w16_slices(int64_t blocks_n, int64_t kt) {
-  return std::max<int64_t>(1, std::min<int64_t>(256 / blocks_n, kt / 8));
+  const int64_t least = blocks_n <= 32 && kt <= 16 ? 4 : 8;
+  return std::max<int64_t>(1, std::min<int64_t>(256 / blocks_n, kt / least));
 }
 // Threads of the entries that fit any shape above 16 rows.
 int w16_threads(int mt, bool block) { return mt == 4 && !block ? 512 : 64 * kW16Waves; }

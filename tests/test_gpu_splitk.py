@@ -1,7 +1,7 @@
 """The W8A16 split-K exchange on every form that splits K across blocks:
 the shape-specialized column-group entries of the Llama-3-8B decode layer
 (down K = 14336 and QKV at 32 rows, four slices), the any-width GEMM form of
-17..64 rows (two slices, four, and sixteen where columns are few and K is
+17..64 rows (two to four slices, and sixteen where columns are few and K is
 large; gate/up with two weights per tile), the column-group form of a width
 that is no multiple of 64 at 128 rows (seven slices, the last block loading
 six partials in two batches), and the 128-row GEMM form (four slices at BN 64,
@@ -42,6 +42,8 @@ CASES = [
     ("dense", 4096, 14336, 32, 32, "lf_fp8_w8a16_dense_k14336_m32", 4),
     ("qkv", 6144, 4096, 32, 27, "lf_fp8_w8a16_qkv_k4096_q4096_kv1024_m32", 4),
     ("dense", 4096, 2048, 32, 17, "lf_fp8_w8a16_dense_m32", 2),
+    ("gate_up", 1024, 2048, 32, 30, "lf_fp8_w8a16_gate_up_m32", 4),
+    ("dense", 144, 1536, 64, 33, "lf_fp8_w8a16_dense_m64", 3),
     ("gate_up", 4096, 8192, 32, 30, "lf_fp8_w8a16_gate_up_m32", 4),
     ("dense", 256, 16384, 64, 61, "lf_fp8_w8a16_dense_m64", 16),
     ("gate_up", 128, 16384, 32, 25, "lf_fp8_w8a16_gate_up_m32", 16),
