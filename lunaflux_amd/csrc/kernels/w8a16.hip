@@ -1112,45 +1112,36 @@ struct GatedMlpFixed {
 
 extern "C" {
 
-#define LF_W8A16_ENTRIES(MT, M, D, XC)                                                              \
-  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_dense_m##M(              \
+// The column-group form at any shape; BLOCK: weights with 128 x 128 block
+// scales. (Up to 64 rows most shapes run the LDS-tiled GEMM of w8a16_gemm.hip
+// under the _m16 / _m32 / _m64 symbols; _cg_: these, where they are faster.)
+#define LF_W8A16_ENTRIES(SUFFIX, MT, D, XC, BLOCK)                                            \
+  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_dense##SUFFIX(            \
       const int32_t *counts, const uint16_t *x, const uint8_t *w, uint16_t *y, uint8_t *ws) { \
-    w8a16_kernel<LF_W16_WAVES, MT, 0, D, XC>(counts, x, w, w, w, y, ws);              \
-  }                                                                                          \
-  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_qkv_m##M(                \
-      const int32_t *counts, const uint16_t *x, const uint8_t *wq, const uint8_t *wk,        \
-      const uint8_t *wv, uint16_t *y, uint8_t *ws) {                                         \
-    w8a16_kernel<LF_W16_WAVES, MT, 1, D, XC>(counts, x, wq, wk, wv, y, ws);           \
-  }                                                                                          \
-  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_gate_up_m##M(            \
-      const int32_t *counts, const uint16_t *x, const uint8_t *wg, const uint8_t *wu,        \
-      uint16_t *h, uint8_t *ws) {                                                            \
-    w8a16_kernel<LF_W16_WAVES, MT, 2, D, XC>(counts, x, wg, wu, wu, h, ws);           \
+    w8a16_kernel<LF_W16_WAVES, MT, 0, D, XC, BLOCK>(counts, x, w, w, w, y, ws);               \
+  }                                                                                           \
+  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_qkv##SUFFIX(              \
+      const int32_t *counts, const uint16_t *x, const uint8_t *wq, const uint8_t *wk,         \
+      const uint8_t *wv, uint16_t *y, uint8_t *ws) {                                          \
+    w8a16_kernel<LF_W16_WAVES, MT, 1, D, XC, BLOCK>(counts, x, wq, wk, wv, y, ws);            \
+  }
+#define LF_W8A16_GATE_UP_ENTRY(SUFFIX, MT, D, XC, BLOCK)                                      \
+  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_gate_up##SUFFIX(          \
+      const int32_t *counts, const uint16_t *x, const uint8_t *wg, const uint8_t *wu,         \
+      uint16_t *h, uint8_t *ws) {                                                             \
+    w8a16_kernel<LF_W16_WAVES, MT, 2, D, XC, BLOCK>(counts, x, wg, wu, wu, h, ws);            \
   }
 
-// (17..64 rows: the LDS-tiled GEMM of w8a16_gemm.hip under the _m32 and _m64
-// symbols)
-LF_W8A16_ENTRIES(1, 16, 4, 4)
-LF_W8A16_ENTRIES(8, 128, 2, 2)
-
-// The same column-group form over weights with 128 x 128 block scales.
-#define LF_W8A16_B128_ENTRIES(MT, M, D, XC)                                                     \
-  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_dense_b128_m##M(         \
-      const int32_t *counts, const uint16_t *x, const uint8_t *w, uint16_t *y, uint8_t *ws) { \
-    w8a16_kernel<LF_W16_WAVES, MT, 0, D, XC, true>(counts, x, w, w, w, y, ws);               \
-  }                                                                                          \
-  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_qkv_b128_m##M(           \
-      const int32_t *counts, const uint16_t *x, const uint8_t *wq, const uint8_t *wk,        \
-      const uint8_t *wv, uint16_t *y, uint8_t *ws) {                                         \
-    w8a16_kernel<LF_W16_WAVES, MT, 1, D, XC, true>(counts, x, wq, wk, wv, y, ws);            \
-  }                                                                                          \
-  __global__ __launch_bounds__(LF_W16_WAVES * 64) void lf_fp8_w8a16_gate_up_b128_m##M(       \
-      const int32_t *counts, const uint16_t *x, const uint8_t *wg, const uint8_t *wu,        \
-      uint16_t *h, uint8_t *ws) {                                                            \
-    w8a16_kernel<LF_W16_WAVES, MT, 2, D, XC, true>(counts, x, wg, wu, wu, h, ws);            \
-  }
-
-LF_W8A16_B128_ENTRIES(8, 128, 2, 2)
+LF_W8A16_ENTRIES(_m16, 1, 4, 4, false)
+LF_W8A16_GATE_UP_ENTRY(_m16, 1, 4, 4, false)
+LF_W8A16_ENTRIES(_cg_m32, 2, 4, 4, false)
+LF_W8A16_ENTRIES(_m128, 8, 2, 2, false)
+LF_W8A16_GATE_UP_ENTRY(_m128, 8, 2, 2, false)
+LF_W8A16_ENTRIES(_b128_cg_m16, 1, 4, 4, true)
+LF_W8A16_GATE_UP_ENTRY(_b128_cg_m16, 1, 4, 4, true)
+LF_W8A16_ENTRIES(_b128_cg_m32, 2, 4, 4, true)
+LF_W8A16_ENTRIES(_b128_m128, 8, 2, 2, true)
+LF_W8A16_GATE_UP_ENTRY(_b128_m128, 8, 2, 2, true)
 
 #ifndef LF_W16T_WAVES
 #define LF_W16T_WAVES 8

@@ -630,17 +630,19 @@ LF_W16_GEMM_DENSE_QKV(_b128_m128_n128, true, 512, 128, 128, 2, 4, 2, 4)
 LF_W16_GEMM_GATE_UP(_b128_m128_n128, true, 512, 128, 128, 2, 4, 2, 4)
 
 // Profiles of 17..64 rows (block-scaled: 1..64), any width that is a
-// multiple of 16, where no shape-specialized entry is built (w8a16.hip): 64
-// dense / QKV columns per block, 64 gate and 64 up columns for gate/up. At
+// multiple of 16, where no shape-specialized entry is built and column groups
+// are not faster (csrc/pack.cpp, w16_column_groups): 64 dense / QKV columns per
+// block, 64 gate and 64 up columns for gate/up. At
 // these row counts the kernel is bound by bytes in flight: 32 / 64 rows of
 // activations are a quarter / half of the 128-row stage, which leaves LDS
 // for weight rings of 3-8 stages (40-64 KiB of weights in flight per block).
-// They replace column-group kernels whose rolled register ring drained at
-// every k-tile. Llama-3-8B as one of two tensor-parallel ranks, M = 61, us
-// before -> now: qkv (3072 x 4096) 23.2 -> 11.1, o (4096 x 2048) 19.0 ->
-// 9.3, gate/up (7168 x 4096) 32.8 -> 18.7, down (4096 x 7168) 26.1 -> 14.8
-// (2.0 TB/s of weights); M = 24: qkv 13.2 -> 9.1, o 9.0 -> 8.1, gate/up 16.9
-// -> 15.9, down 12.8 -> 12.5.
+// Column groups (w8a16.hip), whose rolled register ring drains at every k-tile,
+// against this form: Llama-3-8B as one of two tensor-parallel ranks, M = 61, us:
+// qkv (3072 x 4096) 23.2 -> 11.1, o (4096 x 2048) 19.0 -> 9.3, gate/up (7168 x
+// 4096) 32.8 -> 18.7, down (4096 x 7168) 26.1 -> 14.8 (2.0 TB/s of weights); M =
+// 24: qkv 13.2 -> 9.1, o 9.0 -> 8.1, gate/up 16.9 -> 15.9. At 33-64 rows it is
+// behind only at K = 1024 and 24576 columns or more (49152 x 1024 at 61 rows
+// 25.8 against 24.6; K 768 and 1280 20.3 / 26.6 against 20.8 / 27.8).
 LF_W16_GEMM_DENSE_QKV(_m32, false, 256, 32, 64, 2, 2, 3, 6)
 LF_W16_GEMM_GATE_UP(_m32, false, 256, 32, 128, 1, 4, 3, 3)
 LF_W16_GEMM_DENSE_QKV(_m64, false, 512, 64, 64, 4, 2, 3, 6)

@@ -64,8 +64,9 @@ inline int64_t swizzled_offset(int64_t n, int64_t k, int64_t columns) {
 // workspace. 17..64 rows (mt 2, 4; block-scaled also mt 1) run the LDS-tiled
 // GEMM of w8a16_gemm.hip, which cuts K into w16_slices slices: exactly those
 // blocks are launched, as a block's LDS rings leave room for one or two per
-// CU and a spare block costs its start. 65..128 rows of a width that is no
-// multiple of 64 run the column-group form of w8a16.hip on about 512 blocks.
+// CU and a spare block costs its start. The column-group form of w8a16.hip, on
+// about 512 blocks (two per CU), runs 65..128 rows of a width that is no
+// multiple of 64, and smaller profiles where w16_column_groups says so.
 constexpr int kW16Waves = 4;
 constexpr int kW16TileWaves = 8;
 // kernels/w8a16_gemm.hip, w16_slices
@@ -75,25 +76,54 @@ int64_t w16_slices(int64_t blocks_n, int64_t kt) {
 }
 // Threads of the entries that fit any shape above 16 rows.
 int w16_threads(int mt, bool block) { return mt == 4 && !block ? 512 : 64 * kW16Waves; }
+// Column groups up to 32 rows (the _cg_ entries): where the launch streams many
+// bytes, their two blocks per CU keep more weights in flight than one GEMM
+// block does, as long as the 512 or so blocks are one round on the chip.
+// groups, split: theirs. Measured with weights that no cache holds, GEMM form /
+// column groups (us, at 17 and 32 rows; block-scaled at 1 and 16 rows):
+//   32768 x 512, 1024, 2048: 7.6 / 6.2 and 7.7 / 6.8, 13.5 / 9.3 and 13.4 / 9.9,
+//     17.3 / 14.9 and 16.9 / 15.5; the kW16UnsplitGroups and more
+//   8192 x 5120: 15.7 / 13.2 and 15.1 / 13.8; 10240 x 5120: 21.0 / 15.2 and
+//     19.6 / 15.8; 4096 x 11008: 19.1 / 15.2 and 17.7 / 15.8; 4096 x 7168: 13.9 /
+//     12.6 and 13.2 / 13.3; up to 24 MiB within 10 % either way
+//   GEMM ahead where column groups need a second round (560 blocks: 7168 x 5120
+//     16.4 / 18.0 and 14.7 / 16.5; 640: 20480 x 2048 15.9 / 17.9 and 15.4 / 18.0)
+//     or are narrow (2048 x 11008 14.7 / 15.2 and 13.5 / 15.5), and for gate/up
+//     (8192 x 5120 22.9 / 23.2 and 22.5 / 22.7)
+//   block-scaled, 16 rows: 4096 x 5120 11.1 / 10.0 and 10.7 / 10.5; 6144 x 3072
+//     9.6 / 8.7 and 9.8 / 9.2; 8192 x 7168 19.2 / 15.2 and 18.1 / 15.1; 7168 x
+//     5120 (560 blocks) 14.1 / 13.0 and 13.4 / 13.1; 2048 x 5120 9.7 / 10.5 and
+//     9.2 / 11.4; gate/up 18944 x 3072 28.9 / 25.6 and 29.9 / 26.8, 8192 x 5120
+//     21.5 / 20.4 and 20.2 / 20.1, 11008 x 5120 24.3 / 26.6 and 23.8 / 28.4
+constexpr int64_t kW16UnsplitGroups = 342;  // 512 / groups rounds to 1
+bool w16_column_groups(int mt, bool block, bool gate_up, int64_t n, int64_t k, int64_t groups, int64_t split) {
+  constexpr int64_t kMiB = 1 << 20;
+  if (mt == 1) return block && (gate_up ? n > 16384 : n >= 4096 && n * k >= 12 * kMiB);
+  if (mt != 2 || gate_up) return false;
+  return groups >= kW16UnsplitGroups || (n >= 4096 && n * k > 24 * kMiB && groups * split <= 512);
+}
 struct W8a16Split {
   int mt;
-  bool one_tile;
+  bool one_tile, column_groups;
   int64_t groups, split;
 };
-bool w8a16_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
+bool w8a16_split(int64_t n, int64_t k, int32_t max_tokens, bool gate_up, bool block, W8a16Split *out) {
   if (n % 16 != 0 || max_tokens > 128) return false;
   const int mt = max_tokens <= 16 ? 1 : max_tokens <= 32 ? 2 : max_tokens <= 64 ? 4 : 8;
   const int64_t kt = k / 128, tiles = n / 16;
   out->mt = mt;
-  out->one_tile = mt == 1;
+  out->one_tile = mt == 1 && !block;
+  out->column_groups = false;
   if (out->one_tile) {
     out->groups = tiles;
     out->split = 1;
     return tiles <= INT32_MAX;
   }
   const int64_t groups = (tiles + kW16Waves - 1) / kW16Waves;
-  const int64_t split = mt == 8 ? std::min(kt, std::max<int64_t>(1, (512 + groups / 2) / groups))
-                                : w16_slices(groups, kt);
+  // (a slice's block scales are staged in LDS: at most 128 k-tiles)
+  const int64_t cg_split = std::max<int64_t>(block ? (kt + 127) / 128 : 1, std::min(kt, (512 + groups / 2) / groups));
+  out->column_groups = mt == 8 || w16_column_groups(mt, block, gate_up, n, k, groups, cg_split);
+  const int64_t split = out->column_groups ? cg_split : w16_slices(groups, kt);
   if (groups * split > INT32_MAX) return false;
   out->groups = groups;
   out->split = split;
@@ -105,9 +135,8 @@ bool w8a16_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
 // (w8a16_gemm below, the _b128_m128_n{BN} symbols; every block-scaled width
 // is a multiple of 128, so a 16-column fragment lies in one 128-row scale
 // block), except vocabulary-wide dense shapes, which keep the column-group
-// form (its block scales of a slice are staged in LDS: at most 128 k-tiles);
-// every other profile (also <= 16 rows) the GEMM form's _b128_m16 / _m32 /
-// _m64 entries, the grid as above.
+// form; every other profile (also <= 16 rows) the forms above (w8a16_split),
+// _b128_m16 / _m32 / _m64 or _b128_cg_m16 / _m32.
 bool w8a16_b128_entry(int32_t e) {
   return e == LF_FP8_ENTRY_W8A16_DENSE_B128 || e == LF_FP8_ENTRY_W8A16_QKV_B128 ||
          e == LF_FP8_ENTRY_W8A16_GATE_UP_B128;
@@ -118,16 +147,9 @@ int32_t w8a16_channel_entry(int32_t e) {
          : e == LF_FP8_ENTRY_W8A16_QKV_B128 ? LF_FP8_ENTRY_W8A16_QKV
                                              : LF_FP8_ENTRY_W8A16_GATE_UP;
 }
-bool w8a16_b128_split(int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
-  if (n % 128 != 0 || k % 128 != 0 || !w8a16_split(n, k, max_tokens, out)) return false;
-  const int64_t kt = k / 128, tiles = n / 16;
-  if (out->one_tile) {  // <= 16 rows: the GEMM form too
-    out->one_tile = false;
-    out->groups = (tiles + kW16Waves - 1) / kW16Waves;
-    out->split = w16_slices(out->groups, kt);
-  }
-  if (out->mt == 8) out->split = std::max<int64_t>(out->split, (kt + 127) / 128);
-  return out->groups * out->split <= INT32_MAX;
+bool w8a16_b128_split(int32_t entry, int64_t n, int64_t k, int32_t max_tokens, W8a16Split *out) {
+  return n % 128 == 0 && k % 128 == 0 &&
+         w8a16_split(n, k, max_tokens, entry == LF_FP8_ENTRY_W8A16_GATE_UP_B128, true, out);
 }
 
 // Shape-specialized W8A16 entries (w8a16.hip, "LF_W16_FIXED_*"): compiled for
@@ -657,7 +679,7 @@ static int64_t w8a16_workspace(int32_t entry, int64_t n, int64_t k, int64_t nq, 
   if (w8a16_b128_entry(entry)) {
     W8a16Split sp;
     if (n <= 0 || k <= 0 || max_tokens <= 0 || n > kMaxDim || k > kMaxDim ||
-        !w8a16_b128_split(n, k, max_tokens, &sp)) {
+        !w8a16_b128_split(entry, n, k, max_tokens, &sp)) {
       return -1;
     }
     W8a16Gemm gm;
@@ -677,7 +699,7 @@ static int64_t w8a16_workspace(int32_t entry, int64_t n, int64_t k, int64_t nq, 
   }
   W8a16Split sp;
   if (n <= 0 || k <= 0 || k % 128 != 0 || max_tokens <= 0 || n > kMaxDim || k > kMaxDim ||
-      !w8a16_split(n, k, max_tokens, &sp)) {
+      !w8a16_split(n, k, max_tokens, entry == LF_FP8_ENTRY_W8A16_GATE_UP, false, &sp)) {
     return -1;
   }
   W8a16Gemm gm;
@@ -687,9 +709,9 @@ static int64_t w8a16_workspace(int32_t entry, int64_t n, int64_t k, int64_t nq, 
   }
   // One 1 KiB fp32 accumulator fragment per (slice, 16-column tile, weight,
   // 16-row tile), then one arrival counter per column group. The GEMM form
-  // (mt 2, 4) stores whole blocks of tiles.
+  // stores whole blocks of tiles.
   const int64_t nw = entry == LF_FP8_ENTRY_W8A16_GATE_UP ? 2 : 1;
-  const int64_t tiles = sp.mt == 8 ? n / 16 : sp.groups * kW16Waves;
+  const int64_t tiles = sp.column_groups ? n / 16 : sp.groups * kW16Waves;
   const int64_t need = sp.split == 1 ? 256
                                      : align_up(sp.split * tiles * nw * sp.mt * 1024, 256) +
                                            align_up(sp.groups * 4, 256);
@@ -917,7 +939,7 @@ static int32_t launch_geometry(int32_t entry, int64_t n, int64_t k, int64_t nq, 
     case LF_FP8_ENTRY_W8A16_QKV:
     case LF_FP8_ENTRY_W8A16_GATE_UP: {
       W8a16Split sp;
-      if (!w8a16_split(n, k, max_tokens, &sp)) return LF_INVALID_ARGUMENT;
+      if (!w8a16_split(n, k, max_tokens, entry == LF_FP8_ENTRY_W8A16_GATE_UP, false, &sp)) return LF_INVALID_ARGUMENT;
       const char *op = entry == LF_FP8_ENTRY_W8A16_DENSE ? "dense"
                        : entry == LF_FP8_ENTRY_W8A16_QKV ? "qkv"
                                                          : "gate_up";
@@ -934,8 +956,8 @@ static int32_t launch_geometry(int32_t entry, int64_t n, int64_t k, int64_t nq, 
         w8a16_fixed_geometry(*f, n, &gx, &bx);
         break;
       }
-      std::snprintf(buffer, sizeof(buffer), "lf_fp8_w8a16_%s_m%d%s", op, 16 * sp.mt,
-                    sp.one_tile ? "_t1" : "");
+      std::snprintf(buffer, sizeof(buffer), "lf_fp8_w8a16_%s%s_m%d%s", op,
+                    sp.column_groups && sp.mt != 8 ? "_cg" : "", 16 * sp.mt, sp.one_tile ? "_t1" : "");
       name = buffer;
       gx = static_cast<int32_t>(sp.groups * sp.split);
       bx = sp.one_tile ? 64 * kW16TileWaves : w16_threads(sp.mt, false);
@@ -945,7 +967,7 @@ static int32_t launch_geometry(int32_t entry, int64_t n, int64_t k, int64_t nq, 
     case LF_FP8_ENTRY_W8A16_QKV_B128:
     case LF_FP8_ENTRY_W8A16_GATE_UP_B128: {
       W8a16Split sp;
-      if (!w8a16_b128_split(n, k, max_tokens, &sp)) return LF_INVALID_ARGUMENT;
+      if (!w8a16_b128_split(entry, n, k, max_tokens, &sp)) return LF_INVALID_ARGUMENT;
       const char *op = entry == LF_FP8_ENTRY_W8A16_DENSE_B128 ? "dense"
                        : entry == LF_FP8_ENTRY_W8A16_QKV_B128 ? "qkv"
                                                               : "gate_up";
@@ -962,7 +984,8 @@ static int32_t launch_geometry(int32_t entry, int64_t n, int64_t k, int64_t nq, 
         w8a16_fixed_geometry(*f, n, &gx, &bx);
         break;
       }
-      std::snprintf(buffer, sizeof(buffer), "lf_fp8_w8a16_%s_b128_m%d", op, 16 * sp.mt);
+      std::snprintf(buffer, sizeof(buffer), "lf_fp8_w8a16_%s_b128%s_m%d", op,
+                    sp.column_groups && sp.mt != 8 ? "_cg" : "", 16 * sp.mt);
       name = buffer;
       gx = static_cast<int32_t>(sp.groups * sp.split);
       bx = w16_threads(sp.mt, true);

@@ -249,7 +249,7 @@ def test_w8a16_any_shape_grid_holds_the_kernels_slices(entry, cols, k):
     for n in (16, 48, 64, 1040, 4096, 7184, 16384, 40000):
         for m in (17, 32, 33, 64):
             dims, sym = fp8.launch_geometry(entry, n, k, m)
-            if not sym.endswith(f"_m{m if m in (32, 64) else 32 if m == 17 else 64}") or "_k" in sym:
+            if not sym.endswith(f"_m{m if m in (32, 64) else 32 if m == 17 else 64}") or "_k" in sym or "_cg_" in sym:
                 continue
             rows, blocks = (32 if m <= 32 else 64), -(-n // 64)
             slices = max(1, min(256 // blocks, k // 128 // (4 if blocks <= 32 and k <= 2048 else 8)))
@@ -258,6 +258,37 @@ def test_w8a16_any_shape_grid_holds_the_kernels_slices(entry, cols, k):
             if slices > 1:
                 need = slices * blocks * 64 * cols * rows * 4
                 assert fp8.w8a16_workspace_bytes(entry, n, k, m) >= need + blocks * 4
+
+
+def test_w8a16_column_group_rule():
+    """Column groups up to 32 rows: dense and QKV above 24 MiB of weights and
+    from 4096 columns on (block-scaled up to 16 rows: 12 MiB) as long as they are
+    one round of 512 blocks, or where they are unsplit (342 groups of 64
+    columns and more); gate/up only block-scaled above 16384 columns. Whole
+    slices of whole groups, slices of at most 128 k-tiles with block scales,
+    and their partials in the workspace."""
+    D, Q, G = _abi.ENTRY_W8A16_DENSE, _abi.ENTRY_W8A16_QKV, _abi.ENTRY_W8A16_GATE_UP
+    DB, QB, GB = (fp8._BLOCK_ENTRIES[("w8a16", op)] for op in ("dense", "qkv", "gate_up"))
+    cg = lambda e, n, k, m: "_cg_" in fp8.launch_geometry(e, n, k, m)[1]
+    for e in (D, Q, DB, QB):
+        assert cg(e, 4096, 6272, 17) and cg(e, 4096, 6272, 32) and not cg(e, 4096, 6144, 32)
+        assert not cg(e, 2048, 16384, 32)                     # narrow
+        assert not cg(e, 7168, 8192, 32)                      # 560 blocks
+        assert cg(e, 21888, 128, 32) and not cg(e, 21760, 128, 32)  # 342 groups unsplit, 340 in two slices
+        assert not cg(e, 8192, 8192, 33) and not cg(e, 8192, 8192, 64)
+    for e in (DB, QB):
+        assert cg(e, 4096, 3072, 1) and cg(e, 4096, 3072, 16) and not cg(e, 4096, 2944, 16)
+        assert not cg(e, 3968, 8192, 16)
+    assert not cg(G, 32768, 8192, 32) and not cg(GB, 32768, 8192, 32)
+    assert cg(GB, 16512, 512, 16) and not cg(GB, 16384, 8192, 16)
+    for e, n, k, m, cols in ((D, 4096, 6272, 32, 1), (DB, 4096, 3072, 16, 1), (DB, 8192, 32768, 16, 1),
+                             (GB, 16512, 2048, 16, 2), (QB, 21888, 32768, 32, 1)):
+        dims, sym = fp8.launch_geometry(e, n, k, m)
+        groups, kt = n // 64, k // 128
+        slices = max(1, min(kt, (512 + groups // 2) // groups), -(-kt // 128) if "b128" in sym else 1)
+        assert dims.grid == (groups * slices, 1, 1) and dims.block == (256, 1, 1)
+        need = slices * (n // 16) * cols * (1 if m == 16 else 2) * 1024
+        assert fp8.w8a16_workspace_bytes(e, n, k, m) >= (need + groups * 4 if slices > 1 else 256)
 
 
 @pytest.mark.parametrize("entry", [_abi.ENTRY_W8A16_QKV, _abi.ENTRY_W8A16_QKV_B128])

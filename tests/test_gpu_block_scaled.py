@@ -165,6 +165,55 @@ def test_block_scaled_w8a16(rt, op, m, max_tokens):
     check_op(op, "w8a16", y, x, ws, rows, cols, f"b128 w8a16 {op} m={m}/{max_tokens}")
 
 
+@pytest.mark.parametrize("op,n,k,m,max_tokens,symbol", [
+    ("dense", 4096, 3072, 1, 16, "dense_b128_cg_m16"),        # 64 groups, eight slices of three k-tiles
+    ("dense", 24576, 512, 16, 16, "dense_b128_cg_m16"),       # unsplit
+    ("qkv", 4352, 3072, 9, 16, "qkv_b128_cg_m16"),            # 4096 + 128 + 128, 68 groups
+    ("gate_up", 16512, 256, 13, 16, "gate_up_b128_cg_m16"),   # 258 groups, two slices of a k-tile
+    ("dense", 4096, 6272, 17, 32, "dense_b128_cg_m32"),
+    ("qkv", 21888, 128, 31, 32, "qkv_b128_cg_m32"),           # 342 groups, one k-tile
+    ("dense", 4096, 6272, 32, 32, "dense_cg_m32"),            # per-channel scales
+    ("qkv", 21904, 384, 29, 32, "qkv_cg_m32"),                # 343 groups, the last of one tile
+])
+def test_w8a16_column_groups_any_shape(rt, op, n, k, m, max_tokens, symbol):
+    """The column-group entries that fit any shape, as the geometry picks them
+    up to 32 rows: against the oracle over a column sample with the last
+    columns; rows past M untouched; three launches on one workspace agree bit
+    for bit."""
+    from lunaflux_amd import fp8
+    rng = np.random.default_rng(12500 + n + k + m)
+    block = "_b128_" in symbol
+    x = synth.activations(rng, m, k)
+    xa = rt.context.upload(np.concatenate([x, np.zeros((max_tokens - m, k), np.uint16)]))
+    ya = rt.context.allocate(max_tokens * n * 2)
+    sizes = [n, n] if op == "gate_up" else [n - 256, 128, 128] if op == "qkv" else [n]
+    ws = [spread_weight(rng, r, k) if block else synth.weight(rng, r, k) for r in sizes]
+    up = [rt.upload_weight(q, s, fp8.BLOCK128 if block else fp8.PER_CHANNEL) for q, s in ws]
+    bound = {"dense": rt.bind_dense, "qkv": rt.bind_qkv, "gate_up": rt.bind_gate_up}[op](
+        "w8a16", rt.step_counts(m), _region(xa, alignment=256), *up, _region(ya, alignment=256), max_tokens)
+    assert [s.name for s in bound.steps] == ["lf_fp8_w8a16_" + symbol]
+    ya.copy_from_host(np.full(max_tokens * n, SENTINEL, np.uint16))
+    outs = []
+    for _ in range(3):
+        bound.launch(rt.stream, synchronous=True)
+        outs.append(ya.read(np.uint16, (max_tokens, n)))
+    assert all(np.array_equal(outs[0], y) for y in outs[1:]) and np.all(outs[0][m:] == SENTINEL)
+    cols = np.unique(np.concatenate([[0, n - 300, n - 257, n - 256, n - 129, n - 128, n - 1], rng.choice(n, 250)]))
+    rows_of = deq_rows if block else lambda q, s, c: o.dequantize(q[c], s[c])
+    bk = bound_k(k) if block else k
+    xr = x_ref(x, "w8a16")
+    label = f"{symbol} n={n} k={k} m={m}"
+    if op == "gate_up":
+        wg, wu = (rows_of(q, s, cols) for q, s in ws)
+        g, u = o.dense_projection(xr, wg), o.dense_projection(xr, wu)
+        parity(outs[0][:m][:, cols], o.silu_mul_array(g, u), label=label,
+               midpoint_tol=swiglu_midpoint_tol(g, u, abs_sum(xr, wg), abs_sum(xr, wu), bk))
+        return
+    wr = np.concatenate([rows_of(q, s, cols[(cols >= a) & (cols < a + len(q))] - a)
+                         for (q, s), a in zip(ws, np.cumsum([0] + sizes[:-1]))])
+    parity(outs[0][:m][:, cols], o.dense_projection(xr, wr), k=bk, s_abs=abs_sum(xr, wr), label=label)
+
+
 def w8a8_quantized_rows(bound, m, k, max_tokens):
     """(codes [m, K], scales [m, K / 128]) from the one-launch workspace:
     sync area (256 + 128 bands bytes), codes [cap, K], scales [K / 128][cap],
