@@ -169,10 +169,12 @@ struct W8a16Fixed {
   int64_t min_n = 0;  // chosen only for N >= min_n (earlier rows win)
 };
 constexpr int64_t kWideN = 16384;
-// Unsplit gate/up at 32 rows: 64 columns per block, so below 12288 columns
-// (192 blocks) too few blocks for 256 CUs, where the GEMM form's K split is
-// faster (M = 24, us: 7168 columns 16.9 -> 15.9, 3584 15.6 -> 12.1).
-constexpr int64_t kFullN32 = 12288;
+// Unsplit gate/up at 32 rows: 64 columns per block, so with few columns too few
+// blocks for 256 CUs, where the GEMM form's K split is faster. M = 32, us, this
+// entry / the GEMM form: 3584 columns 15.6 / 11.4, 6144 16.4 / 16.6, 7168 16.8 /
+// 17.9 with weights that no cache holds and 16.6 / 16.1 with weights left in the
+// MALL, 8192 16.9 / 19.6 and 16.8 / 17.4, 10240 17.6 / 21.4, 11264 18.4 / 22.0.
+constexpr int64_t kFullN32 = 8192;
 constexpr W8a16Fixed kW8a16Fixed[] = {
     {LF_FP8_ENTRY_W8A16_DENSE, 4096, 0, 0, 1, true, 2, 1, "lf_fp8_w8a16_dense_wide_k4096_m16", kWideN},
     {LF_FP8_ENTRY_W8A16_DENSE, 4096, 0, 0, 2, true, 4, 1, "lf_fp8_w8a16_dense_wide_k4096_m32", kWideN},

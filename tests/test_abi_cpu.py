@@ -143,6 +143,11 @@ def test_launch_geometry():
     dims, sym = fp8.launch_geometry(_abi.ENTRY_W8A16_GATE_UP, 14336, 4096, 16)
     assert sym == "lf_fp8_w8a16_gate_up_k4096_m16" and dims.grid == (448, 1, 1)
     assert dims.block == (128, 1, 1)
+    # (at 32 rows from 8192 columns on; fewer: the GEMM form, which splits K)
+    for e, tail in ((_abi.ENTRY_W8A16_GATE_UP, ""), (_abi.ENTRY_W8A16_GATE_UP_B128, "_b128")):
+        for n, name, grid in ((8192, "k4096_m32", 128), (10240, "k4096_m32", 160), (7168, "m32", 112 * 2)):
+            dims, sym = fp8.launch_geometry(e, n, 4096, 32)
+            assert sym == f"lf_fp8_w8a16_gate_up{tail}_{name}" and dims.grid == (grid, 1, 1), (n, sym, dims)
     # QKV at 32 rows: 8 tiles per block over 4 K-slices (48 groups x 4)
     dims, sym = fp8.launch_geometry(_abi.ENTRY_W8A16_QKV, 6144, 4096, 32, qkv_split=(4096, 1024))
     assert sym == "lf_fp8_w8a16_qkv_k4096_q4096_kv1024_m32" and dims.grid == (192, 1, 1)
