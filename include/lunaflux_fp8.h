@@ -489,13 +489,15 @@ int32_t lunaflux_fp8_moe_launch_geometry(int32_t entry,
  *  lf_moe_route_sort_q (counts, desc, logits, x, ws) in place of
  * lf_moe_route_sort, larger block-scaled ones
  *  lf_moe_route_q (counts, desc, logits, x, ws)
- * in place of lf_moe_route and lf_moe_quant_tokens, and block-scaled ones with K <= 3072 in both GEMMs and a
- * hidden width that is a multiple of 256
+ * in place of lf_moe_route and lf_moe_quant_tokens, and block-scaled ones with
+ * K <= 3072 in both GEMMs and a hidden width that is a multiple of 256
  *  lf_moe_gate_up_t128x256_b128_q (counts, desc, wg, wu, ws)
  *  lf_moe_down_t128x256_b128      (counts, desc, wd, ws)
  * (128 x 256 tiles; the gate/up epilogue quantizes h, so there is no hidden
- * quantizer launch). Every other step is the geometry's above; the steps of
- * one operation all come from one of the two functions. */
+ * quantizer launch), except the smallest and largest profiles, where the
+ * grouped GEMV and the 256 x 256 tiles are faster. Every other step is the
+ * geometry's above; the steps of one operation all come from one of the two
+ * functions. */
 int32_t lunaflux_fp8_moe_step_geometry(int32_t entry,
                                        const lf_fp8_moe_desc *desc,
                                        int32_t max_tokens, int32_t dims[7],

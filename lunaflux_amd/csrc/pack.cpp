@@ -1176,18 +1176,46 @@ int64_t lunaflux_fp8_moe_sync_offset(const lf_fp8_moe_desc *d, int32_t max_token
 
 // Block-scaled profiles: 128 x 256 tiles (kernels/moe.hip,
 // grouped_gemm_t128x256), where both K fit its scale table and its 32-bit
-// activation offsets. Against the forms moe_geometry gives
-// below, 64 experts of 2048 x 1408, top 6, us: whole operation on the GEMV
-// form 4 tokens 49.0 -> 47.6, 12 tokens 63.9 -> 58.3, 32 tokens 93.1 -> 91.8
-// (no hidden quantizer launch); gate/up + down 60 tokens 153 -> 82, 250 tokens
-// 211 -> 114, 900 tokens 323 -> 154, 1500 tokens 432 -> 192 (all 128 x 128
-// tiles before), 4096 tokens 369 -> 355 (256 x 256). Per-channel profiles stay
-// on their forms: 8 experts of 4096 x 14336, top 2, gate/up + down 60 tokens
-// 271 -> 264, 250 tokens 297 -> 289, but 1024 tokens 497 -> 513 us.
+// activation offsets, except where an older form is the faster one. Whole
+// operation, us, older form -> this one, routing launches the same:
+//  128 x 128 tiles (more than 32 tokens, under 256 rows per expert): 64 experts
+//    of 2048 x 1408, top 6, 48 / 256 / 1024 / 2048 tokens 244 / 249 / 284 / 490 ->
+//    125 / 134 / 162 / 247; 8 experts of 3072 x 3072, top 2, 64 / 512 tokens 126 /
+//    358 -> 58 / 93
+//  256 x 256 tiles: the same 64 experts at 3072 / 4096 / 8192 / 12288 / 16384
+//    tokens (288 / 384 / 768 / 1152 / 1536 rows per expert) 376 / 419 / 723 / 993 /
+//    1324 -> 330 / 405 / 734 / 1068 / 1392; 128 experts of 2048 x 768, top 8, 16384
+//    / 24576 tokens 1158 / 1668 -> 1228 / 1799; 8 experts of 3072 x 3072, 3072 /
+//    16384 tokens 292 / 1218 -> 276 / 1286. From 1024 rows per expert on half a
+//    tile of padding is small and 256-row tiles stream the weights half as often;
+//    under 16384 rows in all they leave CUs idle (4 experts of 512 x 512, 4096
+//    tokens 55.4 -> 50.6).
+//  the GEMV form (up to 32 tokens), uniform / skewed routing: the 64 experts at 1 /
+//    4 / 12 / 24 tokens 31.4 / 47.7 / 87.7 / 119.0 and 30.9 / 42.1 / 50.0 / 62.5 ->
+//    32.4 / 44.6 / 91.2 / 117.8 and 31.8 / 37.2 / 44.3 / 50.6; 8 experts of 3072 x
+//    3072, 1 / 2 / 4 / 16 tokens 33.6 / 39.3 / 51.5 / 56.3 -> 38.3 / 41.6 / 48.6 /
+//    52.2; 8 of 2048 x 1408, 1 / 4 / 16 / 24 tokens 26.9 / 35.2 / 38.2 / 39.6 and
+//    27.0 / 34.1 / 38.1 / 48.9 -> 29.0 / 39.1 / 40.6 / 41.4 and 29.1 / 38.5 / 39.5 /
+//    42.0; 4 of 2816 x 1408, 1 / 8 / 16 tokens 30.0 / 38.0 / 39.5 -> 32.1 / 42.5 /
+//    43.0. Where the down GEMM has a tile for at most 64 CUs and the k-tiles are
+//    many, the GEMV form's narrower strips fill more of the chip, and up to 16
+//    tokens it reads every weight once whatever the routing (16 rows at a time);
+//    with few k-tiles the launch it needs for the hidden quantizer costs more (8
+//    experts of 768 x 768, 1 / 16 tokens 23.2 / 27.0 -> 23.7 / 25.3).
+// Per-channel profiles stay on their forms: 8 experts of 4096 x 14336, top 2,
+// gate/up + down 60 tokens 271 -> 264, 250 tokens 297 -> 289, but 1024 tokens 497
+// -> 513 us.
 static bool moe_t128x256(const lf_fp8_moe_desc *d, int64_t T) {
   constexpr int64_t kMaxK = 128 * 24;  // kT128x256MaxKT
-  return d->group == 128 && d->hidden % 256 == 0 && d->hidden <= kMaxK && d->inter <= kMaxK &&
-         T * d->top_k * std::max<int64_t>(d->hidden, d->inter) < (int64_t(1) << 32);
+  const int64_t A = T * d->top_k;
+  if (d->group != 128 || d->hidden % 256 != 0 || d->hidden > kMaxK || d->inter > kMaxK ||
+      A * std::max<int64_t>(d->hidden, d->inter) >= (int64_t(1) << 32)) {
+    return false;
+  }
+  const bool gemv = T <= 16 && std::min<int64_t>(d->experts, A) * (d->hidden / 256) <= 64 &&
+                    d->hidden + d->inter >= 3072;
+  const bool t256 = A >= 16384 && A >= 1024 * static_cast<int64_t>(d->experts);
+  return !gemv && !t256;
 }
 
 // step: the forms lunaflux_fp8_moe_step_geometry gives.

@@ -665,13 +665,17 @@ def test_moe_step_geometry_forms(group, hidden, inter):
     routing launches above 32 tokens, the token quantizer on blocks of its own
     up to there with block scales, 128 x 256 tiles (and no hidden quantizer)
     for block scales where both K are at most 24 k-tiles and the hidden width
-    is a multiple of 256; every other step the same, and what one refuses the
-    other does too."""
+    is a multiple of 256, but neither up to 16 tokens where the down GEMM has
+    at most 64 tiles of at least 24 k-tiles in all nor from 1024 rows per
+    expert and 16384 rows on; every other step the same, and what one refuses
+    the other does too."""
     from lunaflux_amd import moe
     desc = moe.moe_descriptor(16, 4, 1, hidden, inter, group)
-    for t in (1, 32, 33, 100, 256, 257, 1024, 5000, 1 << 20):
+    for t in (1, 2, 16, 17, 32, 33, 100, 256, 257, 1024, 4095, 4096, 5000, 1 << 20):
         wide = group == 128 and hidden % 256 == 0 and max(hidden, inter) <= 3072 and (
             t * 4 * max(hidden, inter) < 1 << 32)
+        wide = wide and not (t <= 16 and min(16, 4 * t) * hidden // 256 <= 64 and hidden + inter >= 3072)
+        wide = wide and t < 4096                              # 1024 rows per expert
         tiles = t * 4 // 128 + 16
         for entry in range(1, 9):
             old, new = moe.launch_geometry(entry, desc, t), moe.step_geometry(entry, desc, t)
