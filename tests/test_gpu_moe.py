@@ -30,6 +30,29 @@ def rt():
     return ProjectionRuntime(0)
 
 
+@pytest.fixture
+def bound(monkeypatch):
+    """The operations moe_expert_mlp binds in a test, in order."""
+    from lunaflux_amd import moe
+    ops, bind = [], moe.bind_moe
+
+    def recording(*args, **kwargs):
+        ops.append(bind(*args, **kwargs))
+        return ops[-1]
+    monkeypatch.setattr(moe, "bind_moe", recording)
+    return ops
+
+
+def bind_recorded_steps(monkeypatch):
+    """Bindings take the steps recorded plans name (launch_geometry)."""
+    from lunaflux_amd import moe
+    monkeypatch.setattr(moe, "step_geometry", moe.launch_geometry)
+
+
+def step_names(op):
+    return [s.name[len("lf_moe_"):] for s in op.steps]
+
+
 def expert_weights(rng, experts, rows, cols, block):
     qs, ss = [], []
     for _ in range(experts):
@@ -175,19 +198,38 @@ def test_moe_block128(rt, t, e, k, mode, max_tokens):
     check_output(x, weights, ex, w, out, True, f"moe block128 t={t} e={e} k={k}", st)
 
 
+@pytest.mark.parametrize("t,e,k,hidden,inter", [
+    (100, 8, 2, 384, 256),      # hidden not a multiple of 256
+    (60, 5, 3, 640, 128),
+    (40, 4, 1, 3328, 128),      # more k-tiles than the 128 x 256 form's scale table
+    (300, 3, 2, 256, 3200),
+])
+def test_moe_block128_square_tiles(rt, bound, t, e, k, hidden, inter):
+    """Block-scaled shapes that neither the 128 x 256 nor the 256 x 256 tiles
+    take: 128 x 128 tiles and the per-group hidden quantizer's own launch."""
+    rng = np.random.default_rng(820 + t + e)
+    x, logits, weights, out, st = run_case(rt, rng, t, e, k, hidden, inter, 1, block=True)
+    assert step_names(bound[0]) == ["route_q", "sort_count", "sort", "gate_up_b128", "quant_hidden", "down_b128",
+                                    "combine"]
+    ex, w = check_routing(logits, k, 1, st)
+    check_output(x, weights, ex, w, out, True, f"moe square tiles t={t} {hidden}x{inter}", st, wide_h=hidden > 3072)
+
+
 @pytest.mark.parametrize("t,e,k,hidden,inter,block,one_expert", [
     (32, 64, 6, 640, 1408, True, False), (32, 64, 6, 640, 1408, True, True),
     (17, 8, 2, 256, 384, False, False), (32, 8, 2, 384, 256, False, True),
     (3, 16, 4, 256, 640, True, False), (1, 4, 1, 256, 256, False, False),
+    (16, 8, 2, 256, 2816, True, True),
 ])
-def test_moe_gemv(rt, t, e, k, hidden, inter, block, one_expert):
+def test_moe_gemv(rt, bound, monkeypatch, t, e, k, hidden, inter, block, one_expert):
     """Profiles of at most 32 tokens run the grouped GEMV entries (either
-    scale mode): ragged expert loads, K of 2, 3, 5 and 11 k-tiles (not
+    scale mode): ragged expert loads, K of 2, 3, 5, 11 and 22 k-tiles (not
     multiples of the load ring), and every token on one expert (32 rows:
-    both 16-row fragments)."""
-    from lunaflux_amd import moe
-    d = moe.moe_descriptor(e, k, 1 if block else 0, hidden, inter, 128 if block else 0)
-    assert moe.launch_geometry(4, d, 32)[1] == "lf_moe_gate_up_gemv"
+    both 16-row fragments). A width the 128 x 256 tiles would take (256)
+    runs them as recorded plans name them, but for the last case, which the
+    binding's rule gives to the GEMV form."""
+    if hidden == 256 and block and inter < 2816:
+        bind_recorded_steps(monkeypatch)
     rng = np.random.default_rng(950 + t + e + hidden)
     logits = None
     if one_expert:
@@ -195,7 +237,8 @@ def test_moe_gemv(rt, t, e, k, hidden, inter, block, one_expert):
         logits[:, 3] = 10.0
     mode = 1 if block else 0
     x, logits, weights, out, st = run_case(rt, rng, t, e, k, hidden, inter, mode, block=block,
-                                           logits=logits, max_tokens=32)
+                                           logits=logits, max_tokens=16 if inter == 2816 else 32)
+    assert step_names(bound[0])[1:] == ["gate_up_gemv", "quant_hidden", "down_gemv", "combine"]
     ex, w = check_routing(logits, k, mode, st)
     if one_expert:
         assert (ex[:, 0] == 3).all()
@@ -258,56 +301,56 @@ def test_moe_zero_tokens(rt):
     (1024, 8, 2, 512, 384, 1.5, False), (700, 4, 2, 256, 256, 0.0, False),
     (1100, 8, 2, 256, 640, 3.0, False), (1024, 8, 2, 512, 384, 1.5, True),
     (700, 4, 2, 256, 256, 0.0, True), (1100, 8, 2, 256, 640, 3.0, True),
-    (1500, 16, 4, 768, 384, 1.0, "zero_groups"),
+    (1500, 16, 4, 768, 384, 1.0, "zero_groups"), (4200, 16, 4, 256, 128, 1.0, True),
 ])
-def test_moe_t256(rt, t, e, k, hidden, inter, skew, block):
+def test_moe_t256(rt, bound, monkeypatch, t, e, k, hidden, inter, skew, block):
     """Profiles averaging >= 256 routed rows per expert run the grouped GEMMs
     on 256 x 256 tiles: experts with several 256-row tiles, a partial last
     tile, skewed load (bias N(0, skew)) and, for the larger skew, experts left
     with few or no rows; per-channel and 128 x 128 block scales (rescaled
     accumulators), the latter also with all-zero activation groups and
-    weight blocks (zero scales carried over)."""
-    from lunaflux_amd import _abi, moe
+    weight blocks (zero scales carried over). Block-scaled profiles under
+    16384 rows run them as recorded plans name them."""
     zero = block == "zero_groups"
     block = bool(block)
     mode = 1 if block else 0
-    desc = moe.moe_descriptor(e, k, mode, hidden, inter, 128 if block else 0)
-    suffix = "_b128" if block else ""
-    # no hidden-quantizer launch: block scales, the gate/up epilogue quantizes
-    # h; per-token scales, the down launch does as its first counted step.
-    # check_output compares the codes and scales bit for bit with the
-    # quantizer applied to the device's bf16 h
-    assert moe.launch_geometry(_abi.MOE_GATE_UP, desc, t)[1] == "lf_moe_gate_up_t256" + suffix + ("_q" if block else "")
-    assert moe.launch_geometry(_abi.MOE_QUANT_HIDDEN, desc, t)[1] == ""
-    assert moe.launch_geometry(_abi.MOE_DOWN, desc, t)[1] == "lf_moe_down_t256" + ("_b128" if block else "_aq")
+    if block and t * k < 16384:
+        bind_recorded_steps(monkeypatch)
     rng = np.random.default_rng(950 + t + e + block)
     logits = (rng.standard_normal((t, e)) + rng.normal(0, skew, e)).astype(np.float32)
     x, logits, weights, out, st = run_case(rt, rng, t, e, k, hidden, inter, mode, block=block,
                                            logits=logits, zero_groups=zero)
+    # no hidden-quantizer launch: block scales, the gate/up epilogue quantizes
+    # h; per-token scales, the down launch does as its first counted step.
+    # check_output compares the codes and scales bit for bit with the
+    # quantizer applied to the device's bf16 h
+    assert step_names(bound[0])[-3:] == (["gate_up_t256_b128_q", "down_t256_b128", "combine"] if block else
+                                         ["gate_up_t256", "down_t256_aq", "combine"])
     ex, w = check_routing(logits, k, mode, st)
     check_output(x, weights, ex, w, out, block, f"moe t256 t={t} e={e} skew={skew} block={block}", st)
 
 
 @pytest.mark.parametrize("block", [False, True])
-def test_moe_t256_row_boundaries(rt, block):
+def test_moe_t256_row_boundaries(rt, bound, monkeypatch, block):
     """256-row tiles whose live rows end exactly at or just past the 32-row
     boundaries of the loading waves (a wave loads the A rows of one 32-row
     fragment and skips its loads when all of them are past the tile's last
     row): experts routed 288 (a 32-row last tile), 33, 64, 65, 31, 1, 352
-    and 1214 rows, top-1 over one-hot logits, both scale modes."""
-    from lunaflux_amd import _abi, moe
+    and 1214 rows, top-1 over one-hot logits, both scale modes (block scales
+    as recorded plans name the steps)."""
+    if block:
+        bind_recorded_steps(monkeypatch)
     rows = [288, 33, 64, 65, 31, 1, 352, 1214]
     e, k, hidden, inter = len(rows), 1, 256, 256
     t = sum(rows)
     mode = 1 if block else 0
-    desc = moe.moe_descriptor(e, k, mode, hidden, inter, 128 if block else 0)
-    assert moe.launch_geometry(_abi.MOE_DOWN, desc, t)[1].startswith("lf_moe_down_t256")
     rng = np.random.default_rng(960 + block)
     assign = rng.permutation(np.repeat(np.arange(e), rows))
     logits = (0.1 * rng.standard_normal((t, e))).astype(np.float32)
     logits[np.arange(t), assign] = 5.0
     x, logits, weights, out, st = run_case(rt, rng, t, e, k, hidden, inter, mode, block=block,
                                            logits=logits)
+    assert step_names(bound[0])[-2] == ("down_t256_b128" if block else "down_t256_aq")
     ex, w = check_routing(logits, k, mode, st)
     assert np.diff(st["offsets"]).tolist() == rows
     check_output(x, weights, ex, w, out, block, f"moe t256 row boundaries block={block}", st)
@@ -389,25 +432,21 @@ def test_moe_combine_every_top_k(rt, k):
     ([90, 70, 200, 12, 64, 33], 2, 768, 384, True),
     ([1, 0, 0, 17, 2], 1, 256, 256, False),     # a decode step
 ])
-def test_moe_t128x256(rt, rows, k, hidden, inter, zero):
+def test_moe_t128x256(rt, bound, rows, k, hidden, inter, zero):
     """Block-scaled profiles above 32 tokens on 128 x 256 tiles: exact rows
     per expert (top k over logits that pick the experts), stage by stage and
     end to end against the oracle, the fused quantizer's codes and scales
     bit for bit on the device's bf16 h."""
-    from lunaflux_amd import _abi, moe
     e, total = len(rows), sum(rows)
     t = total // k
-    desc = moe.moe_descriptor(e, k, 1, hidden, inter, 128)
-    names = [moe.step_geometry(s, desc, t)[1] for s in (_abi.MOE_ROUTE, _abi.MOE_GATE_UP, _abi.MOE_QUANT_HIDDEN,
-                                                        _abi.MOE_DOWN)]
-    assert names == ["lf_moe_route_q" if t > 32 else "lf_moe_route_sort_q", "lf_moe_gate_up_t128x256_b128_q", "",
-                     "lf_moe_down_t128x256_b128"]
     rng = np.random.default_rng(970 + total + hidden)
     logits = (0.1 * rng.standard_normal((t, e))).astype(np.float32)
     if k == 1:
         logits[np.arange(t), rng.permutation(np.repeat(np.arange(e), rows))] = 5.0
     x, logits, weights, out, st = run_case(rt, rng, t, e, k, hidden, inter, 1, block=True, logits=logits,
                                            zero_groups=zero)
+    assert step_names(bound[0]) == (["route_q", "sort_count", "sort"] if t > 32 else ["route_sort_q"]) + [
+        "gate_up_t128x256_b128_q", "down_t128x256_b128", "combine"]
     ex, w = check_routing(logits, k, 1, st)
     if k == 1:
         assert np.diff(st["offsets"]).tolist() == rows

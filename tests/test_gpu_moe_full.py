@@ -6,8 +6,9 @@ per-expert bias N(0, 1.5), e4m3 weights with per-channel scales. Config 5:
 64 experts, top-6 (softmax over all experts), hidden 2048, intermediate
 1408, 128 x 128 block scales with per-token-per-128-group activations,
 Zipf(1.1) expert popularity, at 4096 and 32 tokens. These run the kernels the
-benchmark times at those shapes (the 256 x 256 grouped GEMMs, the K = 14336
-down loop, the grouped GEMV form at 32 tokens).
+benchmark times at those shapes (the 256 x 256 and 128 x 256 grouped GEMMs, the
+K = 14336 down loop), and those that recorded plans name for config 5 (256 x
+256 tiles, the grouped GEMV form at 32 tokens).
 
 At full size the oracle cannot recompute every GEMM in seconds, so:
 * bit-exact at full size: routing ids, the stable sort, inverse positions,
@@ -35,7 +36,7 @@ import oracle_lib as o
 from lunaflux_amd import synth
 from parity import (abs_sum, combine, combine_tol, moved_codes_explained, parity,
                     swiglu_midpoint_tol)
-from test_gpu_moe import check_routing
+from test_gpu_moe import bind_recorded_steps, bound, check_routing, step_names  # noqa: F401 (bound: a fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -240,17 +241,18 @@ def zipf_logits(rng, t, e):
     return logits + np.log(1.0 / np.arange(1, e + 1) ** 1.1).astype(np.float32)[rng.permutation(e)]
 
 
-@pytest.mark.parametrize("t,gemm", [(4096, "t256_b128"), (32, "gemv")])
-def test_moe_config5_fine_grained_full_shape(rt, t, gemm):
-    from lunaflux_amd import _abi, moe
+@pytest.mark.parametrize("t,gemm,recorded", [(4096, "t128x256_b128", False), (32, "t128x256_b128", False),
+                                             (4096, "t256_b128", True), (32, "gemv", True)])
+def test_moe_config5_fine_grained_full_shape(rt, bound, monkeypatch, t, gemm, recorded):
+    """The forms a binding takes, and those recorded plans name."""
+    if recorded:
+        bind_recorded_steps(monkeypatch)
     e, k, hidden, inter = 64, 6, 2048, 1408
-    desc = moe.moe_descriptor(e, k, 1, hidden, inter, 128)
-    # (t256 with block scales: the gate/up epilogue quantizes h)
-    fused = "_q" if gemm == "t256_b128" else ""
-    assert moe.launch_geometry(_abi.MOE_GATE_UP, desc, t)[1] == f"lf_moe_gate_up_{gemm}{fused}"
-    assert moe.launch_geometry(_abi.MOE_DOWN, desc, t)[1] == f"lf_moe_down_{gemm}"
     rng = np.random.default_rng(50 + t)
     logits = zipf_logits(rng, t, e)
     x, weights, out, st = run_full(rt, rng, t, e, k, hidden, inter, 1, True, logits)
+    # (tiles: the gate/up epilogue quantizes h)
+    gemms = [n for n in step_names(bound[0]) if "gate_up" in n or "down" in n]
+    assert gemms == ["gate_up_" + gemm + ("" if gemm == "gemv" else "_q"), "down_" + gemm]
     check_full(x, weights, out, st, logits, k, 1, True, rng, f"moe config5 t={t}")
     assert st["offsets"][-1] == t * k
