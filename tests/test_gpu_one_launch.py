@@ -20,7 +20,7 @@ import oracle_lib as o
 from lunaflux_amd import _abi, fp8, synth
 from lunaflux_amd.device import DeviceError
 from lunaflux_amd.fp8 import _region
-from parity import abs_sum, parity
+from parity import abs_sum, parity, swiglu_midpoint_tol
 
 pytestmark = pytest.mark.gpu
 
@@ -196,6 +196,89 @@ def test_w8a8_gated_mlp_one_launch(rt, hidden, inter, max_tokens, symbol):
             wdr = o.dequantize(qd[cols], sd[cols])
             parity(y1[rows][:, cols], o.dense_projection(hr, wdr), k=inter, s_abs=abs_sum(hr, wdr),
                    label=f"{symbol} down")
+
+
+@pytest.fixture
+def recorded(monkeypatch):
+    """Bindings take the one-launch entries that recorded plans name, also
+    where they would take the split W8A8 form."""
+    monkeypatch.setattr(fp8, "w8a8_split_geometry", lambda *args: None)
+
+
+@pytest.mark.parametrize("k", [4096, 14336])
+def test_recorded_256x128_entry_at_full_width(rt, recorded, k):
+    """The 256 x 128 one-launch entry (4096 columns at 2048 rows, where
+    bindings take the split form): the two launches' bits, and the oracle on
+    sampled rows and columns."""
+    rng = np.random.default_rng(9700 + k)
+    n, max_tokens, m = 4096, 2048, 1900
+    q, s, w = weight(rt, rng, n, k)
+    buf = Buffers(rt, max_tokens, k, n)
+    one, two = bind(rt, "dense", buf, m, [w], True), bind(rt, "dense", buf, m, [w], False)
+    assert [st.name for st in one.steps] == ["lf_fp8_w8a8_dense_t256x128_aq"] and len(two.steps) == 2
+    x = synth.activations(rng, m, k)
+    y = buf.run(one, x)
+    assert np.array_equal(y, buf.run(two, x))
+    rows = np.unique(np.concatenate([[0, m - 1], rng.choice(m, 30, replace=False)]))
+    cols = np.sort(rng.choice(n, 192, replace=False))
+    xq, xs = o.quantize_rows(o.bf16_decode(x[rows]))
+    xr, wr = o.dequantize(xq, xs), o.dequantize(q[cols], s[cols])
+    parity(y[rows][:, cols], o.dense_projection(xr, wr), k=k, s_abs=abs_sum(xr, wr), label=f"t256x128_aq k={k}")
+
+
+@pytest.mark.parametrize("hidden,inter,max_tokens,names", [
+    # both halves split; the down projection alone; (recorded) one launch
+    (2048, 4096, 256, ["act_quant_rows", "w8a8_gate_up_t128x256_sk", "act_quant_rows", "w8a8_dense_t128x256_sk"]),
+    (1024, 4096, 256, ["w8a8_gate_up_t128_aq", "act_quant_rows", "w8a8_dense_t128x256_sk"]),
+    (2048, 4096, 256, ["w8a8_gated_mlp_t128_t128"]),
+])
+def test_w8a8_gated_mlp_split_route(rt, request, hidden, inter, max_tokens, names):
+    """W8A8 GatedMlp whose down projection takes the split form, as a binding
+    and as recorded plans run it, at a K that is cut into slices: stage by
+    stage on the device's own h and its codes, over ragged live rows."""
+    if len(names) == 1:
+        request.getfixturevalue("recorded")
+    rng = np.random.default_rng(9800 + hidden)
+    qg, sg, wg = weight(rt, rng, inter, hidden)
+    qu, su, wu = weight(rt, rng, inter, hidden)
+    qd, sd, wd = weight(rt, rng, hidden, inter)
+    buf = Buffers(rt, max_tokens, hidden, hidden)
+    for m in (max_tokens, max_tokens - 60, 17, 0):
+        op = rt.bind_gated_mlp("w8a8", buf.counts_for(m), _region(buf.xa, alignment=256), wg, wu, wd,
+                               _region(buf.ya, alignment=256), max_tokens)
+        assert [st.name[len("lf_fp8_"):] for st in op.steps] == names
+        x = synth.activations(rng, max(m, 1), hidden)[:m]
+        y = buf.run(op, x)
+        assert np.array_equal(buf.run(op, x), y)
+        if m == 0:
+            continue
+        al = lambda v: -(-v // 256) * 256
+        if len(names) == 1:   # workspace: sync area, xq, h [cap, I], hq
+            bands = max_tokens // 128
+            at = 256 + 128 * 3 * bands + al(max_tokens * hidden) + al(max_tokens * 4)
+            h = op.workspace.read(np.uint16, (m, inter), at)
+            hq_at, ws = at + al(max_tokens * inter * 2), op.workspace
+        else:
+            h = op.workspace.read(np.uint16, (m, inter))
+            hq_at, ws = 0, op.parts[1].workspace
+        hq = ws.read(np.uint8, (m, inter), hq_at)
+        hs = ws.read(np.float32, (m,), hq_at + al(m * inter))
+        rows = np.unique(np.concatenate([[0, m - 1], rng.choice(m, 12)]))
+        xq, xs = o.quantize_rows(o.bf16_decode(x[rows]))
+        xr = o.dequantize(xq, xs)
+        hcols = np.sort(rng.choice(inter, 128, replace=False))
+        wgr, wur = o.dequantize(qg[hcols], sg[hcols]), o.dequantize(qu[hcols], su[hcols])
+        g, u = o.dense_projection(xr, wgr), o.dense_projection(xr, wur)
+        parity(h[rows][:, hcols], o.silu_mul_array(g, u), label=f"{names[-1]} m={m} gate/up",
+               midpoint_tol=swiglu_midpoint_tol(g, u, abs_sum(xr, wgr), abs_sum(xr, wur), hidden))
+        hq_ref, hs_ref = o.quantize_rows(o.bf16_decode(h[rows]))
+        np.testing.assert_array_equal(hq[rows], hq_ref)
+        np.testing.assert_array_equal(hs[rows], hs_ref)
+        hr = o.dequantize(hq_ref, hs_ref)
+        cols = np.sort(rng.choice(hidden, 96, replace=False))
+        wdr = o.dequantize(qd[cols], sd[cols])
+        parity(y[rows][:, cols], o.dense_projection(hr, wdr), k=inter, s_abs=abs_sum(hr, wdr),
+               label=f"{names[-1]} m={m} down")
 
 
 def test_aq_sticky_error_and_timeout(rt):
