@@ -1909,7 +1909,7 @@ __global__ __launch_bounds__(1024) void lf_moe_route_sort(const int32_t *counts,
 __global__ __launch_bounds__(1024) void lf_moe_route_sort_q(const int32_t *counts, const int32_t *desc,
                                                             const float *logits, const uint16_t *x, uint8_t *ws) {
   const MoeDesc d = desc_of(desc);
-  if (!desc_ok(d) || d.group == 0) return;
+  if (!desc_ok(d) || d.group == 0 || blockDim.x != kSortThreads) return;
   if (blockIdx.x == 0) {
     route_sort_block<false>(counts, d, logits, x, ws);
     return;
@@ -1920,6 +1920,7 @@ __global__ __launch_bounds__(1024) void lf_moe_route_sort_q(const int32_t *count
                        (static_cast<int>(blockIdx.x) - 1) * kSortWaves + (static_cast<int>(threadIdx.x) >> 6),
                        (static_cast<int>(gridDim.x) - 1) * kSortWaves);
 }
+
 __global__ __launch_bounds__(256) void lf_moe_quant_tokens(const int32_t *counts,
                                                            const int32_t *desc,
                                                            const uint16_t *x, uint8_t *ws) {
@@ -2047,6 +2048,7 @@ __global__ __launch_bounds__(512) void lf_moe_down_t128x256_b128(const int32_t *
   if (!desc_ok(d) || d.group != 128 || header_of(wd).magic != kWeightMagic) return;
   grouped_gemm_t128x256<1, false>(counts, d, wd, wd, ws);
 }
+
 // Small profiles (at most 32 tokens): the grouped GEMV form, either scale
 // mode (the descriptor's group).
 __global__ __launch_bounds__(256) void lf_moe_gate_up_gemv(const int32_t *counts,

@@ -382,6 +382,26 @@ def test_route_sort_q_equals_route_sort(rt, t, e, k, mode, hidden):
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("name", ["lf_moe_route_sort", "lf_moe_route_sort_q"])
+def test_route_sort_rejects_other_block_sizes(rt, name):
+    """The one-block router sorts with exactly 1024 threads: a launch with
+    fewer writes nothing."""
+    from lunaflux_amd import moe
+    from lunaflux_amd.device import KernelArguments, KernelLaunchDimensions
+    from lunaflux_amd.fp8 import LaunchStep, _region
+    rng = np.random.default_rng(995)
+    t, e, k, hidden = 8, 16, 2, 256
+    desc = moe.moe_descriptor(e, k, 1, hidden, 128, 128)
+    ctx = rt.context
+    xa, la = ctx.upload(synth.activations(rng, t, hidden)), ctx.upload(rng.standard_normal((t, e)).astype(np.float32))
+    da, counts, nbytes = ctx.upload(desc.as_bytes()), rt.step_counts(t, decode=False), moe.workspace_bytes(desc, t)
+    ws = ctx.upload(np.full(nbytes, 0x5A, np.uint8))
+    args = [_region(counts, 20, alignment=4), _region(da, 32, alignment=4), _region(la), _region(xa), _region(ws)]
+    LaunchStep(rt.function(name), KernelLaunchDimensions.new((2 if name.endswith("_q") else 1,), (512,)),
+               KernelArguments(args), name).launch(rt.stream)
+    assert np.all(ws.read(np.uint8, (nbytes,)) == 0x5A)
+
+
 @pytest.mark.parametrize("t,prof,e,k,mode,hidden", [(33, 33, 64, 6, 1, 256), (250, 256, 129, 5, 1, 3968),
                                                     (0, 64, 8, 2, 0, 256), (1, 40, 256, 16, 0, 128)])
 def test_route_q_equals_two_launches(rt, t, prof, e, k, mode, hidden):
