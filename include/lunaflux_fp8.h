@@ -100,18 +100,19 @@ int32_t lunaflux_fp8_unpack_weight(const uint8_t *region, int64_t region_bytes,
  * 161-219):
  *  W8A16 ("decode"): bf16 activations, e4m3 weights dequantized to bf16 in
  *    registers (exact), bf16 MFMA, fp32 accumulation, per-channel scale in
- *    the epilogue. Two forms, picked per entry by the launch geometry:
+ *    the epilogue. Three forms, picked per entry by the launch geometry:
  *    one-tile (a block of waves owns one 16-column tile and splits K across
- *    its waves, partials summed in LDS) and column-group (each wave owns one
+ *    its waves, partials summed in LDS), column-group (each wave owns one
  *    16-column tile, a block several adjacent tiles over one K-slice sharing
- *    the activation slice through LDS; with more than one slice the partials
- *    are reduced in a fixed slice order by the last block of each column
- *    group through the workspace). Profiles of 65..128 rows use a third,
- *    LDS-tiled GEMM form (_m128_n64 / _m128_n128: blocks of 8 waves own
- *    128 rows x BN weight columns over a K-slice; activation and weight
- *    tiles stream global -> LDS in two rings loaded by different waves),
- *    except vocabulary-wide dense shapes. Suffix _m16/_m32/_m64/_m128: the
- *    profile's largest M; _k<K>...: a shape-specialized entry.
+ *    the activation slice through LDS) and an LDS-tiled GEMM (a block owns
+ *    the profile's rows x its weight columns over a K-slice; activation and
+ *    weight tiles stream global -> LDS in two rings loaded by different
+ *    waves). With more than one slice the last two reduce their partials in a
+ *    fixed slice order, by the last block of each column block, through the
+ *    workspace. Suffix _m16/_m32/_m64/_m128: the profile's largest M;
+ *    _m16_t1: one-tile; _cg_m16, _cg_m32 and _m128: column-group; _m32, _m64,
+ *    _b128_m16 and _m128_n64 / _m128_n128: the GEMM; _k<K>...: a
+ *    shape-specialized entry, one-tile or column-group.
  *  W8A8 ("prefill"): activations quantized per token to e4m3
  *    (lf_fp8_act_quant_rows), e4m3 x e4m3 MFMA, fp32 accumulation, row scale
  *    x channel scale epilogue. _t256: 256 x 256 tiles of 4 waves
@@ -186,8 +187,10 @@ enum lf_fp8_entry {
 /* Block-scaled projections (checkpoints whose weights carry weight_scale_inv
  * 128 x 128 block scales: W = q s[n / 128][k / 128]); N and K multiples of
  * 128, every Q / K / V width of a QKV operation too.
- *  W8A16: lf_fp8_w8a16_{dense,qkv,gate_up}_b128_m{16,32,64,128} and, for
- *      profiles of 65..128 rows, lf_fp8_w8a16_{op}_b128_m128_n{64,128}
+ *  W8A16: lf_fp8_w8a16_{dense,qkv,gate_up}_b128_m{16,32,64}, _b128_cg_m16 and
+ *      (dense, qkv) _b128_cg_m32, _b128_m128 for vocabulary-wide dense shapes
+ *      and, for other profiles of 65..128 rows,
+ *      lf_fp8_w8a16_{op}_b128_m128_n{64,128}
  *      (the per-channel entry's LDS-tiled GEMM geometry rule, except that
  *      at equal block counts it takes BN 128 where the per-channel entry
  *      takes BN 64); operands and
@@ -259,7 +262,9 @@ int64_t lunaflux_fp8_w8a8_workspace_bytes(int32_t entry, int64_t n, int64_t k, i
  * blocks x slices x row bands. entry: LF_FP8_ENTRY_W8A8_DENSE / _QKV (N the
  * packed width) / _GATE_UP. LF_UNSUPPORTED (-1 bytes) where the form does not
  * take the shape or profile: the operation then runs the forms of
- * lunaflux_fp8_launch_geometry. */
+ * lunaflux_fp8_launch_geometry. Its fp32 sums over K are those of the slices
+ * in order, so its outputs agree with those forms', and with another profile's
+ * (which may have another number of slices), to the rounding of such sums. */
 int32_t lunaflux_fp8_w8a8_split_geometry(int32_t entry, int64_t n, int64_t k, int32_t max_tokens,
                                          int32_t dims[7], char symbol[LF_FP8_SYMBOL_BYTES]);
 int64_t lunaflux_fp8_w8a8_split_workspace_bytes(int32_t entry, int64_t n, int64_t k, int32_t max_tokens);

@@ -1967,8 +1967,8 @@ __global__ __launch_bounds__(512) void lf_fp8_w8a8_gate_up_b128_t256(const int32
                                                                      uint16_t *h, uint8_t *ws) {
   w8a8_b128_wide_one_launch<true, 2>(counts, x, wg, wu, wu, h, ws);
 }
-// The same on 256 x 128 tiles (eight waves of 32 x 128), where 256 x 256
-// tiles would be too few.
+// The same on 256 x 128 tiles (eight waves of 64 x 64), where 256 x 256 tiles
+// would be too few.
 __global__ __launch_bounds__(512) void lf_fp8_w8a8_dense_b128_t256x128(const int32_t *counts,
                                                                        const uint16_t *x, const uint8_t *w,
                                                                        uint16_t *y, uint8_t *ws) {

@@ -417,9 +417,20 @@ bool w8a8_b128_bands(int64_t n, int64_t k, int32_t max_tokens, int64_t *bands) {
 // The standalone block-scaled entries run 256-row bands on 8 waves: 256 x
 // 256 tiles (_b128_t256) for profiles of at least kB128T256Tiles such tiles
 // where the width is a multiple of that tile (256 columns; gate/up: 128
-// outputs), else 256 x 128 tiles (_b128_t256x128; faster than 128 x 128 at
-// every profile measured, 128-8192 rows). Both use 32-bit activation
-// offsets (K < 2^24); past that, 128 x 128 tiles of 4 waves (_b128).
+// outputs), else 256 x 128 tiles (_b128_t256x128). Both use 32-bit activation
+// offsets (K < 2^24); past that, 128 x 128 tiles of 4 waves (_b128). One
+// launch, quantizer inside, us, 128 x 128 / 256 x 128 / 256 x 256 (256 x 256
+// tiles in the launch):
+//   4096 x 4096: 130 rows (16) 43.7 / 36.7 / 53.6, 1024 (64) 46.4 / 39.5 / 56.8,
+//     2048 (128) 58.1 / 46.3 / 57.5, 4096 (256) 117.2 / 92.3 / 78.9
+//   6144 x 4096: 1024 rows (96) 56.6 / 42.0 / 60.5, 2048 (192) 99.1 / 77.9 / 64.3
+//   4096 x 14336: 512 rows (32) 160.7 / 111.5 / 185.5, 2048 (128) 190.8 / 145.5 /
+//     189.3, 4096 (256) 374.7 / 283.7 / 253.6
+//   8192 x 8192: 1024 rows (128) 114.3 / 85.2 / 109.8, 2048 (256) 211.1 / 161.9 /
+//     137.7
+// At K of 1024 the 128 x 128 and 256 x 128 tiles are equal (1024 x 1024 at 512
+// rows 16.9 / 16.4), at two k-tiles 128 x 128 is 0.5 us ahead (256 x 256 9.1 /
+// 9.4).
 constexpr int64_t kB128T256Tiles = 192;
 struct W8a8B128 {
   int form;               // 0: 128 x 128, 1: 256 x 128, 2: 256 x 256
@@ -441,9 +452,12 @@ bool w8a8_b128_tiles(bool gate_up, int64_t n, int64_t k, int32_t max_tokens, W8a
 // Block-scaled W8A8 GatedMlp in one launch: both GEMMs on one tile form and
 // band height, 256 x 256 (_t256, 512 threads) where the gate/up launch of
 // the shape takes it and the hidden width is a multiple of 256, else 128 x
-// 128 (no 256 x 128 form here: kernels/projection.hip, B128Form). (Llama-3-
-// 8B widths, one launch: 256 x 256 270.6 / 548.1 us against 288.9 / 659.3
-// on 128 x 128 at 512 / 2048 rows; 128 x 128 ahead at 128 rows.)
+// 128 (no 256 x 128 form here: kernels/projection.hip, B128Form). One launch,
+// us, 128 x 128 / 256 x 256: Llama-3-8B widths at 130 rows 210 / 232, 256 251 /
+// 256, 512 276 / 255, 1024 362 / 308, 2048 580 / 450, 4096 1155 / 782; 2048 x
+// 5632 at 1024 rows (176 gate/up tiles) 121 / 117, 2048 159 / 145. (As two
+// operations, gate/up and down each in its own form: 151, 159, 181, 250, 431 and
+// 769 us at the former's sizes, so ahead of the one launch up to 2048 rows.)
 // out: the form, band height, the gate/up plus down column blocks and the
 // bands.
 bool w8a8_b128_gated(int64_t hidden, int64_t inter, int32_t max_tokens, W8a8B128 *out) {
@@ -787,6 +801,10 @@ int64_t lunaflux_fp8_w8a8_workspace_bytes(int32_t entry, int64_t n, int64_t k, i
 //     23.2 / 28.7 (1 slice; 2 slices 18.5 / 20.7 / 23.4 / 29.1)
 //   gate/up 14336 x 4096, 130 / 256 rows: 44.0 / 50.6 -> 36.9 / 42.6; past
 //     256 tiles (509 rows, 448) 67.2 -> 73.8, so not there
+// and at 1 / 64 / 128 rows: 4096 x 14336 106.6 / 124.1 / 126.2 -> 31.9 / 39.3 /
+//   47.0; 4096 x 4096 24.4 / 28.1 / 29.8 -> 15.7 / 18.6 / 26.2; 1536 x 4096 24.3 /
+//   28.1 / 29.4 -> 15.1 / 18.0 / 23.1; 256 x 2048 14.8 / 17.9 / 18.4 -> 12.0 / 13.6
+//   / 18.8; gate/up 14336 x 4096 29.0 / 33.6 / 36.0 -> 27.0 / 30.6 / 37.1
 // Shorter K and profiles above 2048 rows are not measured and keep their
 // forms.
 struct W8a8SplitForm {

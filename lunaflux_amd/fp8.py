@@ -410,9 +410,8 @@ class ProjectionRuntime:
     def _block(self, family: str, op: str, counts: Allocation, weights, operands, n: int, k: int,
                max_tokens: int, qkv_split=None) -> BoundOperation:
         """A projection over weights with 128 x 128 block scales: the _B128
-        entry of the family (W8A16: the column-group form with its split-K
-        workspace; W8A8: one launch, the per-128-column-group quantizer
-        inside it)."""
+        entry of the family (W8A16: with its split-K workspace; W8A8: one
+        launch, the per-128-column-group quantizer inside it)."""
         entry = _BLOCK_ENTRIES[(family, op)]
         for w in weights:
             w.admit(entry)
@@ -427,9 +426,13 @@ class ProjectionRuntime:
         (the _aq entry quantizes x inside it), or the act-quant launch and
         the split GEMM where that form takes the shape and profile
         (w8a8_split_geometry); one_launch=False binds the act-quant launch
-        and the GEMM-only launch instead (the one launch's outputs).
-        A weight with 128 x 128 block scales binds the family's _B128 entry
-        (one launch in both families, whatever one_launch says)."""
+        and the GEMM-only launch instead. The one launch and its two launches
+        give the same bits; the split form sums K in slices, whose number
+        depends on the profile, so its outputs agree with theirs, and with
+        another profile's, to the rounding of fp32 sums. It keeps fp32
+        partials of its own (slices x 128 KiB a tile: 33 MB for 4096 x 14336
+        at 512 rows). A weight with 128 x 128 block scales binds the family's
+        _B128 entry (one launch in both families, whatever one_launch says)."""
         _family(family, max_tokens)
         if w.scale_mode == BLOCK128:
             return self._block(family, "dense", counts, [w], [x, w.region, y], w.rows, w.columns,
@@ -456,6 +459,7 @@ class ProjectionRuntime:
     def bind_qkv(self, family: str, counts: Allocation, x: KernelArgument, wq: Fp8Weight,
                  wk: Fp8Weight, wv: Fp8Weight, y: KernelArgument, max_tokens: int,
                  one_launch: bool = True) -> BoundOperation:
+        """Q, K and V into one packed output; the forms of bind_dense."""
         _family(family, max_tokens)
         if not (wq.columns == wk.columns == wv.columns) or wk.rows != wv.rows:
             raise DeviceError("qkv shapes", _abi.LF_INVALID_ARGUMENT)
@@ -489,6 +493,7 @@ class ProjectionRuntime:
     def bind_gate_up(self, family: str, counts: Allocation, x: KernelArgument, wg: Fp8Weight,
                      wu: Fp8Weight, h: KernelArgument, max_tokens: int,
                      one_launch: bool = True) -> BoundOperation:
+        """h = silu(x Wg^T) * (x Wu^T); the forms of bind_dense."""
         _family(family, max_tokens)
         if wg.rows != wu.rows or wg.columns != wu.columns:
             raise DeviceError("gate/up shapes", _abi.LF_INVALID_ARGUMENT)
@@ -520,16 +525,18 @@ class ProjectionRuntime:
                        max_tokens: int, one_launch: bool = True) -> BoundOperation:
         """GatedMlp (model/plan/plan.mbt:47-59) as one launch, the plan's one
         AOT entry point for the operation (lunaflux_fp8_gated_mlp_geometry):
-        W8A8 for any width (x quantizer, gate/up + SwiGLU, h quantizer and
-        down as counted steps of one grid), W8A16 where a one-launch entry is
-        built for the shape and profile. Elsewhere, or with one_launch=False,
-        two launch steps: gate/up + SwiGLU into a bf16 intermediate, then the
-        down projection from it (each W8A8 step then quantizes its input
-        inside its own launch, or, with one_launch=False, in a launch of its
-        own). Every form computes the same values. Weights with 128 x 128
-        block scales: the _B128 GatedMlp entry of the family (W8A8 any width,
-        W8A16 where its one-launch forms are built), else, or with
-        one_launch=False, the two block-scaled launches."""
+        W8A8 where the down projection does not take the split form (x
+        quantizer, gate/up + SwiGLU, h quantizer and down as counted steps of
+        one grid), W8A16 where a one-launch entry is built for the shape and
+        profile. Elsewhere, or with one_launch=False, gate/up + SwiGLU into a
+        bf16 intermediate, then the down projection from it, each as
+        bind_gate_up and bind_dense bind it. Every form computes the same
+        operation on the same quantized values; forms that sum K in another
+        order (the split form's slices) agree to the rounding of fp32 sums and
+        the e4m3 codes of h that it moves. Weights with 128 x 128 block scales:
+        the _B128 GatedMlp entry of the family (W8A8 any width, W8A16 where its
+        one-launch forms are built), else, or with one_launch=False, the two
+        block-scaled launches."""
         if wd.columns != wg.rows or wd.rows != wg.columns:
             raise DeviceError("mlp shapes", _abi.LF_INVALID_ARGUMENT)
         if wg.rows != wu.rows or wg.columns != wu.columns:
@@ -547,7 +554,8 @@ class ProjectionRuntime:
         # a band height, and down has a tile for a quarter of the CUs at 509
         # rows (Llama-3-8B layer, us, one launch -> two operations: 200 rows
         # 264 -> 144, 509 rows 242 -> 181, 900 rows 287 -> 243, 1800 rows 416
-        # -> 403).
+        # -> 403; the MLP alone at 2048 rows, 4096 x 14336 342 -> 341, 4096 x
+        # 7168 182 -> 184, 2048 x 5632 112 -> 116, 2048 x 2048 51 -> 46).
         split_down = (entry == _abi.ENTRY_W8A8_GATED_MLP and one_launch and
                       w8a8_split_geometry(_abi.ENTRY_W8A8_DENSE, wd.rows, wd.columns, max_tokens) is not None)
         geometry = (gated_mlp_geometry(wg.columns, wg.rows, max_tokens, entry)
