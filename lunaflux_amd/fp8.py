@@ -173,6 +173,27 @@ def w8a8_split_geometry(entry: int, n: int, k: int, max_tokens: int):
             _abi.lib().lunaflux_fp8_w8a8_split_workspace_bytes(entry, n, k, max_tokens))
 
 
+def w8a8_gated_mlp_in_two(hidden: int, inter: int, max_tokens: int) -> bool:
+    """Whether a per-channel W8A8 GatedMlp binds as the gate/up and the down
+    operation in turn: where down takes the split form, and above 1024 rows
+    only if its K is sliced there or gate/up takes the split form too. In the
+    one launch both GEMMs share a band height, and down has a tile for a
+    quarter of the CUs at 509 rows. The MLP alone, rows = profile, us, one
+    launch / two operations: 4096 x 14336 at 128 / 509 / 1024 rows 174 / 93,
+    161 / 116, 207 / 186; 5120 x 13824 at 509 / 768 / 1024 rows 170 / 132,
+    224 / 202, 230 / 233; 8192 x 7168 at 768 rows (one slice) 209 / 191; 2048 x
+    5632 at 1280 / 2048 rows (3 / 2 slices) 83 / 76, 112 / 114; 2048 x 2048 at
+    2048 rows (gate/up split) 57 / 49. Above 1024 rows with one slice the two
+    are as good or behind: 4096 x 14336 at 1280 / 1536 / 2048 rows 254 / 260,
+    272 / 270, 324 / 329, 768 rows of a profile of 2048 205 / 210; 4096 x 7168
+    at 1280 / 1536 / 2048 158 / 160, 160 / 165, 169 / 173."""
+    down = w8a8_split_geometry(_abi.ENTRY_W8A8_DENSE, hidden, inter, max_tokens)
+    if down is None:
+        return False
+    return (max_tokens <= 1024 or down[0].grid[1] > 1 or
+            w8a8_split_geometry(_abi.ENTRY_W8A8_GATE_UP, inter, hidden, max_tokens) is not None)
+
+
 def gated_mlp_geometry(hidden: int, inter: int, max_tokens: int,
                        entry: int = _abi.ENTRY_W8A16_GATED_MLP):
     """(dims, symbol) of the one-launch GatedMlp entry (W8A16 or W8A8) for the
@@ -525,10 +546,9 @@ class ProjectionRuntime:
                        max_tokens: int, one_launch: bool = True) -> BoundOperation:
         """GatedMlp (model/plan/plan.mbt:47-59) as one launch, the plan's one
         AOT entry point for the operation (lunaflux_fp8_gated_mlp_geometry):
-        W8A8 where the down projection does not take the split form (x
-        quantizer, gate/up + SwiGLU, h quantizer and down as counted steps of
-        one grid), W8A16 where a one-launch entry is built for the shape and
-        profile. Elsewhere, or with one_launch=False, gate/up + SwiGLU into a
+        W8A8 but for the profiles of w8a8_gated_mlp_in_two (x quantizer,
+        gate/up + SwiGLU, h quantizer and down as counted steps of one grid),
+        W8A16 where a one-launch entry is built for the shape and profile. Elsewhere, or with one_launch=False, gate/up + SwiGLU into a
         bf16 intermediate, then the down projection from it, each as
         bind_gate_up and bind_dense bind it. Every form computes the same
         operation on the same quantized values; forms that sum K in another
@@ -549,17 +569,10 @@ class ProjectionRuntime:
             entry = None
         else:
             entry = _abi.ENTRY_W8A16_GATED_MLP if family == "w8a16" else _abi.ENTRY_W8A8_GATED_MLP
-        # W8A8 where the down projection takes the split form: the gate/up
-        # and the down operation in turn. In the one launch both GEMMs share
-        # a band height, and down has a tile for a quarter of the CUs at 509
-        # rows (Llama-3-8B layer, us, one launch -> two operations: 200 rows
-        # 264 -> 144, 509 rows 242 -> 181, 900 rows 287 -> 243, 1800 rows 416
-        # -> 403; the MLP alone at 2048 rows, 4096 x 14336 342 -> 341, 4096 x
-        # 7168 182 -> 184, 2048 x 5632 112 -> 116, 2048 x 2048 51 -> 46).
-        split_down = (entry == _abi.ENTRY_W8A8_GATED_MLP and one_launch and
-                      w8a8_split_geometry(_abi.ENTRY_W8A8_DENSE, wd.rows, wd.columns, max_tokens) is not None)
+        two_operations = (entry == _abi.ENTRY_W8A8_GATED_MLP and one_launch and
+                          w8a8_gated_mlp_in_two(wg.columns, wg.rows, max_tokens))
         geometry = (gated_mlp_geometry(wg.columns, wg.rows, max_tokens, entry)
-                    if one_launch and entry is not None and not split_down else None)
+                    if one_launch and entry is not None and not two_operations else None)
         if geometry is not None:
             for w in (wg, wu, wd):
                 w.admit(entry)

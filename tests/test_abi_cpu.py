@@ -339,6 +339,21 @@ def test_w8a8_split_geometry():
     assert fp8.w8a8_split_geometry(_abi.ENTRY_W8A8_DENSE, 4096, 4096, 0) is None
 
 
+@pytest.mark.parametrize("hidden,inter,last", [
+    (4096, 14336, 1024),   # down in slices to 1024 rows, whole above
+    (4096, 7168, 1024),
+    (8192, 7168, 1024),    # whole from 513 rows; past 256 tiles above 1024
+    (2048, 5632, 2048),    # two slices still at 2048 rows
+    (2048, 2048, 2048),    # down whole, gate/up takes the split form too
+    (2048, 1920, 0),       # K of down below the split form's
+])
+def test_w8a8_gated_mlp_in_two(hidden, inter, last):
+    """A W8A8 GatedMlp binds as two operations up to `last` rows and as the
+    one launch above them."""
+    for m in (1, 128, 509, 512, 513, 1024, 1025, 1536, 2048, 2049, 8192):
+        assert fp8.w8a8_gated_mlp_in_two(hidden, inter, m) == (m <= last), m
+
+
 def test_one_launch_w8a8_geometry_and_workspace():
     """The _aq entries: the GEMM-only entry's tile form, 256 quantizer blocks
     ahead of its tiles, workspace = sync area (128 B + one counter per row
