@@ -344,7 +344,7 @@ def lm_head_bench(rt, launches=20):
 
 def host_threads():
     """The host cores this process may use: the CPU affinity set, capped by
-    OMP_NUM_THREADS where the machine sets it (the GPU box gives each GPU a
+    OMP_NUM_THREADS where the machine sets it (a shared host gives each GPU a
     share of its cores and says so there)."""
     n = len(os.sched_getaffinity(0)) if hasattr(os, "sched_getaffinity") else (os.cpu_count() or 1)
     cap = os.environ.get("OMP_NUM_THREADS", "")
@@ -721,11 +721,11 @@ def summarize_traffic(fetch_csv, write_csv, kernel):
         "workload": "Llama-3-8B gate/up (4096 -> 2 x 14336, SwiGLU), M=32, one launch",
         "commands": [
             "cd /tmp && export TMPDIR=/tmp && timeout -s KILL 120 rocprofv3 --pmc FETCH_SIZE "
-            "--output-format csv -d $GRAFT_REPO_ROOT/gpurun_out/prof_fetch -o fetch -- python3 "
-            "$GRAFT_REPO_ROOT/bench.py --pmc-pass",
+            "--output-format csv -d $OUT/prof_fetch -o fetch -- python3 "
+            "$REPO/bench.py --pmc-pass",
             "cd /tmp && export TMPDIR=/tmp && timeout -s KILL 120 rocprofv3 --pmc WRITE_SIZE "
-            "--output-format csv -d $GRAFT_REPO_ROOT/gpurun_out/prof_write -o write -- python3 "
-            "$GRAFT_REPO_ROOT/bench.py --pmc-pass",
+            "--output-format csv -d $OUT/prof_write -o write -- python3 "
+            "$REPO/bench.py --pmc-pass",
             "python3 bench.py --summarize-traffic <fetch_counter_collection.csv> "
             "<write_counter_collection.csv>",
         ],

@@ -1,7 +1,7 @@
 /*
  * lf_oracle.h - CPU correctness oracle for the FP8 projection path.
  *
- * TEST INFRASTRUCTURE ONLY. This library is the checker: only tests/,
+ * TEST INFRASTRUCTURE ONLY. This library is the oracle: only tests/,
  * __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it. The
  * product (lunaflux_amd, liblunaflux_hip.so, the gfx950 code object) never
  * links, loads or calls it, and has no CPU fallback through it.

@@ -1,6 +1,6 @@
 """ctypes binding of the CPU oracle (oracle/liblf_oracle.so).
 
-Test infrastructure: the oracle is the checker for the HIP path. Only tests,
+Test infrastructure: the HIP path is checked against the oracle. Only tests,
 ``__graft_entry__.smoke()`` and bench.py's cpu_baseline leg load it.
 """
 from __future__ import annotations
